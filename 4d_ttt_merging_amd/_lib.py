@@ -58,6 +58,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
         _i64x3, _i64x3, _i64x3, _i64x3, _c_int, _c_p, _c_size, _c_p,
     ]),
+    "vgo_mass_bias_attn_f32_workspace": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(_c_size)]),
+    "vgo_mass_bias_attn_f32_fwd_ws": (_c_int, [
+        _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+        _i64x3, _i64x3, _i64x3, _i64x3, _c_p, _c_size, _c_p,
+    ]),
     "vgo_mass_bias_attn_fwd_static": (_c_int, [
         _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
         _i64x3, _i64x3, _i64x3, _i64x3, _c_int, _c_p,

@@ -46,14 +46,14 @@
 //    units of the remaining tasks are split evenly over all G (stream-K on
 //    the last round only); tasks cut between work-groups are finished by
 //    attn_merge_kernel from fp32 partial states.
-// fp32 path: exact fp32 arithmetic, one query row per lane, K/V tiles in LDS.
+// fp32 path: attention_f32.hip.
 #include <algorithm>
 #include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
 
-#include "vgo_common.h"
+#include "attention_f32.h"
 
 namespace vgo {
 namespace {
@@ -87,24 +87,6 @@ struct Mma<f16_t> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }
 };
-
-// (x[l], x[l ^ 32]) for every lane l in one VALU op: v_permlane32_swap
-// exchanges the upper half of one register with the lower half of another.
-__device__ __forceinline__ void both_halves(float x, float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  a = __uint_as_float(r[0]);
-  b = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float half_max(float x) {
-  float a, b;
-  both_halves(x, a, b);
-  return fmaxf(a, b);
-}
-__device__ __forceinline__ float half_sum(float x) {
-  float a, b;
-  both_halves(x, a, b);
-  return a + b;  // identical in both halves: IEEE addition commutes
-}
 
 // Position of key `kk` (0..63) inside a V^T row.  Within every 16-key group the
 // two middle quads are swapped, which is the order in which S^T's accumulator
@@ -158,15 +140,6 @@ struct PPLaunch {
   AttnArgs<T> p[2];
   PPSchedule s;
 };
-
-// First unit of work-group w under the static stream-K partition.
-__host__ __device__ __forceinline__ int64_t sk_begin(int64_t w, int64_t units, int64_t groups) {
-  return w * units / groups;
-}
-// Work-group whose range holds unit u.
-__host__ __device__ __forceinline__ int64_t sk_owner(int64_t u, int64_t units, int64_t groups) {
-  return ((u + 1) * groups - 1) / units;
-}
 
 // LDS stages: 2 (register-staged kernel) or 4 (DMA kernel); a stage holds a
 // K tile, a V^T tile and the tile's 64 key biases (fp32).
@@ -1106,93 +1079,6 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(PPLaunch<T> L) {
   }
 }
 
-// fp32: one query per lane; 64 queries per work-group; K/V tiles of 64 keys.
-constexpr int kF32Keys = 64;
-constexpr int kF32Chunk = 32;  // keys summed on their own before joining the running sums
-__global__ __launch_bounds__(64) void attn_f32_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    const float* __restrict__ bias, float* __restrict__ out, int heads, int nq, int nk,
-    int n_qblocks, int64_t qsb, int64_t qsh, int64_t qsn, int64_t ksb, int64_t ksh, int64_t ksn,
-    int64_t vsb, int64_t vsh, int64_t vsn, int64_t osb, int64_t osh, int64_t osn,
-    float scale_log2) {
-  __shared__ float k_lds[kF32Keys][kD + 1];
-  __shared__ float v_lds[kF32Keys][kD];
-  __shared__ float b_lds[kF32Keys];
-  const int task = xcd_remap(blockIdx.x, gridDim.x);
-  const int bh = task / n_qblocks;
-  const int qblk = task - bh * n_qblocks;
-  const int b = bh / heads;
-  const int h = bh - b * heads;
-  const int lane = threadIdx.x;
-  const int row = qblk * 64 + lane;
-  const float* kb_ptr = k + b * ksb + h * ksh;
-  const float* vb_ptr = v + b * vsb + h * vsh;
-
-  float qr[kD], acc[kD];
-  const float* qrow = q + b * qsb + h * qsh + static_cast<int64_t>(row < nq ? row : 0) * qsn;
-#pragma unroll
-  for (int d = 0; d < kD; ++d) {
-    qr[d] = row < nq ? qrow[d] : 0.0f;
-    acc[d] = 0.0f;
-  }
-  float m = -__builtin_inff(), l = 0.0f;
-  for (int kt = 0; kt < nk; kt += kF32Keys) {
-    __syncthreads();
-    for (int i = lane; i < kF32Keys * kD; i += 64) {
-      const int key = i / kD, d = i % kD;
-      const bool ok = kt + key < nk;
-      k_lds[key][d] = ok ? kb_ptr[(kt + key) * ksn + d] : 0.0f;
-      v_lds[key][d] = ok ? vb_ptr[(kt + key) * vsn + d] : 0.0f;
-    }
-    {
-      const int key = kt + lane;
-      b_lds[lane] = key < nk ? (bias ? bias[key] * kLog2e : 0.0f) : -__builtin_inff();
-    }
-    __syncthreads();
-    // 32 keys at a time, each chunk's P and P.V summed on their own and then added to
-    // the running totals: the rounding of the sums grows with sqrt(32) + sqrt(nk / 32)
-    // instead of sqrt(nk), which keeps the output within 1e-5 of the exact result at
-    // tens of thousands of keys.
-#pragma unroll
-    for (int j0 = 0; j0 < kF32Keys; j0 += kF32Chunk) {
-      float logit[kF32Chunk];
-      float mx = -__builtin_inff();
-#pragma unroll
-      for (int j = 0; j < kF32Chunk; ++j) {
-        float dot = 0.0f;
-#pragma unroll
-        for (int d = 0; d < kD; ++d) dot = fmaf(qr[d], k_lds[j0 + j][d], dot);
-        logit[j] = dot * scale_log2 + b_lds[j0 + j];
-        mx = fmaxf(mx, logit[j]);
-      }
-      const float mnew = fmaxf(m, mx);
-      // No finite logit yet (every key so far of mass 0): every P is 0 and the
-      // sums stay 0, where -inf - -inf would make them NaN.
-      const float base = mnew == -__builtin_inff() ? 0.0f : mnew;
-      const float corr = exp2f(m - base);
-      float lc = 0.0f, accc[kD];
-#pragma unroll
-      for (int d = 0; d < kD; ++d) accc[d] = 0.0f;
-#pragma unroll
-      for (int j = 0; j < kF32Chunk; ++j) {
-        const float p = exp2f(logit[j] - base);
-        lc += p;
-#pragma unroll
-        for (int d = 0; d < kD; ++d) accc[d] = fmaf(p, v_lds[j0 + j][d], accc[d]);
-      }
-      l = fmaf(l, corr, lc);
-#pragma unroll
-      for (int d = 0; d < kD; ++d) acc[d] = fmaf(acc[d], corr, accc[d]);
-      m = mnew;
-    }
-  }
-  if (row < nq) {
-    float* orow = out + b * osb + h * osh + static_cast<int64_t>(row) * osn;
-#pragma unroll
-    for (int d = 0; d < kD; ++d) orow[d] = acc[d] / l;
-  }
-}
-
 // Packs V of every (batch, head) into V^T tiles for the DMA kernel:
 // vt[bh][d][j'] = V[bh][key j][d] with j' = vt_pos(j) inside each 16-key group
 // (the key order of the P operand), zeros past n_key, npad = ntiles * 64
@@ -1266,20 +1152,6 @@ constexpr int64_t kMinUnitsPerGroup = 8;  // key tiles per work-group, at least
 // A split tail task is cut into at most about this many pieces, which bounds
 // the partial states attn_merge_kernel reads per query.
 constexpr int64_t kMaxPieces = 32;
-
-// One attention problem of a call, as the C ABI describes it.
-struct Problem {
-  const void* q;
-  const void* k;
-  const void* v;
-  const void* bias;
-  void* out;
-  int64_t batch, heads, nq, nk;
-  const int64_t* qs;
-  const int64_t* ks;
-  const int64_t* vs;
-  const int64_t* os;
-};
 
 // The stream-K schedule of an attn_pp_kernel launch over `count` problems;
 // the workspace query and the launch compute the same one on one device.
@@ -1484,22 +1356,6 @@ int launch_pp(const Problem* pr, int count, void* workspace, size_t workspace_by
   return check_launch("mass_bias_attention(merge)");
 }
 
-int launch_f32(const void* q, const void* k, const void* v, const void* bias, void* out,
-               int64_t batch, int64_t heads, int64_t nq, int64_t nk, const int64_t* qs,
-               const int64_t* ks, const int64_t* vs, const int64_t* os, hipStream_t stream) {
-  const int64_t n_qblocks = (nq + 63) / 64;
-  const int64_t total = n_qblocks * batch * heads;
-  VGO_REQUIRE(total <= 0x7fffffff, "mass_bias_attention: grid too large");
-  const float scale_log2 = 1.0f / 8.0f * kLog2e;
-  hipLaunchKernelGGL(attn_f32_kernel, dim3(static_cast<unsigned>(total)), dim3(64), 0, stream,
-                     static_cast<const float*>(q), static_cast<const float*>(k),
-                     static_cast<const float*>(v), static_cast<const float*>(bias),
-                     static_cast<float*>(out), static_cast<int>(heads), static_cast<int>(nq),
-                     static_cast<int>(nk), static_cast<int>(n_qblocks), qs[0], qs[1], qs[2], ks[0],
-                     ks[1], ks[2], vs[0], vs[1], vs[2], os[0], os[1], os[2], scale_log2);
-  return check_launch("mass_bias_attention(f32)");
-}
-
 }  // namespace
 }  // namespace vgo
 
@@ -1554,8 +1410,7 @@ int attn_run(const Problem* problems, const int64_t* head_dims, int count, int d
   if (dtype == VGO_F32) {
     for (int i = 0; i < n; ++i) {
       const Problem& p = live[i];
-      const int status = launch_f32(p.q, p.k, p.v, p.bias, p.out, p.batch, p.heads, p.nq, p.nk, p.qs,
-                                    p.ks, p.vs, p.os, s);
+      const int status = launch_attn_f32(p, nullptr, 0, s);
       if (status != VGO_OK) return status;
     }
     return VGO_OK;
@@ -1633,6 +1488,39 @@ extern "C" int vgo_mass_bias_attn_fwd_ws(const void* q, const void* k, const voi
   const Problem p = single_problem(q, k, v, log_mass, out, batch, heads, n_query, n_key, q_stride,
                                    k_stride, v_stride, o_stride);
   return attn_run(&p, &head_dim, 1, dtype, workspace, workspace_bytes, true, stream);
+}
+
+extern "C" int vgo_mass_bias_attn_f32_workspace(int64_t batch, int64_t heads, int64_t n_query,
+                                                int64_t n_key, size_t* bytes) {
+  using namespace vgo;
+  VGO_REQUIRE(bytes, "mass_bias_attention: null size pointer");
+  *bytes = 0;
+  VGO_REQUIRE(batch >= 0 && heads >= 0 && n_query >= 0 && n_key >= 0, "mass_bias_attention: negative size");
+  if (batch == 0 || heads == 0 || n_query == 0 || n_key == 0) return VGO_OK;
+  const Problem p = single_problem(nullptr, nullptr, nullptr, nullptr, nullptr, batch, heads, n_query,
+                                   n_key, nullptr, nullptr, nullptr, nullptr);
+  *bytes = attn_f32_workspace(p);
+  return VGO_OK;
+}
+
+extern "C" int vgo_mass_bias_attn_f32_fwd_ws(const void* q, const void* k, const void* v,
+                                             const void* log_mass, void* out, int64_t batch,
+                                             int64_t heads, int64_t n_query, int64_t n_key,
+                                             int64_t head_dim, const int64_t q_stride[3],
+                                             const int64_t k_stride[3], const int64_t v_stride[3],
+                                             const int64_t o_stride[3], void* workspace,
+                                             size_t workspace_bytes, void* stream) {
+  using namespace vgo;
+  const Problem p = single_problem(q, k, v, log_mass, out, batch, heads, n_query, n_key, q_stride,
+                                   k_stride, v_stride, o_stride);
+  bool empty = false;
+  const int status = check_problem(p, head_dim, VGO_F32, &empty);
+  if (status != VGO_OK || empty) return status;
+  const size_t need = attn_f32_workspace(p);
+  if (need > 0 && (workspace == nullptr || workspace_bytes < need))
+    return fail(VGO_EWORKSPACE, "mass_bias_attention: workspace too small");
+  VGO_REQUIRE(aligned(workspace, 16), "mass_bias_attention: workspace must be 16-byte aligned");
+  return launch_attn_f32(p, workspace, need, as_stream(stream));
 }
 
 extern "C" int vgo_mass_bias_attn_fwd_static(const void* q, const void* k, const void* v,

@@ -203,18 +203,6 @@ void launch_vec(const T* tb, int64_t table_stride, const int32_t* index, const f
 // Work-groups resident per CU for the persistent launch (MI355X: 256 CUs).
 constexpr int64_t kProjectBlocksPerCu = 8;
 
-int device_cus() {
-  static thread_local int cached = 0;
-  if (cached > 0) return cached;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus <= 0)
-    cus = 256;
-  cached = cus;
-  return cached;
-}
-
 template <typename T>
 int launch_project(const void* table, int64_t table_stride, const int32_t* index,
                    const float* weight, const int32_t* order, void* out, int64_t out_stride,

@@ -27,15 +27,6 @@
 namespace vgo {
 namespace {
 
-// Stream-K partition: work-group w of `groups` runs units [sk_begin(w), sk_begin(w + 1)).
-__host__ __device__ __forceinline__ int64_t sk_begin(int64_t w, int64_t units, int64_t groups) {
-  return w * units / groups;
-}
-// Work-group whose range holds unit u.
-__host__ __device__ __forceinline__ int64_t sk_owner(int64_t u, int64_t units, int64_t groups) {
-  return ((u + 1) * groups - 1) / units;
-}
-
 constexpr int kTile = 128;       // dictionary rows and source rows per work-group step
 constexpr int kKc = 64;          // K chunk staged in LDS
 

@@ -20,6 +20,17 @@ int check_launch(const char* what) {
   return VGO_OK;
 }
 
+int device_cus() {
+  static thread_local int cached_device = -1, cached = 0;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev == cached_device) return cached;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
+  cached_device = dev;
+  cached = cus;
+  return cached;
+}
+
 }  // namespace vgo
 
 extern "C" const char* vgo_last_error(void) { return vgo::g_last_error.c_str(); }

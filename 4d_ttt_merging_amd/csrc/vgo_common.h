@@ -16,6 +16,9 @@ void set_error(const std::string& msg);
 int fail(int status, const std::string& msg);
 int check_launch(const char* what);
 
+// Compute units of the current device.
+int device_cus();
+
 // Device address of the current device's static scratch (VGO_ATTN_STATIC_SCRATCH_BYTES,
 // csrc/scratch.hip), looked up once per device.
 int static_scratch(void** out);
@@ -68,7 +71,34 @@ __device__ __forceinline__ int xcd_remap(int pid, int total) {
   return xcd < tall ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
 }
 
+// Stream-K partition: work-group w of `groups` runs units [sk_begin(w), sk_begin(w + 1)).
+__host__ __device__ __forceinline__ int64_t sk_begin(int64_t w, int64_t units, int64_t groups) {
+  return w * units / groups;
+}
+// Work-group whose range holds unit u.
+__host__ __device__ __forceinline__ int64_t sk_owner(int64_t u, int64_t units, int64_t groups) {
+  return ((u + 1) * groups - 1) / units;
+}
+
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
+
+// (x[l], x[l ^ 32]) for every lane l in one VALU op: v_permlane32_swap
+// exchanges the upper half of one register with the lower half of another.
+__device__ __forceinline__ void both_halves(float x, float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float half_max(float x) {
+  float a, b;
+  both_halves(x, a, b);
+  return fmaxf(a, b);
+}
+__device__ __forceinline__ float half_sum(float x) {
+  float a, b;
+  both_halves(x, a, b);
+  return a + b;  // identical in both halves: IEEE addition commutes
+}
 
 // max(||row||_2, eps) of a row held as lane l's elements 4(l + 64i) + j in
 // v[i][j] (chunks past `chunks` ignored): squares summed with fused

@@ -76,16 +76,28 @@ def _attention_into_impl(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     the resident work-groups (stream-K, partial states merged by a third
     kernel); split=False takes the entry without a workspace (one
     work-group per 256-query block).  split=None picks by key length
-    (REG_MAX_KEYS).
+    (REG_MAX_KEYS); fp32, which has one kernel, is split over the work-groups
+    wherever its workspace query says so, unless split=False.
     """
-    if split is None:
-        split = k.shape[-2] > REG_MAX_KEYS
     lib = _lib.load()
     p, keep = _problem(q, k, v, bias, out)
     dtype = _lib.dtype_code(q.dtype)
     args = (p.q, p.k, p.v, p.log_mass, p.out, p.batch, p.heads, p.n_query, p.n_key, p.head_dim,
-            p.q_stride, p.k_stride, p.v_stride, p.o_stride, dtype)
+            p.q_stride, p.k_stride, p.v_stride, p.o_stride)
     need = ctypes.c_size_t(0)
+    if dtype == _lib.VGO_F32 and split is not False:
+        _lib.check(lib.vgo_mass_bias_attn_f32_workspace(p.batch, p.heads, p.n_query, p.n_key,
+                                                        ctypes.byref(need)))
+        workspace = None
+        if need.value:
+            workspace = torch.empty(need.value // 4, device=q.device, dtype=torch.float32)
+        _lib.check(lib.vgo_mass_bias_attn_f32_fwd_ws(*args, _lib.ptr(workspace), need.value,
+                                                     _lib.stream_of(q)))
+        del keep
+        return out
+    args += (dtype,)
+    if split is None:
+        split = k.shape[-2] > REG_MAX_KEYS
     if split:
         _lib.check(lib.vgo_mass_bias_attn_workspace(p.batch, p.heads, p.n_query, p.n_key, dtype,
                                                     ctypes.byref(need)))
@@ -111,6 +123,10 @@ def _attention_pair_into_impl(main: tuple, special: tuple) -> None:
         raise ValueError("both attention problems must share one dtype and device")
     p0, keep0 = _problem(*main)
     p1, keep1 = _problem(*special)
+    if main[0].dtype == torch.float32:  # one launch each, split over the work-groups
+        _attention_into_impl(*main)
+        _attention_into_impl(*special)
+        return
     problems = (_lib.AttnProblem * 2)(p0, p1)
     dtype = _lib.dtype_code(main[0].dtype)
     need = ctypes.c_size_t(0)

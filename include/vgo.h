@@ -109,6 +109,24 @@ int vgo_mass_bias_attn_fwd_static(const void* q, const void* k, const void* v,
                                   void* stream);
 
 /*
+ * fp32 mass-bias attention with each task's key tiles split evenly over the
+ * resident work-groups, from a caller-owned workspace of at least
+ * vgo_mass_bias_attn_f32_workspace() bytes (16-byte aligned; the fp32 partial
+ * states of the tasks that are cut; 0 bytes where splitting gains nothing, and
+ * workspace may then be NULL).  Arguments as vgo_mass_bias_attn_fwd with VGO_F32,
+ * which runs the same kernel one task per work-group: the two agree to the
+ * rounding of the fp32 sums.  mass_bias_attention.py:85-129 on fp32 inputs.
+ */
+int vgo_mass_bias_attn_f32_workspace(int64_t batch, int64_t heads, int64_t n_query, int64_t n_key,
+                                     size_t* bytes);
+int vgo_mass_bias_attn_f32_fwd_ws(const void* q, const void* k, const void* v, const void* log_mass,
+                                  void* out, int64_t batch, int64_t heads, int64_t n_query,
+                                  int64_t n_key, int64_t head_dim, const int64_t q_stride[3],
+                                  const int64_t k_stride[3], const int64_t v_stride[3],
+                                  const int64_t o_stride[3], void* workspace,
+                                  size_t workspace_bytes, void* stream);
+
+/*
  * One attention problem of vgo_mass_bias_attn_pair_fwd_ws, with the meaning of
  * vgo_mass_bias_attn_fwd's arguments of the same names (log_mass NULL: no bias).
  */

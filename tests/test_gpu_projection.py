@@ -155,3 +155,17 @@ def test_gather_probe_sums_the_projection_rows(vgo, device, dtype):
     small = table[:, :23].contiguous().to(device)
     with pytest.raises(RuntimeError, match="16-byte"):
         proj.gather_probe(small, idd, wd)
+
+
+@pytest.mark.parametrize("m", [16384, 16385, 98304, 98305])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_column_slices_at_their_edges(vgo, device, dtype, m):
+    """Row counts around a unit of every slice width (4 to 16 rows), and channel counts
+    that end inside a slice or give the eight XCDs unequal shares of the slices, on both
+    sides of the table sizes at which the slice width and the grid change: bit-exact."""
+    for n, d in [(1, 8), (3, 72), (15, 200), (17, 264), (129, 776), (4099, 72)]:
+        print(f"[project] slices dtype={dtype} n={n} m={m} d={d}", flush=True)
+        table, index, weight = _case(n + m + d, n, m, d, dtype)
+        index[0] = torch.tensor([0, m - 1, m - 1, 0], dtype=torch.int32)
+        out = vgo.top4_project(table.to(device), index.to(device), weight.to(device))
+        assert torch.equal(out.cpu(), oracle.top4_project(table, index, weight))

@@ -2,7 +2,9 @@
 
 Every `csrc/*.hip` file is compiled to an object under `_build/` and linked
 into one shared library next to this file.  The library exports only the
-`extern "C"` entry points declared in `include/vgo.h`.
+`extern "C"` entry points declared in `include/vgo.h`.  `csrc/torch_ops.cpp`
+(host code: the torch operators' implementations) becomes `libvgo_torch.so`,
+linked against it and torch.
 """
 from __future__ import annotations
 
@@ -16,6 +18,7 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC = PACKAGE_DIR / "csrc"
 BUILD_DIR = PACKAGE_DIR / "_build"
 LIBRARY = PACKAGE_DIR / "libvgo.so"
+OPS_LIBRARY = PACKAGE_DIR / "libvgo_torch.so"
 OFFLOAD_ARCH = "gfx950"
 
 # Packed fp32 VALU forms are switched off for every device compile.
@@ -59,6 +62,26 @@ def _compile(source: Path) -> Path:
     return obj
 
 
+def _build_torch_ops() -> None:
+    """Compile and link the torch operators against the torch that is imported here."""
+    import torch
+
+    torch_dir = Path(torch.__file__).resolve().parent
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    include = torch_dir / "include"
+    tmp = OPS_LIBRARY.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "c++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{include}", f"-I{include / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{rocm / 'include'}",
+           str(CSRC / "torch_ops.cpp"), "-o", str(tmp), f"-L{torch_dir / 'lib'}", "-ltorch", "-ltorch_cpu",
+           "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{PACKAGE_DIR}", f"-l:{LIBRARY.name}", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"building {OPS_LIBRARY.name} failed:\n{proc.stderr}")
+    os.replace(tmp, OPS_LIBRARY)
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
     """Compile every kernel for gfx950 and link `libvgo.so`; returns its path."""
     BUILD_DIR.mkdir(exist_ok=True)
@@ -79,6 +102,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     if proc.returncode != 0:
         raise RuntimeError(f"hipcc link failed:\n{proc.stderr}")
     os.replace(tmp, LIBRARY)
+    _build_torch_ops()
     if verbose:
         print(f"built {LIBRARY}")
     return LIBRARY

@@ -14,6 +14,7 @@ import torch
 
 PACKAGE_DIR = Path(__file__).resolve().parent
 LIBRARY_PATH = PACKAGE_DIR / "libvgo.so"
+OPS_LIBRARY_PATH = PACKAGE_DIR / "libvgo_torch.so"
 
 VGO_OK = 0
 VGO_EINVAL = -1
@@ -151,10 +152,25 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+_ops_loaded = False
 
 
 class ExtensionUnavailable(RuntimeError):
     """Raised when the HIP library is missing or cannot be loaded."""
+
+
+def load_ops() -> bool:
+    """Load `libvgo_torch.so`, the implementations of torch.ops.vgo.*, once; False while it is
+    not built (the operators then have schemas but no kernels)."""
+    global _ops_loaded
+    with _lock:
+        if not _ops_loaded and OPS_LIBRARY_PATH.exists() and LIBRARY_PATH.exists():
+            try:
+                torch.ops.load_library(str(OPS_LIBRARY_PATH))
+            except OSError as error:
+                raise ExtensionUnavailable(f"vgo torch operators failed to load: {error}") from error
+            _ops_loaded = True
+        return _ops_loaded
 
 
 def load() -> ctypes.CDLL:
@@ -162,13 +178,13 @@ def load() -> ctypes.CDLL:
     global _lib
     if _lib is not None:
         return _lib
+    if not load_ops():
+        raise ExtensionUnavailable(
+            f"vgo HIP extension is unavailable: {LIBRARY_PATH} and {OPS_LIBRARY_PATH} are not built "
+            "(run __graft_entry__.build())")
     with _lock:
         if _lib is not None:
             return _lib
-        if not LIBRARY_PATH.exists():
-            raise ExtensionUnavailable(
-                f"vgo HIP extension is unavailable: {LIBRARY_PATH} is not built "
-                "(run __graft_entry__.build())")
         try:
             lib = ctypes.CDLL(str(LIBRARY_PATH))
         except OSError as error:

@@ -37,6 +37,7 @@ from torch import Tensor, nn
 
 from . import _kernels, profiling
 from .mass_bias_attention import _attention_into, _attention_pair_into
+from .token_merging import TokenPlan
 
 
 class _null:
@@ -459,6 +460,9 @@ class SelfAttentionBlock(nn.Module):
     def forward(self, x: Tensor, rope=None) -> Tensor:
         """Inference forward of block.py:89-129 (no stochastic depth)."""
         if self._fused_rows(x):
+            arguments = self._native_dense(x, rope)
+            if arguments is not None:
+                return torch.ops.vgo.dense_block(x, *arguments)
             return self._fused_tail(x, self.attn(self._norm1_input(x), rope=rope))
         x_attn = x + self.ls1(self.attn(self.norm1(x), rope=rope))
         return x_attn + self.ls2(self.mlp(self.norm2(x_attn)))
@@ -470,9 +474,14 @@ class SelfAttentionBlock(nn.Module):
         computes it, or already cast to the autocast dtype (`norm1_for_plan`)."""
         if self.training:
             raise RuntimeError("token compaction is inference-only")
+        fused = self._fused_rows(x)
+        if fused:
+            arguments = self._native_merged(x, token_plan, normalized)
+            if arguments is not None:
+                return torch.ops.vgo.merged_block(x, *arguments)
         if normalized is None:
-            normalized = self._norm1_input(x) if self._fused_rows(x) else self.norm1(x)
-        if self._fused_rows(x):
+            normalized = self._norm1_input(x) if fused else self.norm1(x)
+        if fused:
             self.attn._check_hooks()
             y = self.attn._forward_merged(normalized, None, None, token_plan)
             restore_map_for = getattr(token_plan, "restore_map_for", None)
@@ -545,9 +554,96 @@ class SelfAttentionBlock(nn.Module):
             x_attn, h = _kernels.restore_residual_layer_norm(
                 x, table, index, weight, _ls_gamma(self.ls1), _ln_args(self.norm2),
                 norm_dtype=_autocast_dtype())
-        out, _, _ = _kernels.residual_layer_norm(x_attn, self.mlp(h).reshape(x.shape),
+        return self._mlp_tail(x_attn, h)
+
+    def _mlp_tail(self, x_attn: Tensor, h: Tensor) -> Tensor:
+        """x_attn + ls2(mlp(h)), h being norm2(x_attn) in the autocast dtype."""
+        linears = self._native_mlp() if _plain_call(x_attn) else None
+        if linears is not None:
+            return torch.ops.vgo.mlp_tail(x_attn, h, *linears, _ls_gamma(self.ls2))
+        out, _, _ = _kernels.residual_layer_norm(x_attn, self.mlp(h).reshape(x_attn.shape),
                                                  _ls_gamma(self.ls2))
         return out
+
+    # ---------------------------------------------------- native sequences ----
+    # Eager inference runs the launches of a block (or of its MLP) from one operator, which
+    # costs a fraction of the Python calls between them.  It applies where the modules are this
+    # package's own and nothing watches the calls in between: no hooks, replaced forwards,
+    # dispatch modes, tracing or profiling spans.  The launches and results are the same.
+    def _native_mlp(self) -> tuple | None:
+        """(fc1 weight, bias, fc2 weight, bias) in the autocast dtype, or None."""
+        mlp = self.mlp
+        if not (_plain(mlp, Mlp) and _plain(mlp.act, nn.GELU)
+                and mlp.act.approximate == "none" and _plain(mlp.drop, nn.Dropout)
+                and not (mlp.drop.training and mlp.drop.p > 0)):
+            return None
+        return _cast_linears(mlp.fc1, mlp.fc2)
+
+    def _native_parameters(self, x: Tensor) -> tuple | None:
+        """(norms, eps, linears, gammas, heads) of torch.ops.vgo.dense_block and merged_block
+        for an x [B, N, C], or None."""
+        attn = self.attn
+        if x.ndim != 3 or not _plain(attn, SelfAttention):
+            return None
+        mlp = self._native_mlp()
+        if mlp is None or not (_plain(attn.proj_drop, nn.Dropout)
+                               and not (attn.proj_drop.training and attn.proj_drop.p > 0)):
+            return None
+        attn._check_hooks()
+        if attn.qkv.in_features != attn.num_heads * 64 or attn.qkv.in_features != x.shape[-1]:
+            return None
+        head_norms = (None, None, None, None)
+        head_eps = 1e-5
+        if attn.use_qk_norm:
+            q_norm, k_norm = attn.q_norm, attn.k_norm
+            if q_norm.eps != k_norm.eps:
+                return None
+            head_norms = (q_norm.weight, q_norm.bias, k_norm.weight, k_norm.bias)
+            head_eps = q_norm.eps
+        projections = _cast_linears(attn.qkv, attn.proj)
+        if projections is None:
+            return None
+        norm1, norm2 = self.norm1, self.norm2
+        return ([norm1.weight, norm1.bias, norm2.weight, norm2.bias, *head_norms],
+                [norm1.eps, norm2.eps, head_eps], [*projections, *mlp],
+                [_ls_gamma(self.ls1), _ls_gamma(self.ls2)], attn.num_heads)
+
+    def _native_dense(self, x: Tensor, rope) -> tuple | None:
+        """The arguments of torch.ops.vgo.dense_block after x, or None."""
+        if not _plain_call(x):
+            return None
+        sin = cos = None
+        if rope is not None:
+            sin, cos = rope
+            if sin.ndim != 2 or x.ndim != 3 or sin.shape[0] > x.shape[1]:
+                return None
+        parameters = self._native_parameters(x)
+        return None if parameters is None else (*parameters, sin, cos, _autocast_dtype())
+
+    def _native_merged(self, x: Tensor, plan, normalized: Tensor | None) -> tuple | None:
+        """The arguments of torch.ops.vgo.merged_block after x, or None: one batch element and a
+        plain TokenPlan that pools and removes tokens."""
+        if not _plain_call(x):
+            return None
+        dtype = _autocast_dtype()
+        if (type(plan) is not TokenPlan or x.ndim != 3 or x.shape[0] != 1 or self.attn.training
+                or plan.original_tokens != x.shape[1] or plan.kept_tokens == plan.original_tokens
+                or not (plan.pool_sources or plan.pool_mask is not None)):
+            return None
+        log_mass = plan.key_log_mass
+        if log_mass is not None and log_mass.numel() != plan.kept_tokens:
+            return None
+        qkv = plan.precomputed_qkv
+        given = qkv if qkv is not None else normalized
+        if given is not None and (given.dtype != dtype or type(given) is not Tensor or not given.is_contiguous()
+                                  or given.shape != (1, x.shape[1], x.shape[2] * (1 if qkv is None else 3))):
+            return None
+        parameters = self._native_parameters(x)
+        if parameters is None:
+            return None
+        csr, counts = plan._cluster_csr(0)
+        return (normalized if qkv is None else None, qkv, csr.offsets, csr.order, counts, plan._contribution(0),
+                plan._inverse32(0), log_mass, *parameters, dtype)
 
     def _fused_tail(self, x: Tensor, y: Tensor) -> Tensor:
         """x_attn = x + ls1(y); return x_attn + ls2(mlp(norm2(x_attn))) with two row passes."""
@@ -555,9 +651,44 @@ class SelfAttentionBlock(nn.Module):
             y = y.reshape(x.shape).contiguous()
         x_attn, h, _ = _kernels.residual_layer_norm(x, y, _ls_gamma(self.ls1), _ln_args(self.norm2),
                                                     norm_dtype=_autocast_dtype())
-        out, _, _ = _kernels.residual_layer_norm(x_attn, self.mlp(h).reshape(x.shape),
-                                                 _ls_gamma(self.ls2))
-        return out
+        return self._mlp_tail(x_attn, h)
+
+
+# Methods whose replacement on an instance a native sequence would pass by.
+_METHODS = frozenset(("forward", "compute_attention", "_forward_merged", "_merged_fused", "_dense_fused", "_attend",
+                      "_attention_dtype", "_fusable", "_norm_params", "_bias", "_cast_params", "_cast_sources"))
+
+
+def _plain(module: nn.Module, *types: type) -> bool:
+    """The module is exactly one of `types` and calling it runs that class's code alone."""
+    return (type(module) in types and not module._forward_hooks and not module._forward_pre_hooks
+            and not module._backward_hooks and not module._backward_pre_hooks
+            and _METHODS.isdisjoint(module.__dict__))
+
+
+def _plain_call(x: Tensor) -> bool:
+    """Nothing observes the calls a block makes: no tracing, dispatch or function mode, tensor
+    subclass, global module hook or profiling span."""
+    return (type(x) in (Tensor, nn.Parameter) and not torch.compiler.is_compiling() and not profiling.enabled()
+            and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and not nn.modules.module._has_any_global_hook())
+
+
+def _cast_linears(*linears: nn.Module) -> tuple | None:
+    """(weight, bias, weight, bias, ...) as each Linear's own forward would hand them to the
+    GEMM under autocast, or None where one would not use its cast copies."""
+    dtype = _autocast_dtype()
+    if (dtype is None or not torch.is_autocast_cache_enabled() or torch.cuda.is_current_stream_capturing()):
+        return None
+    cast = []
+    for linear in linears:
+        if not _plain(linear, Linear, LinearKMaskedBias) or not linear.weight.is_cuda:
+            return None
+        pair = linear._cast_params(dtype)
+        if pair is None:
+            return None
+        cast += pair
+    return tuple(cast)
 
 
 def _autocast_dtype() -> torch.dtype | None:

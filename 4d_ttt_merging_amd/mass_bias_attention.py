@@ -8,8 +8,6 @@ allocation.  The arithmetic runs in the hand-written HIP kernel
 """
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _lib
@@ -44,99 +42,29 @@ def _problem(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bias: torch.Tens
     return problem, (q, k, v, bias, out)
 
 
-# Key lengths up to this run faster on the entry without a workspace.  Measured
-# on MI355X over 32,928 queries x 16 heads split into equal self-attention
-# problems: at 1,029 / 1,536 / 2,058 keys the register-staged kernel takes
-# 0.79 / 0.86 / 0.97 of the ping-pong kernel's time, at 3,087 / 4,116 / 8,232
-# keys 1.05 / 1.08 / 1.19.  With few key tiles per 512-query task the ping-pong
-# kernel's V^T pack, pipeline fill and partly empty tasks do not pay off.
-REG_MAX_KEYS = 2560
-
-
 def _attention_into(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                     bias: torch.Tensor | None, out: torch.Tensor, *,
                     split: bool | None = None) -> torch.Tensor:
-    """`_attention_into_impl` through the operator torch.ops.vgo.attention_into."""
-    torch.ops.vgo.attention_into(q, k, v, bias, out, -1 if split is None else int(split))
-    return out
-
-
-def _attention_pair_into(main: tuple, special: tuple) -> None:
-    """`_attention_pair_into_impl` through the operator torch.ops.vgo.attention_pair_into."""
-    torch.ops.vgo.attention_pair_into(*main, *special)
-
-
-def _attention_into_impl(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
-                         bias: torch.Tensor | None, out: torch.Tensor, *,
-                         split: bool | None = None) -> torch.Tensor:
-    """Run the kernel on [B,H,N,64] views (any batch/head/token strides) into `out`.
+    """Run the kernel on [B,H,N,64] views (any batch/head/token strides) into `out`
+    (torch.ops.vgo.attention_into).
 
     split=True takes the workspace entry: V^T packed per head, 512-query
     blocks on the 8-wave kernel, (query block, key tile) work balanced over
     the resident work-groups (stream-K, partial states merged by a third
     kernel); split=False takes the entry without a workspace (one
-    work-group per 256-query block).  split=None picks by key length
-    (REG_MAX_KEYS); fp32, which has one kernel, is split over the work-groups
-    wherever its workspace query says so, unless split=False.
+    work-group per 256-query block).  split=None picks by key length; fp32,
+    which has one kernel, is split over the work-groups wherever its workspace
+    query says so, unless split=False.
     """
-    lib = _lib.load()
-    p, keep = _problem(q, k, v, bias, out)
-    dtype = _lib.dtype_code(q.dtype)
-    args = (p.q, p.k, p.v, p.log_mass, p.out, p.batch, p.heads, p.n_query, p.n_key, p.head_dim,
-            p.q_stride, p.k_stride, p.v_stride, p.o_stride)
-    need = ctypes.c_size_t(0)
-    if dtype == _lib.VGO_F32 and split is not False:
-        _lib.check(lib.vgo_mass_bias_attn_f32_workspace(p.batch, p.heads, p.n_query, p.n_key,
-                                                        ctypes.byref(need)))
-        workspace = None
-        if need.value:
-            workspace = torch.empty(need.value // 4, device=q.device, dtype=torch.float32)
-        _lib.check(lib.vgo_mass_bias_attn_f32_fwd_ws(*args, _lib.ptr(workspace), need.value,
-                                                     _lib.stream_of(q)))
-        del keep
-        return out
-    args += (dtype,)
-    if split is None:
-        split = k.shape[-2] > REG_MAX_KEYS
-    if split:
-        _lib.check(lib.vgo_mass_bias_attn_workspace(p.batch, p.heads, p.n_query, p.n_key, dtype,
-                                                    ctypes.byref(need)))
-    if need.value == 0:
-        status = lib.vgo_mass_bias_attn_fwd(*args, _lib.stream_of(q))
-    else:
-        workspace = torch.empty(need.value // 4, device=q.device, dtype=torch.float32)
-        status = lib.vgo_mass_bias_attn_fwd_ws(*args, workspace.data_ptr(), need.value,
-                                               _lib.stream_of(q))
-    _lib.check(status)
-    del keep
+    torch.ops.vgo.attention_into(q, k, v, bias, out, -1 if split is None else int(split))
     return out
 
 
-def _attention_pair_into_impl(main: tuple, special: tuple) -> None:
-    """Merged attention and the dense special-query pass in one launch.
-
-    `main` and `special` are (q, k, v, bias, out) as for `_attention_into`;
-    each output receives its problem's result (vgo_mass_bias_attn_pair_fwd_ws).
-    """
-    lib = _lib.load()
-    if main[0].dtype != special[0].dtype or main[0].device != special[0].device:
-        raise ValueError("both attention problems must share one dtype and device")
-    p0, keep0 = _problem(*main)
-    p1, keep1 = _problem(*special)
-    if main[0].dtype == torch.float32:  # one launch each, split over the work-groups
-        _attention_into_impl(*main)
-        _attention_into_impl(*special)
-        return
-    problems = (_lib.AttnProblem * 2)(p0, p1)
-    dtype = _lib.dtype_code(main[0].dtype)
-    need = ctypes.c_size_t(0)
-    _lib.check(lib.vgo_mass_bias_attn_pair_workspace(problems, 2, dtype, ctypes.byref(need)))
-    workspace = None
-    if need.value:
-        workspace = torch.empty(need.value // 4, device=main[0].device, dtype=torch.float32)
-    _lib.check(lib.vgo_mass_bias_attn_pair_fwd_ws(
-        problems, 2, dtype, _lib.ptr(workspace), need.value, _lib.stream_of(main[0])))
-    del keep0, keep1
+def _attention_pair_into(main: tuple, special: tuple) -> None:
+    """Merged attention and the dense special-query pass in one launch
+    (torch.ops.vgo.attention_pair_into).  `main` and `special` are (q, k, v, bias, out) as
+    for `_attention_into`; each output receives its problem's result."""
+    torch.ops.vgo.attention_pair_into(*main, *special)
 
 
 def mass_bias_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,

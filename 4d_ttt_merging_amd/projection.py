@@ -16,8 +16,9 @@ from . import _kernels, _lib
 def top4_project(table: torch.Tensor, index: torch.Tensor, weight: torch.Tensor, *,
                  out: torch.Tensor | None = None, order: torch.Tensor | None = None) -> torch.Tensor:
     """Gather four rows of `table` [M, D] per output row and take their weighted sum
-    (torch.ops.vgo.top4_project, or top4_project_into with `out`); see
-    `_top4_project_impl`.  `order` (int32 [N], e.g. from `locality_order`) only sets
+    (torch.ops.vgo.top4_project, or top4_project_into with `out`): index [N, 4] int32,
+    weight [N, 4] float32.  Zero weights skip their gather; an out-of-range index with a
+    non-zero weight yields a NaN row (the kernel never reads outside the table).  `order` (int32 [N], e.g. from `locality_order`) only sets
     the order the rows are computed in; the result is the same."""
     _lib.require_gpu(table, index, weight, out, order)
     if order is not None:
@@ -58,45 +59,3 @@ def gather_probe(table: torch.Tensor, index: torch.Tensor, weight: torch.Tensor)
         table.data_ptr(), table.stride(0), index.data_ptr(), weight.data_ptr(), sums.data_ptr(),
         index.shape[0], table.shape[0], table.shape[1], _lib.dtype_code(table.dtype), _lib.stream_of(table)))
     return sums
-
-
-def _top4_project_impl(table: torch.Tensor, index: torch.Tensor, weight: torch.Tensor, *,
-                       out: torch.Tensor | None = None,
-                       order: torch.Tensor | None = None) -> torch.Tensor:
-    """Gather four rows of `table` [M, D] per output row and take their weighted sum.
-
-    index: [N, 4] int32, weight: [N, 4] float32 (both contiguous).  Zero weights
-    skip their gather; an out-of-range index with a non-zero weight yields a NaN
-    row (the kernel never reads outside the table).
-    """
-    lib = _lib.load()
-    _lib.require_gpu(table, index, weight, out)
-    if table.ndim != 2 or index.ndim != 2 or index.shape[1] != 4 or weight.shape != index.shape:
-        raise ValueError("top4_project requires table [M,D], index [N,4] and weight [N,4]")
-    if index.dtype != torch.int32 or weight.dtype != torch.float32:
-        raise ValueError("top4_project requires int32 indices and float32 weights")
-    index = index.contiguous()
-    weight = weight.contiguous()
-    if table.stride(-1) != 1:
-        table = table.contiguous()
-    n_rows, dim = index.shape[0], table.shape[1]
-    if out is None:
-        out = torch.empty((n_rows, dim), device=table.device, dtype=table.dtype)
-    elif out.shape != (n_rows, dim) or out.dtype != table.dtype or out.stride(-1) != 1:
-        raise ValueError("top4_project output must be [N, D] of the table dtype")
-    if order is not None:
-        if order.shape != (n_rows,) or order.dtype != torch.int32:
-            raise ValueError("top4_project order must be int32 [N]")
-        order = order.contiguous()
-        status = lib.vgo_top4_project_ordered(
-            table.data_ptr(), table.stride(0), index.data_ptr(), weight.data_ptr(), order.data_ptr(),
-            out.data_ptr(), out.stride(0), n_rows, table.shape[0], dim, _lib.dtype_code(table.dtype),
-            _lib.stream_of(table))
-    else:
-        status = lib.vgo_top4_project(
-            table.data_ptr(), table.stride(0), index.data_ptr(), weight.data_ptr(), out.data_ptr(),
-            out.stride(0), n_rows, table.shape[0], dim, _lib.dtype_code(table.dtype),
-            _lib.stream_of(table),
-        )
-    _lib.check(status)
-    return out

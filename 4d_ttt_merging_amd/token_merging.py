@@ -20,8 +20,6 @@ layout, with torch's CPU generator exactly as the reference draws them.
 """
 from __future__ import annotations
 
-import ctypes
-
 import functools
 import math
 from dataclasses import dataclass, field
@@ -541,35 +539,12 @@ def build_fastvggt_plan(
     if not tokens.is_cuda:
         raise RuntimeError("vgo kernels run on the GPU only; got a CPU tensor")
 
-    best = torch.empty((batch, sources.numel()), device=device, dtype=torch.float32)
-    target = torch.empty((batch, sources.numel()), device=device, dtype=torch.int32)
     if prenormalized and tokens.dtype != torch.bfloat16:
         raise ValueError("prenormalized FastVGGT tokens must be bf16 unit rows")
-    for b in range(batch):
-        x = _as_rows(tokens[b])
-        if prenormalized:
-            src, src_rows = x, sources
-            dst = x.index_select(0, destinations)
-        else:
-            src, src_rows = _kernels.normalize_rows(x, sources, 1e-12), None
-            dst = _kernels.normalize_rows(x, destinations, 1e-12)
-        _kernels.similarity_topk(src, dst, 1, src_rows=src_rows, index_dtype=torch.int32,
-                                 out=(best[b].view(-1, 1), target[b].view(-1, 1)))
+    best, target = torch.ops.vgo.fastvggt_match(tokens, sources, destinations, prenormalized)
     if after_match is not None:
         after_match()
-    keep = torch.empty((batch, total - removed), device=device, dtype=torch.int64)
-    inverse = torch.empty((batch, total), device=device, dtype=torch.int64)
-    flags = torch.empty((batch, sources.numel()), device=device, dtype=torch.uint8)
-    lib = _kernels._lib.load()
-    need = ctypes.c_size_t(0)
-    _kernels._lib.check(lib.vgo_fastvggt_assemble_workspace(batch, sources.numel(), total,
-                                                            ctypes.byref(need)))
-    workspace = torch.empty(max(need.value // 4, 1), device=device, dtype=torch.int32)
-    status = lib.vgo_fastvggt_assemble_ws(
-        best.data_ptr(), target.data_ptr(), sources.data_ptr(), destinations.data_ptr(), batch,
-        sources.numel(), destinations.numel(), total, removed, keep.data_ptr(), inverse.data_ptr(),
-        flags.data_ptr(), workspace.data_ptr(), need.value, _kernels._lib.stream_of(tokens))
-    _kernels._lib.check(status)
+    keep, inverse, flags = torch.ops.vgo.fastvggt_assemble(best, target, sources, destinations, total, removed)
     plan = TokenPlan(keep, inverse, total)
     # Match results stay on the device for diagnostics and tests.
     plan._derived["match"] = (sources, destinations, best, target, flags)

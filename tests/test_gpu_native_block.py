@@ -1,0 +1,110 @@
+"""Blocks run as one native operator against the same blocks run call by call.
+
+A forward hook on the MLP's activation makes a block run call by call; both routes launch
+the same kernels, so the results are equal bit for bit.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _block(vgo, dim, heads, device, **kw):
+    torch.manual_seed(dim + heads)
+    block = vgo.SelfAttentionBlock(dim, heads, qkv_bias=True, mask_k_bias=True, **kw).eval().to(device)
+    for p in block.parameters():
+        torch.nn.init.normal_(p, std=0.2 if p.ndim == 1 else p.shape[-1] ** -0.5)
+    return block
+
+
+def _both(block, call):
+    """(native result, call-by-call result, hook calls during each)."""
+    native = call()
+    fired = []
+    handle = block.mlp.act.register_forward_hook(lambda *a: fired.append(1))
+    try:
+        return native, call(), len(fired)
+    finally:
+        handle.remove()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dim,heads,kw", [(128, 2, dict(use_qk_norm=True, init_values=0.5)),
+                                          (256, 4, dict(use_qk_norm=False, proj_bias=False, ffn_bias=False))])
+def test_dense_block(vgo, device, dtype, dim, heads, kw):
+    layers = __import__("importlib").import_module("4d_ttt_merging_amd.layers")
+    block = _block(vgo, dim, heads, device, **kw)
+    x = torch.randn(3, 37, dim, device=device)
+    for rope in (None, layers.rope_sincos(4, 8, 64, device=device)):
+        with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+            assert block._native_dense(x, rope) is not None
+            native, plain, fired = _both(block, lambda: block(x, rope))
+        assert fired == 1 and torch.equal(native, plain)
+    with torch.autocast("cuda", dtype=dtype):
+        assert block(x).requires_grad  # grad mode: call by call, on the torch rows
+
+
+@pytest.mark.parametrize("mass", [True, False])
+def test_merged_block(vgo, device, mass):
+    block = _block(vgo, 128, 2, device, use_qk_norm=True, init_values=0.5)
+    x = torch.randn(1, 90, 128, device=device)
+    inverse = torch.arange(90, device=device) % 41
+    counts = torch.bincount(inverse).float()
+    plan = vgo.TokenPlan(torch.arange(41, device=device)[None], inverse[None], 90,
+                         key_log_mass=counts.log()[None] if mass else None)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        h32, h = block.norm1_for_plan(x)
+        for normalized in (None, h, h32):  # fp32 rows take the call-by-call route
+            assert (block._native_merged(x, plan, normalized) is None) == (normalized is h32)
+            native, plain, fired = _both(block, lambda: block.forward_compacted(x, plan, normalized=normalized))
+            assert fired == 1 and torch.equal(native, plain)
+        plan.precomputed_qkv = block.attn.qkv(h)
+        native, plain, _ = _both(block, lambda: block.forward_compacted(x, plan, normalized=h))
+        assert torch.equal(native, plain)
+        plan.precomputed_qkv = None
+        bad = vgo.TokenPlan(plan.keep, plan.inverse, 90, key_log_mass=torch.zeros(1, 40, device=device))
+        with pytest.raises(ValueError, match="log_key_mass length"):
+            block.forward_compacted(x, bad)
+
+
+def test_replaced_modules_run_call_by_call(vgo, device):
+    """Subclasses, replaced methods, dispatch modes and global hooks all see their calls."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    block = _block(vgo, 128, 2, device, use_qk_norm=True)
+    x = torch.randn(1, 20, 128, device=device)
+
+    class Seen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        ref = block(x)
+        with Seen() as seen:
+            assert torch.equal(block(x), ref)
+        assert any("attention_into" in n for n in seen.names) and not any("dense_block" in n for n in seen.names)
+        calls = []
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: calls.append(type(m).__name__))
+        assert torch.equal(block(x), ref)
+        handle.remove()
+        assert "Mlp" in calls
+        block.attn.compute_attention = lambda **kw: torch.zeros(1, 20, 128, device=device, dtype=torch.bfloat16)
+        assert block._native_dense(x, None) is None and not torch.equal(block(x), ref)
+
+
+def test_operators_refuse_backward_and_vmap(vgo, device):
+    table = torch.randn(8, 16, device=device, requires_grad=True)
+    index = torch.zeros(5, 4, dtype=torch.int32, device=device)
+    weight = torch.rand(5, 4, device=device)
+    out = vgo.top4_project(table, index, weight)
+    with pytest.raises(RuntimeError):
+        out.sum().backward()
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda t: torch.ops.vgo.top4_project(t, index, weight))(torch.randn(2, 8, 16, device=device))

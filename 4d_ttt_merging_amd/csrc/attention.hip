@@ -656,6 +656,156 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_reg_kernel(AttnArgs<T> a)
     run(std::integral_constant<int, kQB>{});
 }
 
+// ------------------------------------------------- key-split kernel -------
+// Problems of few tasks (few_tasks): one work-group per 32 queries of one (batch, head),
+// its four waves sharing the queries and splitting the keys -- wave w runs
+// tiles w, w + 4, ... from a private LDS tile (loaded into registers a tile
+// ahead; a wave's LDS operations are in order, so the loop has no barrier) and
+// the four states are merged through LDS.  The bound there is the serial chain
+// of a task (load, then score, softmax and P.V per tile), not any pipe: a
+// quarter of the tiles in a row and eight times the work-groups of the
+// register-staged kernel.
+constexpr int kSplitQ = 32;           // queries per work-group
+constexpr int kSplitRow = kD + 4;     // padded fp32 row of a wave's state
+template <typename T>
+__global__ __launch_bounds__(kWaves * 64, 2) void attn_split_kernel(AttnArgs<T> a) {
+  typedef typename Mma<T>::op8 op8;
+  typedef typename Mma<T>::op4 op4;
+  __shared__ __attribute__((aligned(16))) T tile_lds[kWaves][2 * kTileElems];  // K, V^T per wave
+  __shared__ __attribute__((aligned(16))) float b_lds[kWaves][kBN];
+  __shared__ float m_lds[kWaves][kSplitQ], l_lds[kWaves][kSplitQ];
+  static_assert(sizeof(float) * kSplitQ * kSplitRow <= sizeof(T) * 2 * kTileElems, "state fits the tile");
+  const int task = static_cast<int>(xcd_remap(blockIdx.x, gridDim.x));
+  const int bh = task / a.n_qblocks;
+  const int qw0 = (task - bh * a.n_qblocks) * kSplitQ;
+  const int b = bh / a.heads;
+  const int h = bh - b * a.heads;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  T* kl = tile_lds[wave];
+  T* vl = kl + kTileElems;
+  float* bl = b_lds[wave];
+
+  // Pass i of a tile: K rows st and st + 32, V keys 2 st and 2 st + 1, chunk sc.
+  const int last_key = a.nk - 1;
+  const int ksn = static_cast<int>(a.ksn), vsn = static_cast<int>(a.vsn);
+  const int sc = lane & 7;
+  const T* kcol = a.k + b * a.ksb + h * a.ksh + 8 * sc;
+  const T* vcol = a.v + b * a.vsb + h * a.vsh + 8 * sc;
+  struct Pass {  // 16-byte chunks as words, which stay in registers across the loop
+    i32x4 k0, k1, v0, v1;
+  };
+  Pass p0, p1, p2, p3;
+  T pb = static_cast<T>(0.0f);
+  // Rows past n_key read a valid row; their bias is -inf.
+  auto load_pass = [&](Pass& p, int kt, int st) {
+    p.k0 = *reinterpret_cast<const i32x4*>(kcol + min(kt + st, last_key) * ksn);
+    p.k1 = *reinterpret_cast<const i32x4*>(kcol + min(kt + st + 32, last_key) * ksn);
+    p.v0 = *reinterpret_cast<const i32x4*>(vcol + min(kt + 2 * st, last_key) * vsn);
+    p.v1 = *reinterpret_cast<const i32x4*>(vcol + min(kt + 2 * st + 1, last_key) * vsn);
+  };
+  auto load = [&](int tile) {
+    const int kt = tile * kBN, st = lane >> 3;
+    load_pass(p0, kt, st);
+    load_pass(p1, kt, st + 8);
+    load_pass(p2, kt, st + 16);
+    load_pass(p3, kt, st + 24);
+    if (a.bias) pb = a.bias[min(kt + lane, last_key)];
+  };
+  auto store_pass = [&](const Pass& p, int st) {
+    *reinterpret_cast<i32x4*>(kl + st * kD + ((sc ^ swz(st)) << 3)) = p.k0;
+    *reinterpret_cast<i32x4*>(kl + (st + 32) * kD + ((sc ^ swz(st + 32)) << 3)) = p.k1;
+    const int vpos = vt_pos(2 * st);
+    const int vphys = (vpos >> 3) ^ sc;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      // Dim 8 sc + e of keys 2 st and 2 st + 1: the low or the high halves of word e / 2.
+      const uint32_t lo = p.v0[e >> 1], hi = p.v1[e >> 1];
+      *reinterpret_cast<uint32_t*>(vl + (8 * sc + e) * kD + (vpos & 7) + ((vphys ^ e) << 3)) =
+          __builtin_amdgcn_perm(hi, lo, e & 1 ? 0x07060302u : 0x05040100u);
+    }
+  };
+  auto store = [&](int tile) {
+    const int st = lane >> 3;
+    store_pass(p0, st);
+    store_pass(p1, st + 8);
+    store_pass(p2, st + 16);
+    store_pass(p3, st + 24);
+    const bool valid = tile * kBN + lane < a.nk;
+    bl[lane] = valid ? (a.bias ? to_f32(pb) : 0.0f) : -__builtin_inff();
+  };
+
+  WaveAttn<T, 1> w;
+  if (wave < a.ntiles) load(wave);
+  w.init(a.q + b * a.qsb + h * a.qsh, a.qsn, qw0, a.nq, a.c);
+  auto step = [&](auto first, int tile) {
+    store(tile);
+    __builtin_amdgcn_wave_barrier();
+    if (tile + kWaves < a.ntiles) load(tile + kWaves);
+    f32x16 s[1][2];
+    op8 p[1][4];
+    if constexpr (decltype(first)::value) {
+      w.template scores<true>(kl, bl, s);
+      w.softmax_first(s, p);
+    } else {
+      w.scores(kl, bl, s);
+      w.softmax(s, kl, bl, p);
+    }
+    w.pv(vl, p);
+    __builtin_amdgcn_wave_barrier();
+  };
+  if (wave < a.ntiles) {
+    step(std::true_type{}, wave);
+    for (int tile = wave + kWaves; tile < a.ntiles; tile += kWaves) step(std::false_type{}, tile);
+  }
+
+  // The wave's state over its own tile: O rows (fp32, unnormalised), mref and sum.
+  float* state = reinterpret_cast<float*>(kl);
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(state + w.l32 * kSplitRow + dt * 32 + 8 * g + 4 * w.hh) =
+          f32x4{w.o[0][dt][4 * g], w.o[0][dt][4 * g + 1], w.o[0][dt][4 * g + 2], w.o[0][dt][4 * g + 3]};
+  const float total = half_sum(w.lsum[0]);
+  if (w.hh == 0) {
+    m_lds[wave][w.l32] = w.mref[0];
+    l_lds[wave][w.l32] = total;
+  }
+  __syncthreads();
+  // Thread: dims 8 (tid % 8).. of query tid / 8.
+  const int ql = static_cast<int>(threadIdx.x) >> 3;
+  const int d0 = (static_cast<int>(threadIdx.x) & 7) * 8;
+  if (qw0 + ql >= a.nq) return;
+  float m = m_lds[0][ql];
+#pragma unroll
+  for (int i = 1; i < kWaves; ++i) m = fmaxf(m, m_lds[i][ql]);
+  float l = 0.0f;
+  f32x4 o0 = {0.0f, 0.0f, 0.0f, 0.0f}, o1 = o0;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) {
+    // m = -inf: no key has mass, every state is zero.
+    const float f = m == -__builtin_inff() ? 1.0f : __builtin_amdgcn_exp2f((m_lds[i][ql] - m) * kLog2e);
+    const float* src = reinterpret_cast<const float*>(tile_lds[i]) + ql * kSplitRow + d0;
+    const f32x4 x0 = *reinterpret_cast<const f32x4*>(src), x1 = *reinterpret_cast<const f32x4*>(src + 4);
+    l = fmaf(l_lds[i][ql], f, l);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o0[e] = fmaf(x0[e], f, o0[e]);
+      o1[e] = fmaf(x1[e], f, o1[e]);
+    }
+  }
+  T* dst = a.out + b * a.osb + h * a.osh + static_cast<int64_t>(qw0 + ql) * a.osn + d0;
+  op4 r0, r1;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    r0[e] = static_cast<T>(o0[e] / l);
+    r1[e] = static_cast<T>(o1[e] / l);
+  }
+  *reinterpret_cast<op4*>(dst) = r0;
+  *reinterpret_cast<op4*>(dst + 4) = r1;
+}
+
 // ------------------------------------------------- ping-pong kernel -------
 // Workspace path.  A task is 512 queries of one (batch, head): 8 waves x 64
 // queries in two groups of four; a SIMD holds one wave of each group (waves w
@@ -1246,6 +1396,25 @@ int launch_reg(const Problem& pr, hipStream_t stream) {
   return check_launch("mass_bias_attention");
 }
 
+// The key-split kernel runs where its work-groups are at most one and a half
+// rounds of the two it keeps resident per CU.  Measured (bf16, us, register-
+// staged / key-split kernel): 80 work-groups (160 x 160 x 16 heads) 8.6 / 4.7,
+// 272 (522 x 522) 18.1 / 10.4, 528 (1,044 x 522) 18.3 / 15.3, 576 (4 x 261 x 261)
+// 12.3 / 11.4, 704 (2 x 700 x 700) 20.6 / 15.6; past that the register-staged
+// kernel's larger tasks read K and V less often: 1,040 (2,058 x 1,029) 29.2 /
+// 31.3, 1,152 (8 x 261 x 261) 12.7 / 17.0, 1,408 (4 x 700 x 700) 21.4 / 26.4.
+int64_t split_tasks(const Problem& pr) { return (pr.nq + kSplitQ - 1) / kSplitQ * pr.batch * pr.heads; }
+bool few_tasks(const Problem& pr) { return split_tasks(pr) <= int64_t{device_cus()} * 3; }
+
+template <typename T>
+int launch_split(const Problem& pr, hipStream_t stream) {
+  VGO_REQUIRE(pr.nk < 0x7fffffff - kWaves * kBN, "mass_bias_attention: grid too large");
+  const AttnArgs<T> a = make_args<T>(pr, kSplitQ);
+  hipLaunchKernelGGL((attn_split_kernel<T>), dim3(static_cast<unsigned>(split_tasks(pr))), dim3(kWaves * 64), 0,
+                     stream, a);
+  return check_launch("mass_bias_attention");
+}
+
 // Kernel timing (vgo_attn_kernel_timing): while it is on, every attn_pp_kernel
 // launch made outside stream capture on the device it was switched on for is
 // bracketed by a pair of HIP events from a fixed pool, so the kernel's own
@@ -1419,7 +1588,9 @@ int attn_run(const Problem* problems, const int64_t* head_dims, int count, int d
     return dtype == VGO_BF16 ? launch_pp<bf16_t>(live, n, workspace, workspace_bytes, s)
                              : launch_pp<f16_t>(live, n, workspace, workspace_bytes, s);
   for (int i = 0; i < n; ++i) {
-    const int status = dtype == VGO_BF16 ? launch_reg<bf16_t>(live[i], s) : launch_reg<f16_t>(live[i], s);
+    const int status = few_tasks(live[i])
+                           ? (dtype == VGO_BF16 ? launch_split<bf16_t>(live[i], s) : launch_split<f16_t>(live[i], s))
+                           : (dtype == VGO_BF16 ? launch_reg<bf16_t>(live[i], s) : launch_reg<f16_t>(live[i], s));
     if (status != VGO_OK) return status;
   }
   return VGO_OK;

@@ -27,6 +27,44 @@
 namespace vgo {
 namespace {
 
+// The dictionary split of a launch whose source count is only known on the
+// device (n_src is its bound): every work-group, and the merge of the lists after
+// them, derives it from the count it reads, and only the count's tasks run, spread
+// over all XCDs.  (With the bound's split and remap, a tenth of the sources kept one
+// XCD's CUs busy for as long as all of them would have: top-4 of 2,380 of 23,808
+// sources against 8,960 rows 504 us, now 110; of 15,000 of 150,000 against 52,000
+// 12.9 ms, now 1.8.)  parts x count stays within the `lists` the workspace holds.
+struct DeviceSplit {
+  int slots = 0;      // resident work-groups
+  int64_t lists = 0;  // n_src x the host's parts
+};
+// The split that costs least, (rounds of resident work-groups) x (dictionary tiles per part +
+// a half-tile fixed cost) as choose_parts, among those that fill one to four rounds and, for
+// many source tiles, a few small ones.
+__host__ __device__ __forceinline__ int device_parts(const DeviceSplit& s, int count, int tile, int n_dict) {
+  const int src_tiles = (count + tile - 1) / tile;
+  const int dict_tiles = (n_dict + tile - 1) / tile;
+  if (src_tiles <= 0) return 1;
+  const int cap = static_cast<int>(s.lists / count < dict_tiles ? s.lists / count : dict_tiles);
+  int best = 1, best_cost = 0x7fffffff;
+  const int tries = 2 * src_tiles > s.slots ? 8 : 4;
+  for (int t = 1; t <= tries; ++t) {
+    int p = t <= 4 ? s.slots * t / src_tiles : 2 * (t - 4);
+    p = p < 1 ? 1 : p > cap ? cap : p;
+    const int cost = (src_tiles * p + s.slots - 1) / s.slots * (2 * ((dict_tiles + p - 1) / p) + 1);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = p;
+    }
+  }
+  return best;
+}
+// Work-groups that cover device_parts x source tiles for every count up to src_tiles tiles.
+inline int64_t device_groups(const DeviceSplit& s, int64_t src_tiles) {
+  return 2 * src_tiles > s.slots ? std::max<int64_t>(8 * src_tiles, int64_t{4} * s.slots)
+                                 : int64_t{4} * s.slots;
+}
+
 constexpr int kTile = 128;       // dictionary rows and source rows per work-group step
 constexpr int kKc = 64;          // K chunk staged in LDS
 
@@ -128,17 +166,24 @@ __global__ __launch_bounds__(256, 2) void sim_topk_kernel(
     const bf16_t* __restrict__ dict,
     int64_t dict_stride, int n0, int off1, int n_dict, int dim, int tiles_per_part,
     uint64_t* __restrict__ partial, int parts, bf16_t* __restrict__ scores,
-    int64_t scores_stride) {
+    int64_t scores_stride, DeviceSplit split) {
   // Double-buffered dictionary (a) and source (b) chunks.
   __shared__ __attribute__((aligned(16))) bf16_t a_lds[2 * kTileElems];
   __shared__ __attribute__((aligned(16))) bf16_t b_lds[2 * kTileElems];
 
   int ns = n_src;
-  if (n_src_dev) ns = min(ns, *n_src_dev);
+  int tasks = gridDim.x;
+  if (n_src_dev) {
+    ns = min(ns, *n_src_dev);
+    parts = device_parts(split, ns, kTile, n_dict);
+    tiles_per_part = ((n_dict + kTile - 1) / kTile + parts - 1) / parts;
+    tasks = (ns + kTile - 1) / kTile * parts;
+    if (static_cast<int>(blockIdx.x) >= tasks) return;
+  }
   // 1-D grid, dictionary part fastest, XCD-remapped: the work-groups resident
   // on one XCD at a time cover a few source tiles (kept in its L2 across their
   // dictionary tiles) against all dictionary parts.
-  const int task = xcd_remap(blockIdx.x, gridDim.x);
+  const int task = xcd_remap(blockIdx.x, tasks);
   const int s0 = (task / parts) * kTile;
   if (s0 >= ns) return;
   const int part = task % parts;
@@ -402,14 +447,25 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
     const bf16_t* __restrict__ dict,
     int64_t dict_stride, int n0, int off1, int n_dict, int dim, int tiles_per_part,
     uint64_t* __restrict__ partial, int parts, bf16_t* __restrict__ scores,
-    int64_t scores_stride, int units) {
+    int64_t scores_stride, int units, DeviceSplit split) {
   static_assert(!kStreamK || K == 1, "the stream-K schedule is the top-1 kernel's");
   __shared__ __attribute__((aligned(16))) bf16_t a_lds[kRStages * kRTileElems];
   __shared__ __attribute__((aligned(16))) bf16_t b_lds[kRStages * kRTileElems];
 
   int ns = n_src;
-  if (n_src_dev) ns = min(ns, *n_src_dev);
-  const int task = xcd_remap(blockIdx.x, gridDim.x);
+  int tasks = gridDim.x;
+  if (n_src_dev) {
+    ns = min(ns, *n_src_dev);
+    if constexpr (!kStreamK) {
+      // Only the tasks of the sources there are, over all XCDs: remapping the whole
+      // grid would leave a small count to the first XCD.
+      parts = device_parts(split, ns, kRTile, n_dict);
+      tiles_per_part = ((n_dict + kRTile - 1) / kRTile + parts - 1) / parts;
+      tasks = (ns + kRTile - 1) / kRTile * parts;
+      if (static_cast<int>(blockIdx.x) >= tasks) return;
+    }
+  }
+  const int task = xcd_remap(blockIdx.x, tasks);
   // kStreamK: tiles_per_part is the dictionary's tile count; st_begin / dt_begin
   // are the first unit's tiles, slot_begin the first segment's slot (a later
   // segment starts its source tile, whose first owner is then this work-group).
@@ -874,16 +930,18 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
 // With sk_groups > 0 the lists come from the stream-K top-1 ring kernel: row i's
 // source tile was split over work-groups first..last of the schedule, which
 // wrote four lists each into slots 0 .. last - first of the row's `parts`.
+constexpr int kFinalizeThreads = 64;  // rows per work-group: small counts still spread over the chip
 template <int K>
-__global__ __launch_bounds__(256) void topk_finalize_kernel(
+__global__ __launch_bounds__(kFinalizeThreads) void topk_finalize_kernel(
     const uint64_t* __restrict__ partial, int n_src, const int* __restrict__ n_src_dev, int parts,
     int n0, int off1, float* __restrict__ values, int64_t* __restrict__ index64,
     int32_t* __restrict__ index32, const int64_t* __restrict__ index_map, int sk_units, int sk_groups,
-    int sk_dict_tiles) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
+    int sk_dict_tiles, DeviceSplit split, int tile, int n_dict) {
+  const int i = blockIdx.x * kFinalizeThreads + threadIdx.x;
   int ns = n_src;
   if (n_src_dev) ns = min(ns, *n_src_dev);
   if (i >= ns) return;
+  if (n_src_dev && sk_groups == 0) parts = device_parts(split, ns, tile, n_dict);
   int used = parts;
   if (sk_groups > 0) {
     const int64_t u0 = static_cast<int64_t>(i / kRTile) * sk_dict_tiles;
@@ -893,7 +951,22 @@ __global__ __launch_bounds__(256) void topk_finalize_kernel(
   TopK<K> m;
   m.init();
   const uint64_t* p = partial + static_cast<int64_t>(i) * parts * K;
-  for (int q = 0; q < used * K; ++q) m.insert(p[q]);
+  // Four lists' keys are loaded ahead of their inserts; a list is in descending
+  // order, so its tail is skipped once a key does not enter.
+  for (int q = 0; q < used; q += 4) {
+    uint64_t k[4][K];
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+#pragma unroll
+      for (int t = 0; t < K; ++t) k[l][t] = q + l < used ? p[(q + l) * K + t] : 0ull;
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+#pragma unroll
+      for (int t = 0; t < K; ++t) {
+        if (k[l][t] <= m.k[K - 1]) break;
+        m.insert(k[l][t]);
+      }
+  }
 #pragma unroll
   for (int t = 0; t < K; ++t) {
     const uint64_t key = m.k[t];
@@ -932,8 +1005,16 @@ int64_t resident_groups(bool ring) {
   return cache[ring][dev];
 }
 
-// The ring kernel runs when the dimension is a whole number of its K chunks.
-inline bool use_ring(int64_t dim) { return dim % kRKc == 0; }
+// The ring kernel runs when the dimension is a whole number of its K chunks, except
+// for few tiles: one 256 x 256 tile takes the ring 28 us (top-1) to 45 us (top-4),
+// a 128 x 128 tile of the staged kernel 17 and 30 us, and both leave CUs idle there.
+// Measured (us, top-1 / top-4, ring against staged, dim 1,024): 576 x 448 33 / 60
+// against 22 / 35, 2,304 x 1,000 (36 ring tiles) 34 / 63 against 24 / 40, 2,304 x
+// 2,304 (81) 33 / 54 against 31 / 59, 5,544 x 1,500 (132) 37 / 66 against 48 / 72.
+constexpr int64_t kStagedTiles = 64;
+inline bool use_ring(int64_t n_src, int64_t n_dict, int64_t dim) {
+  return dim % kRKc == 0 && (n_src + kRTile - 1) / kRTile * ((n_dict + kRTile - 1) / kRTile) > kStagedTiles;
+}
 
 // Dictionary split for a kernel with `tile` x `tile` steps: the number of parts
 // that minimises (rounds of resident work-groups) x (dictionary tiles per
@@ -1034,8 +1115,8 @@ extern "C" int vgo_similarity_topk(const void* src, int64_t src_row_stride, int6
                   dict_off1 + (n_dict - dict_n0) <= dict_capacity,
               "similarity_topk: dictionary ranges exceed the dictionary");
   VGO_REQUIRE(src_rows || n_src <= src_capacity, "similarity_topk: more sources than rows");
-  const bool ring = use_ring(dim);
-  const StreamK sk = ring && topk == 1 && !scores ? stream_k_schedule(n_src, n_dict) : StreamK{};
+  const bool ring = use_ring(n_src, n_dict, dim);
+  const StreamK sk = ring && topk == 1 && !scores && !n_src_device ? stream_k_schedule(n_src, n_dict) : StreamK{};
   const int parts = sk.groups > 0 ? sk.lists : choose_parts(n_src, n_dict, topk, ring);
   const size_t need = static_cast<size_t>(n_src) * parts * topk * sizeof(uint64_t);
   VGO_REQUIRE(workspace && workspace_bytes >= need, "similarity_topk: workspace too small");
@@ -1046,12 +1127,19 @@ extern "C" int vgo_similarity_topk(const void* src, int64_t src_row_stride, int6
   hipStream_t s = as_stream(stream);
   const int64_t src_tiles = (n_src + tile - 1) / tile;
   VGO_REQUIRE(src_tiles * parts < (1LL << 31), "similarity_topk: grid too large");
-  dim3 grid(static_cast<unsigned>(sk.groups > 0 ? sk.groups : src_tiles * parts));
+  DeviceSplit split;
+  int64_t groups = sk.groups > 0 ? sk.groups : src_tiles * parts;
+  if (n_src_device) {
+    split.slots = static_cast<int>(topk == 1 ? resident_groups<1>(ring) : resident_groups<4>(ring));
+    split.lists = n_src * parts;
+    groups = device_groups(split, src_tiles);
+  }
+  dim3 grid(static_cast<unsigned>(groups));
   uint64_t* partial = static_cast<uint64_t*>(workspace);
   const bf16_t* sp = static_cast<const bf16_t*>(src);
   const bf16_t* dp = static_cast<const bf16_t*>(dict);
   bf16_t* sc = static_cast<bf16_t*>(scores);
-  const int blocks2 = static_cast<int>((n_src + 255) / 256);
+  const int blocks2 = static_cast<int>((n_src + kFinalizeThreads - 1) / kFinalizeThreads);
   if (ring) {
     // 64-bit row addresses per lane; the DMA reads stay inside the buffers
     // (rows are clamped, dim is a multiple of the chunk).
@@ -1059,7 +1147,7 @@ extern "C" int vgo_similarity_topk(const void* src, int64_t src_row_stride, int6
       hipLaunchKernelGGL(kernel, grid, dim3(kRWaves * 64), 0, s, sp, src_row_stride, src_capacity, src_rows,
                          n_src_device, static_cast<int>(n_src), dp, dict_row_stride, static_cast<int>(dict_n0),
                          static_cast<int>(dict_off1), static_cast<int>(n_dict), static_cast<int>(dim),
-                         tiles_per_part, partial, parts, sc, scores_row_stride, sk.units);
+                         tiles_per_part, partial, parts, sc, scores_row_stride, sk.units, split);
     };
     if (sk.groups > 0)
       launch(sim_topk_ring_kernel<1, true>);
@@ -1072,22 +1160,23 @@ extern "C" int vgo_similarity_topk(const void* src, int64_t src_row_stride, int6
                        n_src_device, static_cast<int>(n_src), dp, dict_row_stride,
                        static_cast<int>(dict_n0), static_cast<int>(dict_off1),
                        static_cast<int>(n_dict), static_cast<int>(dim), tiles_per_part, partial,
-                       parts, sc, scores_row_stride);
+                       parts, sc, scores_row_stride, split);
   } else {
     hipLaunchKernelGGL((sim_topk_kernel<4>), grid, dim3(256), 0, s, sp, src_row_stride, src_capacity, src_rows,
                        n_src_device, static_cast<int>(n_src), dp, dict_row_stride,
                        static_cast<int>(dict_n0), static_cast<int>(dict_off1),
                        static_cast<int>(n_dict), static_cast<int>(dim), tiles_per_part, partial,
-                       parts, sc, scores_row_stride);
+                       parts, sc, scores_row_stride, split);
   }
   if (topk == 1)
-    hipLaunchKernelGGL((topk_finalize_kernel<1>), dim3(blocks2), dim3(256), 0, s, partial,
+    hipLaunchKernelGGL((topk_finalize_kernel<1>), dim3(blocks2), dim3(kFinalizeThreads), 0, s, partial,
                        static_cast<int>(n_src), n_src_device, parts, static_cast<int>(dict_n0),
                        static_cast<int>(dict_off1), values, index64, index32, index_map, sk.units, sk.groups,
-                       sk.dict_tiles);
+                       sk.dict_tiles, split, static_cast<int>(tile), static_cast<int>(n_dict));
   else
-    hipLaunchKernelGGL((topk_finalize_kernel<4>), dim3(blocks2), dim3(256), 0, s, partial,
+    hipLaunchKernelGGL((topk_finalize_kernel<4>), dim3(blocks2), dim3(kFinalizeThreads), 0, s, partial,
                        static_cast<int>(n_src), n_src_device, parts, static_cast<int>(dict_n0),
-                       static_cast<int>(dict_off1), values, index64, index32, index_map, 0, 0, 0);
+                       static_cast<int>(dict_off1), values, index64, index32, index_map, 0, 0, 0, split,
+                       static_cast<int>(tile), static_cast<int>(n_dict));
   return check_launch("similarity_topk");
 }

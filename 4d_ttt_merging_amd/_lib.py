@@ -109,6 +109,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_size,
         _c_p,
     ]),
+    "vgo_fastvggt_plan_fits": (_c_int, [_c_i64, _c_i64, _c_i64]),
+    "vgo_fastvggt_plan": (_c_int, [
+        _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p,
+        _c_p, _c_p,
+    ]),
     "vgo_sparse_convex_assemble": (_c_int, [
         _c_p, _c_p, _c_p, _c_p, _c_p, _c_f32, _c_p, _c_i64, _c_i64, _c_f32, _c_p, _c_p, _c_p,
         _c_p, _c_p, _c_p, _c_p,

@@ -710,8 +710,298 @@ __global__ __launch_bounds__(kAThreads) void fva_inverse_kernel(const int32_t* _
     if (sid[k] >= 0 && sid[k] < total) inv[sid[k]] = (dst[k] >= 0 && dst[k] < total) ? inv[dst[k]] : -1;
 }
 
+// ---------------------------------------------------------------------------
+// A whole FastVGGT plan of one batch element in one launch of one work-group: the
+// selection and keep / inverse above, the stable CSR of the clusters, their
+// sizes and log sizes.  As launches these are twenty kernels, all latency: 28 us
+// assembly, 24-31 us CSR and 8 us mass and int32 inverse at up to 12,288 tokens,
+// and 3-4 us of host time for each.  Here every step between two barriers runs
+// in one CU's LDS: 16 us at 1,044 tokens, 17 at 2,632, 31 at 8,528 (54 with
+// every token on one destination).  Its time grows by 2 us per 1,024 tokens, the
+// launches' hardly: 70 us against 73 at 20,580 tokens, 97 against 73 at 32,928,
+// so larger plans take the launches.
+//
+//  * The removed-th largest key by binary search on its bits: a count per bit
+//    is one ballot per 64 keys (held in registers), where a digit histogram
+//    serialises on the few digits that bf16-rounded scores occupy.
+//  * val[t] (u16): a kept token's compact id, a removed one's destination.
+//  * Cluster order: a token's slot within its cluster comes from an LDS counter
+//    in any order; its rank among the cluster's tokens is then counted, except
+//    for clusters over kBigCluster tokens, whose tokens a wave collects in
+//    order from one pass over all of them (identical frames put thousands of
+//    tokens on one destination).
+// Results equal the launches' bit for bit.
+constexpr int kPlanChunks = 12;                      // tokens <= 12 x 1024
+constexpr int kBigCluster = 128;
+
+struct PlanLds {
+  int val_at, cnt_at, bits_at, bytes;  // byte offsets of val u16[total], cnt u16[kept + 2], removed bits
+};
+__host__ __device__ inline PlanLds plan_lds(int total, int kept) {
+  PlanLds l;
+  l.val_at = 0;
+  l.cnt_at = (2 * total + 15) / 16 * 16;
+  l.bits_at = l.cnt_at + (2 * (kept + 2) + 15) / 16 * 16;
+  l.bytes = l.bits_at + (total + 31) / 32 * 4;
+  return l;
+}
+constexpr int kPlanLds = 52 * 1024;  // >= plan_lds(kPlanChunks x kThreads, all of them kept).bytes
+inline bool plan_fits(int64_t n_sources, int64_t total, int64_t removed) {
+  return total <= kPlanChunks * kThreads && n_sources <= total && removed <= n_sources;
+}
+
+// C: chunks of 1,024 tokens (and of sources) the loops are unrolled for; a small plan's time is
+// mostly the fetch of the code it runs through.
+template <int C>
+__global__ __launch_bounds__(kThreads) void fastvggt_plan_kernel(
+    const float* __restrict__ best, const int32_t* __restrict__ target,
+    const int64_t* __restrict__ source_ids, const int64_t* __restrict__ dest_ids, int ns, int nd, int total,
+    int removed, int64_t* __restrict__ keep, int64_t* __restrict__ inverse, int32_t* __restrict__ inverse32,
+    uint8_t* __restrict__ removed_flag, uint32_t* __restrict__ order, int32_t* __restrict__ offsets,
+    float* __restrict__ mass, float* __restrict__ log_mass) {
+  __shared__ __attribute__((aligned(16))) uint32_t state[kPlanLds / 4];
+  __shared__ int counts[2][kWavesS];
+  __shared__ int chunk_cnt[kPlanChunks * kWavesS];
+  __shared__ int scan_lds[kWavesS];
+  __shared__ int big[kPlanChunks * kThreads / kBigCluster];
+  __shared__ int n_big;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint64_t below = (1ull << lane) - 1ull;
+  const int kept = total - removed;
+  const PlanLds at = plan_lds(total, kept);
+  uint16_t* val = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(state) + at.val_at);
+  uint16_t* cnt = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(state) + at.cnt_at);
+  uint32_t* cnt32 = reinterpret_cast<uint32_t*>(cnt);
+  uint32_t* bits = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(state) + at.bits_at);
+  const int s_chunks = (ns + kThreads - 1) / kThreads;
+  const int t_chunks = (total + kThreads - 1) / kThreads;
+
+  for (int i = tid; i < (at.bytes - at.cnt_at) / 4; i += kThreads) cnt32[i] = 0;  // counters and bits
+  if (tid == 0) n_big = 0;
+
+  // ---- keys; the removed-th largest of them.
+  uint32_t key[C];  // 0 past the sources: below every key
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int i = c * kThreads + tid;
+    key[c] = c < s_chunks && i < ns ? ord32(best[i]) : 0u;
+  }
+  int round = 0;
+  auto count_from = [&](uint32_t bound) {  // keys >= bound (> 0), the same in every thread
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      if (c < s_chunks) n += __popcll(__ballot(key[c] >= bound));
+    if (lane == 0) counts[round & 1][wave] = n;
+    __syncthreads();
+    int sum = 0;
+#pragma unroll
+    for (int w = 0; w < kWavesS; ++w) sum += counts[round & 1][w];
+    ++round;
+    return sum;
+  };
+  uint32_t thresh = 0;
+  for (int bit = 31; bit >= 16; --bit)
+    if (count_from(thresh | (1u << bit)) >= removed) thresh |= 1u << bit;
+  // bf16 scores differ in the high half only (the low half of a negative one is all ones).
+  if (count_from(thresh | 0xFFFFu) >= removed) {
+    thresh |= 0xFFFFu;
+  } else if (count_from(thresh | 1u) >= removed) {
+    for (int bit = 15; bit >= 0; --bit)
+      if (count_from(thresh | (1u << bit)) >= removed) thresh |= 1u << bit;
+  }
+  const int need_ties = removed - (thresh == 0xFFFFFFFFu ? 0 : count_from(thresh + 1));
+
+  // ---- ranks of the ties, in source order.
+  // In-place exclusive scan of chunk_cnt[0, chunks x waves) -> each (chunk, wave)'s base.
+  auto scan_chunks = [&](int chunks) {
+    __syncthreads();
+    const int n = chunks * kWavesS;
+    int sum = 0;
+    const int mine = tid < n ? chunk_cnt[tid] : 0;  // n <= 640
+    const int pre = block_exclusive_scan(mine, scan_lds, &sum);
+    if (tid < n) chunk_cnt[tid] = pre;
+    __syncthreads();
+  };
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    if (c < s_chunks) {
+      const uint64_t m = __ballot(key[c] == thresh);
+      if (lane == 0) chunk_cnt[c * kWavesS + wave] = __popcll(m);
+    }
+  scan_chunks(s_chunks);
+  // ---- removed sources and their destinations (0xFFFF: not a token).  Four chunks' ids are
+  // loaded together, whether their sources are removed or not.
+#pragma unroll
+  for (int c0 = 0; c0 < C; c0 += 4)
+    if (c0 < s_chunks) {
+      int64_t sid[4], dst[4];
+      int32_t d[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int i = min((c0 + q) * kThreads + tid, ns - 1);
+        sid[q] = source_ids[i];
+        d[q] = target[i];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bool ok = d[q] >= 0 && d[q] < nd;
+        dst[q] = nd > 0 ? dest_ids[ok ? d[q] : 0] : -1;
+        if (!ok || dst[q] < 0 || dst[q] >= total) dst[q] = 0xFFFF;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int c = c0 + q;
+        if (c >= s_chunks) continue;
+        const int i = c * kThreads + tid;
+        const uint64_t m = __ballot(key[c] == thresh);
+        const int rank = chunk_cnt[c * kWavesS + wave] + __popcll(m & below);
+        const bool rm = i < ns && (key[c] > thresh || (key[c] == thresh && rank < need_ties));
+        if (i < ns) removed_flag[i] = rm ? 1 : 0;
+        if (rm && sid[q] >= 0 && sid[q] < total) {
+          atomicOr(&bits[sid[q] >> 5], 1u << (sid[q] & 31));
+          val[sid[q]] = static_cast<uint16_t>(dst[q]);
+        }
+      }
+    }
+  __syncthreads();
+
+  // ---- compact ids of the kept tokens, ascending; the keep list.
+  auto is_removed = [&](int t) { return ((bits[t >> 5] >> (t & 31)) & 1u) != 0u; };
+  for (int c = 0; c < t_chunks; ++c) {
+    const int t = c * kThreads + tid;
+    const uint64_t m = __ballot(t < total && !is_removed(t));
+    if (lane == 0) chunk_cnt[c * kWavesS + wave] = __popcll(m);
+  }
+  scan_chunks(t_chunks);
+  for (int c = 0; c < t_chunks; ++c) {
+    const int t = c * kThreads + tid;
+    const bool k = t < total && !is_removed(t);
+    const uint64_t m = __ballot(k);
+    const int rank = chunk_cnt[c * kWavesS + wave] + __popcll(m & below);
+    if (k) {
+      val[t] = static_cast<uint16_t>(rank);
+      if (rank < kept) keep[rank] = t;  // always true for a valid (disjoint) source list
+    }
+  }
+  __syncthreads();
+
+  // ---- inverse, and every token's cluster and slot in it (a token without one: cluster `kept`).
+  uint32_t place[C];  // cluster | slot << 16
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int t = c * kThreads + tid;
+    place[c] = 0;
+    if (c < t_chunks && t < total) {
+      int k = val[t];
+      if (is_removed(t)) k = k == 0xFFFF || is_removed(k) ? -1 : val[k];
+      if (k >= kept) k = -1;
+      inverse[t] = k;
+      inverse32[t] = k;
+      const int cluster = k < 0 ? kept : k;
+      const int shift = 16 * (cluster & 1);
+      const uint32_t old = atomicAdd(&cnt32[cluster >> 1], 1u << shift);
+      place[c] = static_cast<uint32_t>(cluster) | (((old >> shift) & 0xFFFFu) << 16);
+    }
+  }
+  __syncthreads();
+
+  // ---- cluster sizes -> offsets (in place), masses.
+  const int per = (kept + 1 + kThreads - 1) / kThreads;
+  const int k0 = min(kept + 1, tid * per), k1 = min(kept + 1, k0 + per);
+  int sum = 0;
+  for (int k = k0; k < k1; ++k) {
+    const int n = cnt[k];
+    sum += n;
+    if (n > kBigCluster) big[atomicAdd(&n_big, 1)] = k;
+  }
+  int all = 0;
+  int run = block_exclusive_scan(sum, scan_lds, &all);
+  for (int k = k0; k < k1; ++k) {
+    const int n = cnt[k];
+    cnt[k] = static_cast<uint16_t>(run);
+    run += n;
+  }
+  if (tid == 0) cnt[kept + 1] = static_cast<uint16_t>(total);
+  __syncthreads();
+  for (int k = tid; k <= kept; k += kThreads) {
+    offsets[k] = cnt[k];
+    if (k < kept) {
+      const float m = static_cast<float>(cnt[k + 1] - cnt[k]);
+      mass[k] = m;
+      log_mass[k] = logf(m);
+    }
+  }
+
+  // ---- cluster members in token order (val's space holds the members now).
+  uint16_t* slot = val;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int t = c * kThreads + tid;
+    if (c < t_chunks && t < total) slot[cnt[place[c] & 0xFFFFu] + (place[c] >> 16)] = static_cast<uint16_t>(t);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int t = c * kThreads + tid;
+    if (c < t_chunks && t < total) {
+      const int cluster = place[c] & 0xFFFFu;
+      const int b = cnt[cluster], e = cnt[cluster + 1];
+      if (e - b <= kBigCluster) {
+        int rank = 0;
+        for (int j = b; j < e; ++j) rank += slot[j] < t;
+        order[b + rank] = static_cast<uint32_t>(t);
+      }
+    }
+  }
+  for (int g = wave; g < n_big; g += kWavesS) {
+    const int cluster = big[g];
+    int pos = cnt[cluster];
+    for (int t0 = 0; t0 < total; t0 += 64) {
+      const int t = t0 + lane;
+      const bool mine = t < total && (cluster == kept ? inverse32[t] < 0 : inverse32[t] == cluster);
+      const uint64_t m = __ballot(mine);
+      if (mine) order[pos + __popcll(m & below)] = static_cast<uint32_t>(t);
+      pos += __popcll(m);
+    }
+  }
+}
+
 }  // namespace
 }  // namespace vgo
+
+extern "C" int vgo_fastvggt_plan_fits(int64_t n_sources, int64_t total_tokens, int64_t removed) {
+  return n_sources >= 1 && removed >= 1 && vgo::plan_fits(n_sources, total_tokens, removed) ? 1 : 0;
+}
+
+extern "C" int vgo_fastvggt_plan(const float* best, const int32_t* target, const int64_t* source_ids,
+                                 const int64_t* dest_ids, int64_t n_sources, int64_t n_dest,
+                                 int64_t total_tokens, int64_t removed, int64_t* keep, int64_t* inverse,
+                                 int32_t* inverse32, uint8_t* removed_flag, uint32_t* order,
+                                 int32_t* offsets, float* mass, float* log_mass, void* stream) {
+  using namespace vgo;
+  VGO_REQUIRE(n_sources >= 0 && n_dest >= 0 && total_tokens >= 0, "fastvggt_plan: negative size");
+  VGO_REQUIRE(removed >= 1 && removed <= n_sources, "fastvggt_plan: removed must lie in [1, sources]");
+  VGO_REQUIRE(n_sources + n_dest <= total_tokens && total_tokens < (1LL << 30),
+              "fastvggt_plan: inconsistent token counts");
+  VGO_REQUIRE(best && target && source_ids && dest_ids && keep && inverse && inverse32 && removed_flag && order &&
+                  offsets && mass && log_mass,
+              "fastvggt_plan: null pointer");
+  if (!plan_fits(n_sources, total_tokens, removed))
+    return fail(VGO_EUNSUPPORTED, "fastvggt_plan: too many tokens for one work-group");
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kThreads), 0, as_stream(stream), best, target, source_ids, dest_ids,
+                       static_cast<int>(n_sources), static_cast<int>(n_dest), static_cast<int>(total_tokens),
+                       static_cast<int>(removed), keep, inverse, inverse32, removed_flag, order, offsets, mass,
+                       log_mass);
+  };
+  if (total_tokens <= 4 * kThreads)
+    launch(fastvggt_plan_kernel<4>);
+  else
+    launch(fastvggt_plan_kernel<kPlanChunks>);
+  return check_launch("fastvggt_plan");
+}
 
 extern "C" int vgo_fastvggt_assemble(const float* best, const int32_t* target,
                                      const int64_t* source_ids, const int64_t* dest_ids,

@@ -561,6 +561,29 @@ std::tuple<Tensor, Tensor, Tensor> fastvggt_assemble(const Tensor& best, const T
   return {keep, inverse, flags};
 }
 
+// fastvggt_assemble of one batch element with its clusters' CSR, sizes and log sizes from one
+// launch: (keep, inverse, flags, inverse as int32, order, offsets, mass, log_mass).
+std::vector<Tensor> fastvggt_plan(const Tensor& best, const Tensor& target, const Tensor& sources,
+                                  const Tensor& destinations, int64_t total, int64_t removed) {
+  require_gpu({&best, &target, &sources, &destinations});
+  const int64_t n_src = sources.numel(), kept = total - removed;
+  TORCH_CHECK_VALUE(best.is_contiguous() && target.is_contiguous() && sources.is_contiguous() &&
+                        destinations.is_contiguous() && best.scalar_type() == at::kFloat &&
+                        target.scalar_type() == at::kInt && sources.scalar_type() == at::kLong &&
+                        destinations.scalar_type() == at::kLong && best.numel() == n_src && target.numel() == n_src &&
+                        kept >= 0,
+                    "fastvggt_plan: contiguous fp32 scores and int32 targets [1, n], int64 ids");
+  const auto ids = sources.options(), i32 = ids.dtype(at::kInt), f32s = ids.dtype(at::kFloat);
+  std::vector<Tensor> r = {at::empty({1, kept}, ids),   at::empty({1, total}, ids), at::empty({1, n_src}, ids.dtype(at::kByte)),
+                           at::empty({total}, i32),     at::empty({total}, i32),    at::empty({kept + 1}, i32),
+                           at::empty({kept}, f32s),     at::empty({kept}, f32s)};
+  check(vgo_fastvggt_plan(ptr<float>(best), ptr<int32_t>(target), ptr<int64_t>(sources), ptr<int64_t>(destinations),
+                          n_src, destinations.numel(), total, removed, ptr<int64_t>(r[0]), ptr<int64_t>(r[1]),
+                          ptr<int32_t>(r[3]), ptr<uint8_t>(r[2]), ptr<uint32_t>(r[4]), ptr<int32_t>(r[5]),
+                          ptr<float>(r[6]), ptr<float>(r[7]), stream_of(best)));
+  return r;
+}
+
 // A merged block (block.py:219-226 under bf16 / f16 autocast) on an fp32 stream x [1, N, C] with a
 // token plan: norm1 and the qkv projection unless given, compaction of the clusters (offsets,
 // order, counts, contribution), mass-bias attention, the output projection, restore (inverse)
@@ -609,7 +632,8 @@ void no_batching(const c10::OperatorHandle& op, c10::DispatchKeySet, torch::jit:
 
 constexpr const char* kPure[] = {"mass_bias_attention", "top4_project", "qkv_epilogue", "residual_layer_norm",
                                  "restore_residual_layer_norm", "mlp_tail", "dense_block", "normalize_rows",
-                                 "csr_build", "segment_mass", "fastvggt_assemble", "fastvggt_match", "merged_block"};
+                                 "csr_build", "segment_mass", "fastvggt_assemble", "fastvggt_match", "fastvggt_plan",
+                                 "merged_block"};
 constexpr const char* kMutating[] = {"attention_into", "attention_pair_into", "top4_project_into",
                                      "top4_project_ordered_into", "compact_into", "compact_multi_into", "similarity_topk"};
 
@@ -634,6 +658,7 @@ TORCH_LIBRARY_IMPL(vgo, CUDA, m) {
   m.impl("segment_mass", segment_mass);
   m.impl("fastvggt_assemble", fastvggt_assemble);
   m.impl("fastvggt_match", fastvggt_match);
+  m.impl("fastvggt_plan", fastvggt_plan);
   m.impl("similarity_topk", similarity_topk);
   m.impl("merged_block", merged_block);
 }

@@ -24,7 +24,7 @@ dispatcher, `torch.compile` and fake-tensor tracing see them as single ops:
   last residual pass, a whole unmerged block (layers/block.py:89-129) and a whole
   merged block over a token plan (:219-226), for eager inference; and the plan
   builders' kernels (`vgo::normalize_rows`, `similarity_topk`, `fastvggt_match`,
-  `fastvggt_assemble`, `csr_build`, `segment_mass`).
+  `fastvggt_assemble`, `fastvggt_plan`, `csr_build`, `segment_mass`).
 
 The CUDA (HIP) implementations are native (csrc/torch_ops.cpp, built into
 `libvgo_torch.so`) and call `libvgo.so` through its C ABI.  The operators a
@@ -93,6 +93,8 @@ _SCHEMAS = (
     "bool want_log) -> (Tensor, Tensor)",
     "fastvggt_assemble(Tensor best, Tensor target, Tensor sources, Tensor destinations, int total, "
     "int removed) -> (Tensor, Tensor, Tensor)",
+    "fastvggt_plan(Tensor best, Tensor target, Tensor sources, Tensor destinations, int total, "
+    "int removed) -> Tensor[]",
 )
 
 _library = torch.library.Library("vgo", "DEF")
@@ -207,3 +209,13 @@ def _(keys, n_buckets):
 def _(offsets, segs_per_row, order, weights, rows, start, want_log):
     return (offsets.new_empty((rows,), dtype=torch.float32),
             offsets.new_empty((rows if want_log else 0,), dtype=torch.float32))
+
+
+@_fake("fastvggt_plan")
+def _(best, target, sources, destinations, total, removed):
+    kept, n_src = total - removed, sources.numel()
+    i32, f32 = dict(dtype=torch.int32), dict(dtype=torch.float32)
+    return [sources.new_empty((1, kept)), sources.new_empty((1, total)),
+            sources.new_empty((1, n_src), dtype=torch.uint8), sources.new_empty((total,), **i32),
+            sources.new_empty((total,), **i32), sources.new_empty((kept + 1,), **i32),
+            sources.new_empty((kept,), **f32), sources.new_empty((kept,), **f32)]

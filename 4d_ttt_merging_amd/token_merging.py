@@ -544,17 +544,26 @@ def build_fastvggt_plan(
     best, target = torch.ops.vgo.fastvggt_match(tokens, sources, destinations, prenormalized)
     if after_match is not None:
         after_match()
-    keep, inverse, flags = torch.ops.vgo.fastvggt_assemble(best, target, sources, destinations, total, removed)
+    if mass_bias and batch != 1:
+        raise ValueError("mass-bias FastVGGT plans support batch size one")
+    one_launch = batch == 1 and _kernels._lib.load().vgo_fastvggt_plan_fits(sources.numel(), total, removed)
+    if one_launch:
+        keep, inverse, flags, inverse32, order, offsets, counts, log_mass = torch.ops.vgo.fastvggt_plan(
+            best, target, sources, destinations, total, removed)
+    else:
+        keep, inverse, flags = torch.ops.vgo.fastvggt_assemble(best, target, sources, destinations, total, removed)
     plan = TokenPlan(keep, inverse, total)
     # Match results stay on the device for diagnostics and tests.
     plan._derived["match"] = (sources, destinations, best, target, flags)
-    if mass_bias:
-        if batch != 1:
-            raise ValueError("mass-bias FastVGGT plans support batch size one")
+    if one_launch:
+        plan._derived[("inverse32", 0)] = inverse32
+    elif mass_bias:
         # One mass pass gives the cluster counts _cluster_csr caches and their logs.
         order, offsets = _kernels.csr_build(plan._inverse32(0), plan.kept_tokens)
         counts, log_mass = _kernels.segment_mass(offsets, 1, order, None, plan.kept_tokens, 0.0,
                                                  want_log=True)
+    if one_launch or mass_bias:
         plan._derived[("csr", 0)] = (_Csr(order, offsets), counts, None)
+    if mass_bias:
         plan.key_log_mass = log_mass.view(1, -1)
     return plan

@@ -310,6 +310,20 @@ int vgo_fastvggt_assemble_ws(const float* best, const int32_t* target, const int
                              size_t workspace_bytes, void* stream);
 
 /*
+ * A whole FastVGGT plan of one batch element in one launch: vgo_fastvggt_assemble's
+ * keep / inverse / removed_flag, inverse as int32, and what vgo_csr_build and
+ * vgo_segment_mass (no weights, start 0) make of it: order [total_tokens],
+ * offsets [kept + 1], mass and log_mass [kept], bit for bit.  For plans that
+ * vgo_fastvggt_plan_fits (1: up to 12,288 tokens); VGO_EUNSUPPORTED otherwise.  token_merging.py:1112-1121, 176-191.
+ */
+int vgo_fastvggt_plan_fits(int64_t n_sources, int64_t total_tokens, int64_t removed);
+int vgo_fastvggt_plan(const float* best, const int32_t* target, const int64_t* source_ids,
+                      const int64_t* dest_ids, int64_t n_sources, int64_t n_dest,
+                      int64_t total_tokens, int64_t removed, int64_t* keep, int64_t* inverse,
+                      int32_t* inverse32, uint8_t* removed_flag, uint32_t* order, int32_t* offsets,
+                      float* mass, float* log_mass, void* stream);
+
+/*
  * Sparse-convex plan assembly (vggt_omega/models/sparse_convex.py:2435-2455):
  * sources = candidates with fit >= threshold (ascending), keep = the rest,
  * original_to_compact, parent = original_to_compact[support], weight = alpha.

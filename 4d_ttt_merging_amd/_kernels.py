@@ -66,6 +66,11 @@ def csr_build(keys: torch.Tensor, n_buckets: int) -> tuple[torch.Tensor, torch.T
     return torch.ops.vgo.csr_build(keys, n_buckets)
 
 
+def corner_csr(parent: torch.Tensor, n_dest: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """csr_build of the (destination, corner) pairs: item p = i*S + c, key = parent*S + c of [M, S] parents."""
+    return torch.ops.vgo.corner_csr(parent, n_dest)
+
+
 def segment_mass(offsets: torch.Tensor, segs_per_row: int, order: torch.Tensor,
                  weights: torch.Tensor | None, rows: int, start: float,
                  want_log: bool = True) -> tuple[torch.Tensor, torch.Tensor | None]:
@@ -83,9 +88,12 @@ def restore_map(total: int, *, device: torch.device, keep: torch.Tensor | None =
     lib = _lib.load()
     # With `inverse` the kernel writes every row; otherwise rows outside keep and
     # source stay zero (zero weights, as the reference's `new_zeros` output).
-    alloc = torch.empty if inverse is not None else torch.zeros
-    index_out = alloc((total, 4), device=device, dtype=torch.int32)
-    weight_out = alloc((total, 4), device=device, dtype=torch.float32)
+    if inverse is not None:
+        index_out = torch.empty((total, 4), device=device, dtype=torch.int32)
+        weight_out = torch.empty((total, 4), device=device, dtype=torch.float32)
+    else:  # one fill for both
+        index_out, weight_out = torch.zeros((2, total, 4), device=device, dtype=torch.int32).unbind()
+        weight_out = weight_out.view(torch.float32)
     n_keep = 0 if keep is None else keep.numel()
     n_source = 0 if source is None else source.numel()
     status = lib.vgo_restore_map(

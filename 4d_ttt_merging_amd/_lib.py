@@ -120,6 +120,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ]),
     "vgo_csr_workspace": (_c_int, [_c_i64, _c_i64, ctypes.POINTER(_c_size)]),
     "vgo_csr_build": (_c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_size, _c_p, _c_p, _c_p]),
+    "vgo_corner_csr": (_c_int, [
+        _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_size, _c_p, _c_p, _c_p,
+    ]),
     "vgo_segment_mass": (_c_int, [
         _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_f32, _c_p, _c_p, _c_p,
     ]),

@@ -15,8 +15,9 @@
 // cluster in ascending token order, divided by their count
 // (token_merging.py:176-191).
 #include <algorithm>
+#include <type_traits>
 
-#include "vgo_common.h"
+#include "block_csr.h"
 
 namespace vgo {
 namespace {
@@ -145,6 +146,61 @@ __global__ __launch_bounds__(256) void bucket_offsets_kernel(const uint32_t* __r
   for (int64_t kk = prev + 1; kk <= k; ++kk) offsets[kk] = e;
   if (e == n - 1)
     for (int64_t kk = k + 1; kk <= n_buckets; ++kk) offsets[kk] = n;
+}
+
+// Bucket of item i of the caller's keys.
+struct RawKeys {
+  const uint32_t* keys;
+  uint32_t buckets;
+  __device__ __forceinline__ uint32_t operator()(int i) const { return sort_key(keys, i, buckets); }
+};
+// Bucket of item p = source * corners + corner of a weighted plan: parent[p] * corners + corner,
+// or past the last bucket without a (valid) parent.
+struct CornerKeys {
+  const int64_t* parent;
+  int corners;
+  int64_t dests;
+  __device__ __forceinline__ uint32_t operator()(int i) const {
+    const int64_t k = parent[i];
+    return static_cast<uint32_t>(k < 0 || k >= dests ? dests * corners : k * corners + i % corners);
+  }
+};
+
+__global__ __launch_bounds__(256) void corner_keys_kernel(CornerKeys key, int n, uint32_t* __restrict__ keys) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) keys[i] = key(i);
+}
+
+// The whole CSR in one launch of one work-group for few items and buckets, where
+// each of the sort's four to thirteen launches is all latency.
+// Measured (us, one launch / the launches): 1,000 items in 1,000 buckets 4.3 / 31,
+// 4,096 in 16,000 12 / 31, 9,604 in 25,028 17 / 31, 12,288 in 40,960 22 / 31 -- the
+// largest that LDS holds is also where the two are about to meet.
+constexpr int kSmallChunks = 12;
+constexpr int kSmallItems = kSmallChunks * kBlockThreads;
+constexpr int kSmallBuckets = 40960;  // 80 KB of 16-bit counters
+template <int C, typename Keys>
+__global__ __launch_bounds__(kBlockThreads) void csr_small_kernel(Keys key, int n, int n_buckets,
+                                                                  uint32_t* __restrict__ order,
+                                                                  int32_t* __restrict__ offsets) {
+  __shared__ uint32_t cnt32[kSmallBuckets / 2 + 2];
+  __shared__ uint16_t slot[kSmallItems];
+  __shared__ BlockCsrLds<kSmallChunks> lds;
+  const int tid = threadIdx.x;
+  uint32_t place[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int i = c * kBlockThreads + tid;
+    place[c] = i < n ? key(i) : 0u;
+  }
+  for (int i = tid; i < (n_buckets + 3) / 2; i += kBlockThreads) cnt32[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    if (c * kBlockThreads + tid < n) place[c] = take_place(cnt32, static_cast<int>(place[c]));
+  }
+  __syncthreads();
+  block_csr<C>(place, n, n_buckets, slot, reinterpret_cast<uint16_t*>(cnt32), lds, order, offsets, [](int, int) {});
 }
 
 __global__ __launch_bounds__(256) void fill_i32_kernel(int32_t* __restrict__ p, int n, int32_t v) {
@@ -628,38 +684,42 @@ extern "C" int vgo_csr_workspace(int64_t n_items, int64_t n_buckets, size_t* byt
   return VGO_OK;
 }
 
-extern "C" int vgo_csr_build(const uint32_t* keys, int64_t n_items, int64_t n_buckets,
-                             void* workspace, size_t workspace_bytes, uint32_t* order,
-                             int32_t* offsets, void* stream) {
-  size_t need = 0;
-  int st = vgo_csr_workspace(n_items, n_buckets, &need);
-  if (st != VGO_OK) return st;
-  VGO_REQUIRE(offsets, "csr_build: null offsets");
-  hipStream_t s = as_stream(stream);
-  const int n = static_cast<int>(n_items);
-  const int nb = static_cast<int>(n_buckets);
-  if (n == 0) {
-    hipLaunchKernelGGL(fill_i32_kernel, dim3((nb + 1 + 255) / 256), dim3(256), 0, s, offsets, nb + 1, 0);
+namespace vgo {
+namespace {
+
+// vgo_csr_build of the keys that `key` makes; `given`: those keys in memory, or null.
+template <typename Keys>
+int csr(Keys key, const uint32_t* given, int n, int nb, void* workspace, uint32_t* order, int32_t* offsets,
+        hipStream_t s) {
+  if (n <= kSmallItems && nb <= kSmallBuckets) {
+    if (n <= 4 * kBlockThreads) {
+      hipLaunchKernelGGL((csr_small_kernel<4, Keys>), dim3(1), dim3(kBlockThreads), 0, s, key, n, nb, order, offsets);
+    } else {
+      hipLaunchKernelGGL((csr_small_kernel<kSmallChunks, Keys>), dim3(1), dim3(kBlockThreads), 0, s, key, n, nb,
+                         order, offsets);
+    }
     return check_launch("csr_build");
   }
-  VGO_REQUIRE(keys && order && workspace, "csr_build: null pointer");
-  VGO_REQUIRE(workspace_bytes >= need && aligned(workspace, 256), "csr_build: workspace too small or misaligned");
   char* ws = static_cast<char*>(workspace);
   uint32_t* ka = reinterpret_cast<uint32_t*>(ws);
   uint32_t* kb = reinterpret_cast<uint32_t*>(ws + align_up(size_t(n) * 4));
   uint32_t* va = reinterpret_cast<uint32_t*>(ws + 2 * align_up(size_t(n) * 4));
   uint32_t* hist = reinterpret_cast<uint32_t*>(ws + 3 * align_up(size_t(n) * 4));
   const int nblocks = (n + kBlockItems - 1) / kBlockItems;
-  const int passes = (key_bits(n_buckets) + 7) / 8;
+  const int passes = (key_bits(nb) + 7) / 8;
   // Value buffers ping-pong between va and `order` so the last pass lands in `order`.
   uint32_t* vbuf[2] = {va, order};
   uint32_t* kbuf[2] = {ka, kb};
   int cur = passes % 2 == 0 ? 1 : 0;  // pass p writes buffer (cur + p + 1) % 2
+  if constexpr (std::is_same_v<Keys, CornerKeys>) {  // pass 0 reads buffer cur, which pass 1 is the first to write
+    hipLaunchKernelGGL(corner_keys_kernel, dim3((n + 255) / 256), dim3(256), 0, s, key, n, kbuf[cur]);
+    given = kbuf[cur];
+  }
   // Pass 0 reads the caller's keys (clamped as it reads them) and the item
   // indices; after `passes` flips the values end in vbuf[(cur + passes) % 2] == order.
   for (int p = 0; p < passes; ++p) {
     const int shift = 8 * p;
-    const uint32_t* kin = p == 0 ? keys : kbuf[cur];
+    const uint32_t* kin = p == 0 ? given : kbuf[cur];
     const uint32_t* vin = p == 0 ? nullptr : vbuf[cur];
     const uint32_t limit = p == 0 ? static_cast<uint32_t>(nb) : 0u;
     hipLaunchKernelGGL(radix_hist_kernel, dim3(nblocks), dim3(kSortThreads), 0, s, kin, n, shift, hist,
@@ -672,6 +732,53 @@ extern "C" int vgo_csr_build(const uint32_t* keys, int64_t n_items, int64_t n_bu
   hipLaunchKernelGGL(bucket_offsets_kernel, dim3((n + 255) / 256), dim3(256), 0, s, kbuf[cur], n,
                      nb, offsets);
   return check_launch("csr_build");
+}
+
+// The checks of vgo_csr_build; *done: no items, the offsets are written.
+int csr_check(const void* keys, int64_t n_items, int64_t n_buckets, void* workspace, size_t workspace_bytes,
+              uint32_t* order, int32_t* offsets, hipStream_t s, bool* done) {
+  *done = false;
+  size_t need = 0;
+  const int st = vgo_csr_workspace(n_items, n_buckets, &need);
+  if (st != VGO_OK) return st;
+  VGO_REQUIRE(offsets, "csr_build: null offsets");
+  if (n_items == 0) {
+    const int nb = static_cast<int>(n_buckets);
+    hipLaunchKernelGGL(fill_i32_kernel, dim3((nb + 1 + 255) / 256), dim3(256), 0, s, offsets, nb + 1, 0);
+    *done = true;
+    return check_launch("csr_build");
+  }
+  VGO_REQUIRE(keys && order && workspace, "csr_build: null pointer");
+  VGO_REQUIRE(workspace_bytes >= need && aligned(workspace, 256), "csr_build: workspace too small or misaligned");
+  return VGO_OK;
+}
+
+}  // namespace
+}  // namespace vgo
+
+extern "C" int vgo_csr_build(const uint32_t* keys, int64_t n_items, int64_t n_buckets,
+                             void* workspace, size_t workspace_bytes, uint32_t* order,
+                             int32_t* offsets, void* stream) {
+  bool done = false;
+  const int st = csr_check(keys, n_items, n_buckets, workspace, workspace_bytes, order, offsets, as_stream(stream),
+                           &done);
+  if (st != VGO_OK || done) return st;
+  return csr(RawKeys{keys, static_cast<uint32_t>(n_buckets)}, keys, static_cast<int>(n_items),
+             static_cast<int>(n_buckets), workspace, order, offsets, as_stream(stream));
+}
+
+extern "C" int vgo_corner_csr(const int64_t* parent, int64_t n_items, int64_t corners, int64_t n_dest,
+                              void* workspace, size_t workspace_bytes, uint32_t* order, int32_t* offsets,
+                              void* stream) {
+  VGO_REQUIRE(corners >= 1 && corners < (1LL << 31) && n_dest >= 1 && n_dest < (1LL << 31) / corners &&
+                  n_items % corners == 0,
+              "corner_csr: bad size");
+  bool done = false;
+  const int st = csr_check(parent, n_items, n_dest * corners, workspace, workspace_bytes, order, offsets,
+                           as_stream(stream), &done);
+  if (st != VGO_OK || done) return st;
+  return csr(CornerKeys{parent, static_cast<int>(corners), n_dest}, nullptr, static_cast<int>(n_items),
+             static_cast<int>(n_dest * corners), workspace, order, offsets, as_stream(stream));
 }
 
 extern "C" int vgo_segment_mass(const int32_t* offsets, int64_t segs_per_row, const uint32_t* items,

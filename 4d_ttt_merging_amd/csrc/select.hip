@@ -12,13 +12,13 @@
 // threshold by source position (the stable sort's rule) and builds keep /
 // inverse, both with ballot-based ordered ranks (one block scan per 64 chunks
 // of 1024 elements).  Integer work, bit-exact, deterministic.
-#include "vgo_common.h"
+#include "block_csr.h"
 
 namespace vgo {
 namespace {
 
-constexpr int kThreads = 1024;
-constexpr int kWavesS = kThreads / 64;
+constexpr int kThreads = kBlockThreads;
+constexpr int kWavesS = kBlockWaves;
 
 // Order-preserving map float -> uint32 (NaN above +inf, -0 folded onto +0),
 // matching the comparison order of torch's descending stable sort.
@@ -27,71 +27,6 @@ __device__ __forceinline__ uint32_t ord32(float x) {
   uint32_t b = __float_as_uint(x);
   if (b == 0x80000000u) b = 0;
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-
-// Exclusive prefix sum over the work-group (kThreads threads); returns the
-// thread's exclusive prefix and writes the total to *total.
-__device__ int block_exclusive_scan(int v, int* lds_waves, int* total) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  int x = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int y = __shfl_up(x, off);
-    if (lane >= off) x += y;
-  }
-  if (lane == 63) lds_waves[wave] = x;
-  __syncthreads();
-  if (wave == 0) {
-    int w = lane < kWavesS ? lds_waves[lane] : 0;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int y = __shfl_up(w, off);
-      if (lane >= off) w += y;
-    }
-    if (lane < kWavesS) lds_waves[lane] = w;  // inclusive scan of wave totals
-  }
-  __syncthreads();
-  const int wave_base = wave > 0 ? lds_waves[wave - 1] : 0;
-  const int t = lds_waves[kWavesS - 1];
-  __syncthreads();
-  *total = t;
-  return wave_base + x - v;
-}
-
-// Ranks, in index order, of the elements whose flag is set: element i = c*kThreads
-// + tid of chunk c.  Chunks are processed 64 at a time: per (chunk, wave) counts
-// from ballots go to LDS, one block scan over those 1024 counts gives every
-// (chunk, wave) its offset, and a lane adds the set flags of lower lanes.
-// `flag(c)` is evaluated twice per chunk; `emit(c, rank)` is called for every
-// set flag.  Returns the number of set flags.
-template <typename Flag, typename Emit>
-__device__ int ordered_ranks(int n_chunks, Flag flag, Emit emit, int* cnt_lds, int* scan_lds) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  int running = 0;
-  for (int c0 = 0; c0 < n_chunks; c0 += 64) {
-    const int nc = min(64, n_chunks - c0);
-    for (int c = 0; c < 64; ++c) {
-      const uint64_t m = c < nc ? __ballot(flag(c0 + c)) : 0ull;
-      if (lane == 0) cnt_lds[c * kWavesS + wave] = __popcll(m);
-    }
-    __syncthreads();
-    const int mine = cnt_lds[threadIdx.x];  // kThreads == 64 * kWavesS entries
-    int sum = 0;
-    const int pre = block_exclusive_scan(mine, scan_lds, &sum);
-    cnt_lds[threadIdx.x] = pre;
-    __syncthreads();
-    const uint64_t below = (1ull << lane) - 1ull;
-    for (int c = 0; c < nc; ++c) {
-      const bool f = flag(c0 + c);
-      const uint64_t m = __ballot(f);
-      if (f) emit(c0 + c, running + cnt_lds[c * kWavesS + wave] + __popcll(m & below));
-    }
-    running += sum;
-    __syncthreads();
-  }
-  return running;
 }
 
 // hist[digit] += 1 for every lane with `valid`.  Keys here cluster in a few
@@ -325,74 +260,85 @@ __global__ __launch_bounds__(kThreads) void fastvggt_assemble_kernel(
 // Buffers are sized for the worst case (n sources, total kept); stats[0] = M
 // (sources), stats[1] = hard candidates, stats[2] = fallback candidates (copied
 // from the device counter), stats[3] = sum of the selected fits.
-__global__ __launch_bounds__(kThreads) void sparse_convex_assemble_kernel(
-    const float* __restrict__ fit, const float* __restrict__ alpha,
-    const int64_t* __restrict__ support, const int64_t* __restrict__ candidate,
-    const float* __restrict__ top1, float easy_threshold, const int* __restrict__ failed_count,
-    int n, int total, float threshold, int64_t* __restrict__ keep, int64_t* __restrict__ o2c,
-    int64_t* __restrict__ source, int64_t* __restrict__ parent, float* __restrict__ weight,
-    float* __restrict__ stats) {
+//
+// Two launches.  The first, one work-group, does what needs ranks over all
+// candidates and tokens: o2c, the statistics, and the candidate of every source
+// (left in the first word of its `parent` row).  Its time is the latency of its
+// loads: they are coalesced and eight chunks of 1,024 are in flight.  The second
+// writes the rest from the whole chip (56 bytes per source, 8 per kept token, which
+// one work-group would store at a few tens of GB/s).  5,672 candidates of 8,658 tokens:
+// 51 us from one work-group whose threads took contiguous runs, now 13.5 + 5.
+__global__ __launch_bounds__(kThreads) void sparse_convex_select_kernel(
+    const float* __restrict__ fit, const int64_t* __restrict__ candidate, const float* __restrict__ top1,
+    float easy_threshold, const int* __restrict__ failed_count, int n, int total, float threshold, int64_t* o2c,
+    int64_t* __restrict__ parent, float* __restrict__ stats) {
   __shared__ int scan_lds[kWavesS];
+  __shared__ int cnt_lds[kThreads];
   __shared__ float red[kWavesS];
   const int tid = threadIdx.x;
-  const int es = (n + kThreads - 1) / kThreads;
-  const int s_begin = min(n, tid * es), s_end = min(n, s_begin + es);
-  const int et = (total + kThreads - 1) / kThreads;
-  const int t_begin = min(total, tid * et), t_end = min(total, t_begin + et);
+  for (int t = tid; t < total; t += kThreads) o2c[t] = 0;
+  __syncthreads();
 
-  int mine = 0, hard = 0;
+  // ---- candidates, 64 chunks at a time
+  int hard = 0, n_sel = 0;
   float fsum = 0.0f;
-  for (int r = s_begin; r < s_end; ++r) {
-    const bool sel = fit[r] >= threshold;
-    mine += sel;
-    if (sel) fsum += fit[r];
-    hard += !(top1 && top1[r] >= easy_threshold);
+  for (int g0 = 0; g0 < n; g0 += 64 * kThreads) {
+    const int chunks = min(64, (n - g0 + kThreads - 1) / kThreads);
+    const uint64_t selected = chunk_bits(chunks, [&](int c0) {
+      float f[8], e[8];
+      int64_t id[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int r = g0 + (c0 + q) * kThreads + tid;
+        f[q] = r < n ? fit[r] : 0.0f;
+        e[q] = r < n && top1 ? top1[r] : 0.0f;
+        id[q] = r < n ? candidate[r] : -1;
+      }
+      uint32_t bits = 0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int r = g0 + (c0 + q) * kThreads + tid;
+        if (r >= n) continue;
+        hard += !(top1 && e[q] >= easy_threshold);
+        if (!(f[q] >= threshold)) continue;
+        bits |= 1u << q;
+        fsum += f[q];
+        if (id[q] >= 0 && id[q] < total) o2c[id[q]] = -1;
+      }
+      return bits;
+    });
+    const int before = n_sel;
+    n_sel += ordered_ranks(
+        chunks, [&](int c) { return ((selected >> c) & 1ull) != 0ull; },
+        [&](int c, int rank) { parent[4 * static_cast<int64_t>(before + rank)] = g0 + c * kThreads + tid; }, cnt_lds,
+        scan_lds);
   }
-  int n_sel = 0;
-  int pos = block_exclusive_scan(mine, scan_lds, &n_sel);
   int n_hard = 0;
   block_exclusive_scan(hard, scan_lds, &n_hard);
-  for (int t = t_begin; t < t_end; ++t) o2c[t] = 0;
-  __syncthreads();
-  for (int r = s_begin; r < s_end; ++r) {
-    if (fit[r] >= threshold) {
-      const int64_t c = candidate[r];
-      source[pos] = c;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) weight[4 * pos + k] = alpha[4 * r + k];
-      if (c >= 0 && c < total) o2c[c] = -1;
-      ++pos;
-    }
-  }
-  __syncthreads();
+
+  // ---- tokens
   int kept = 0;
-  for (int t = t_begin; t < t_end; ++t) kept += o2c[t] == 0;
-  int kept_total = 0;
-  int base = block_exclusive_scan(kept, scan_lds, &kept_total);
-  for (int t = t_begin; t < t_end; ++t) {
-    if (o2c[t] == 0) {
-      o2c[t] = base;
-      keep[base] = t;
-      ++base;
-    }
-  }
   __syncthreads();
-  // Second walk over the selected rows in the same order to fill parent ids.
-  int pos2 = 0;
-  {
-    int dummy = 0;
-    pos2 = block_exclusive_scan(mine, scan_lds, &dummy);
-  }
-  for (int r = s_begin; r < s_end; ++r) {
-    if (fit[r] >= threshold) {
+  for (int g0 = 0; g0 < total; g0 += 64 * kThreads) {
+    const int chunks = min(64, (total - g0 + kThreads - 1) / kThreads);
+    const uint64_t stays = chunk_bits(chunks, [&](int c0) {
+      int64_t v[8];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int64_t sup = support[4 * r + k];
-        parent[4 * pos2 + k] = (sup >= 0 && sup < total) ? o2c[sup] : -1;
+      for (int q = 0; q < 8; ++q) {
+        const int t = g0 + (c0 + q) * kThreads + tid;
+        v[q] = t < total ? o2c[t] : -1;
       }
-      ++pos2;
-    }
+      uint32_t bits = 0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) bits |= static_cast<uint32_t>(v[q] == 0) << q;
+      return bits;
+    });
+    const int before = kept;
+    kept += ordered_ranks(
+        chunks, [&](int c) { return ((stays >> c) & 1ull) != 0ull; },
+        [&](int c, int rank) { o2c[g0 + c * kThreads + tid] = before + rank; }, cnt_lds, scan_lds);
   }
+
   // Deterministic fit sum (fixed thread/wave order).
   float v = fsum;
 #pragma unroll
@@ -407,6 +353,25 @@ __global__ __launch_bounds__(kThreads) void sparse_convex_assemble_kernel(
     stats[2] = failed_count ? static_cast<float>(*failed_count) : 0.0f;
     stats[3] = s;
   }
+}
+
+__global__ __launch_bounds__(256) void sparse_convex_fill_kernel(
+    const float* __restrict__ alpha, const int64_t* __restrict__ support, const int64_t* __restrict__ candidate,
+    const int64_t* __restrict__ o2c, const float* __restrict__ stats, int n, int total, int64_t* __restrict__ keep,
+    int64_t* __restrict__ source, int64_t* parent, float* __restrict__ weight) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < total) {
+    const int64_t k = o2c[i];
+    if (k >= 0) keep[k] = i;
+  }
+  // Four lanes per source; all four have its candidate before any stores its parent.
+  const bool live = i < 4 * static_cast<int64_t>(min(n, static_cast<int>(stats[0])));
+  const int r = __shfl(live && (i & 3) == 0 ? static_cast<int>(parent[i]) : -1, threadIdx.x & 60);
+  if (!live || r < 0 || r >= n) return;
+  const int64_t sup = support[4 * static_cast<int64_t>(r) + (i & 3)];
+  weight[i] = alpha[4 * static_cast<int64_t>(r) + (i & 3)];
+  parent[i] = sup >= 0 && sup < total ? o2c[sup] : -1;
+  if ((i & 3) == 0) source[i >> 2] = candidate[r];
 }
 
 // ---------------------------------------------------------------------------
@@ -725,14 +690,9 @@ __global__ __launch_bounds__(kAThreads) void fva_inverse_kernel(const int32_t* _
 //    is one ballot per 64 keys (held in registers), where a digit histogram
 //    serialises on the few digits that bf16-rounded scores occupy.
 //  * val[t] (u16): a kept token's compact id, a removed one's destination.
-//  * Cluster order: a token's slot within its cluster comes from an LDS counter
-//    in any order; its rank among the cluster's tokens is then counted, except
-//    for clusters over kBigCluster tokens, whose tokens a wave collects in
-//    order from one pass over all of them (identical frames put thousands of
-//    tokens on one destination).
+//  * Cluster order: block_csr.
 // Results equal the launches' bit for bit.
 constexpr int kPlanChunks = 12;                      // tokens <= 12 x 1024
-constexpr int kBigCluster = 128;
 
 struct PlanLds {
   int val_at, cnt_at, bits_at, bytes;  // byte offsets of val u16[total], cnt u16[kept + 2], removed bits
@@ -762,9 +722,8 @@ __global__ __launch_bounds__(kThreads) void fastvggt_plan_kernel(
   __shared__ __attribute__((aligned(16))) uint32_t state[kPlanLds / 4];
   __shared__ int counts[2][kWavesS];
   __shared__ int chunk_cnt[kPlanChunks * kWavesS];
-  __shared__ int scan_lds[kWavesS];
-  __shared__ int big[kPlanChunks * kThreads / kBigCluster];
-  __shared__ int n_big;
+  __shared__ BlockCsrLds<kPlanChunks> csr_lds;
+  int* scan_lds = csr_lds.scan;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint64_t below = (1ull << lane) - 1ull;
@@ -778,7 +737,6 @@ __global__ __launch_bounds__(kThreads) void fastvggt_plan_kernel(
   const int t_chunks = (total + kThreads - 1) / kThreads;
 
   for (int i = tid; i < (at.bytes - at.cnt_at) / 4; i += kThreads) cnt32[i] = 0;  // counters and bits
-  if (tid == 0) n_big = 0;
 
   // ---- keys; the removed-th largest of them.
   uint32_t key[C];  // 0 past the sources: below every key
@@ -888,7 +846,7 @@ __global__ __launch_bounds__(kThreads) void fastvggt_plan_kernel(
   __syncthreads();
 
   // ---- inverse, and every token's cluster and slot in it (a token without one: cluster `kept`).
-  uint32_t place[C];  // cluster | slot << 16
+  uint32_t place[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     const int t = c * kThreads + tid;
@@ -899,73 +857,17 @@ __global__ __launch_bounds__(kThreads) void fastvggt_plan_kernel(
       if (k >= kept) k = -1;
       inverse[t] = k;
       inverse32[t] = k;
-      const int cluster = k < 0 ? kept : k;
-      const int shift = 16 * (cluster & 1);
-      const uint32_t old = atomicAdd(&cnt32[cluster >> 1], 1u << shift);
-      place[c] = static_cast<uint32_t>(cluster) | (((old >> shift) & 0xFFFFu) << 16);
+      place[c] = take_place(cnt32, k < 0 ? kept : k);
     }
   }
   __syncthreads();
-
-  // ---- cluster sizes -> offsets (in place), masses.
-  const int per = (kept + 1 + kThreads - 1) / kThreads;
-  const int k0 = min(kept + 1, tid * per), k1 = min(kept + 1, k0 + per);
-  int sum = 0;
-  for (int k = k0; k < k1; ++k) {
-    const int n = cnt[k];
-    sum += n;
-    if (n > kBigCluster) big[atomicAdd(&n_big, 1)] = k;
-  }
-  int all = 0;
-  int run = block_exclusive_scan(sum, scan_lds, &all);
-  for (int k = k0; k < k1; ++k) {
-    const int n = cnt[k];
-    cnt[k] = static_cast<uint16_t>(run);
-    run += n;
-  }
-  if (tid == 0) cnt[kept + 1] = static_cast<uint16_t>(total);
-  __syncthreads();
-  for (int k = tid; k <= kept; k += kThreads) {
-    offsets[k] = cnt[k];
-    if (k < kept) {
-      const float m = static_cast<float>(cnt[k + 1] - cnt[k]);
-      mass[k] = m;
-      log_mass[k] = logf(m);
-    }
-  }
-
-  // ---- cluster members in token order (val's space holds the members now).
-  uint16_t* slot = val;
-#pragma unroll
-  for (int c = 0; c < C; ++c) {
-    const int t = c * kThreads + tid;
-    if (c < t_chunks && t < total) slot[cnt[place[c] & 0xFFFFu] + (place[c] >> 16)] = static_cast<uint16_t>(t);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int c = 0; c < C; ++c) {
-    const int t = c * kThreads + tid;
-    if (c < t_chunks && t < total) {
-      const int cluster = place[c] & 0xFFFFu;
-      const int b = cnt[cluster], e = cnt[cluster + 1];
-      if (e - b <= kBigCluster) {
-        int rank = 0;
-        for (int j = b; j < e; ++j) rank += slot[j] < t;
-        order[b + rank] = static_cast<uint32_t>(t);
-      }
-    }
-  }
-  for (int g = wave; g < n_big; g += kWavesS) {
-    const int cluster = big[g];
-    int pos = cnt[cluster];
-    for (int t0 = 0; t0 < total; t0 += 64) {
-      const int t = t0 + lane;
-      const bool mine = t < total && (cluster == kept ? inverse32[t] < 0 : inverse32[t] == cluster);
-      const uint64_t m = __ballot(mine);
-      if (mine) order[pos + __popcll(m & below)] = static_cast<uint32_t>(t);
-      pos += __popcll(m);
-    }
-  }
+  // val's space holds the members from here on.
+  block_csr<C>(
+      place, total, kept, val, cnt, csr_lds, order, offsets, [&](int k, int size) {
+        const float m = static_cast<float>(size);
+        mass[k] = m;
+        log_mass[k] = logf(m);
+      });
 }
 
 }  // namespace
@@ -1037,10 +939,15 @@ extern "C" int vgo_sparse_convex_assemble(const float* fit, const float* alpha, 
   VGO_REQUIRE(keep && original_to_compact && stats, "sparse_convex_assemble: null pointer");
   VGO_REQUIRE(n_candidates == 0 || (fit && alpha && support && candidate && source && parent && weight),
               "sparse_convex_assemble: null pointer");
-  hipLaunchKernelGGL(sparse_convex_assemble_kernel, dim3(1), dim3(kThreads), 0, as_stream(stream), fit,
-                     alpha, support, candidate, top1, easy_threshold, failed_count,
-                     static_cast<int>(n_candidates), static_cast<int>(total_tokens), threshold, keep,
-                     original_to_compact, source, parent, weight, stats);
+  const int n = static_cast<int>(n_candidates), total = static_cast<int>(total_tokens);
+  hipLaunchKernelGGL(sparse_convex_select_kernel, dim3(1), dim3(kThreads), 0, as_stream(stream), fit, candidate, top1,
+                     easy_threshold, failed_count, n, total, threshold, original_to_compact, parent, stats);
+  const int64_t items = 4 * n_candidates > total_tokens ? 4 * n_candidates : total_tokens;
+  if (items > 0) {
+    hipLaunchKernelGGL(sparse_convex_fill_kernel, dim3(static_cast<unsigned>((items + 255) / 256)), dim3(256), 0,
+                       as_stream(stream), alpha, support, candidate, original_to_compact, stats, n, total, keep,
+                       source, parent, weight);
+  }
   return check_launch("sparse_convex_assemble");
 }
 

@@ -470,6 +470,22 @@ std::tuple<Tensor, Tensor> csr_build(const Tensor& keys0, int64_t n_buckets) {
   return {order, offsets};
 }
 
+std::tuple<Tensor, Tensor> corner_csr(const Tensor& parent0, int64_t n_dest) {
+  require_gpu({&parent0});
+  const int64_t corners = parent0.size(-1), n = parent0.numel();
+  const Tensor parent = parent0.to(at::kLong).contiguous();
+  const auto options = parent.options().dtype(at::kInt);
+  size_t need = 0;
+  check(vgo_csr_workspace(n, n_dest * corners, &need));
+  const Tensor ws = at::empty({static_cast<int64_t>(need) + 256}, options.dtype(at::kByte));
+  char* base = ptr<char>(ws);
+  base += (256 - reinterpret_cast<uintptr_t>(base) % 256) % 256;
+  Tensor order = at::empty({n}, options), offsets = at::empty({n_dest * corners + 1}, options);
+  check(vgo_corner_csr(ptr<int64_t>(parent), n, corners, n_dest, base, need, ptr<uint32_t>(order),
+                       ptr<int32_t>(offsets), stream_of(parent)));
+  return {order, offsets};
+}
+
 std::tuple<Tensor, Tensor> segment_mass(const Tensor& offsets, int64_t segs_per_row, const Tensor& order,
                                         const OptTensor& weights0, int64_t rows, double start, bool want_log) {
   require_gpu({&offsets, &order, opt(weights0)});
@@ -632,7 +648,7 @@ void no_batching(const c10::OperatorHandle& op, c10::DispatchKeySet, torch::jit:
 
 constexpr const char* kPure[] = {"mass_bias_attention", "top4_project", "qkv_epilogue", "residual_layer_norm",
                                  "restore_residual_layer_norm", "mlp_tail", "dense_block", "normalize_rows",
-                                 "csr_build", "segment_mass", "fastvggt_assemble", "fastvggt_match", "fastvggt_plan",
+                                 "csr_build", "corner_csr", "segment_mass", "fastvggt_assemble", "fastvggt_match", "fastvggt_plan",
                                  "merged_block"};
 constexpr const char* kMutating[] = {"attention_into", "attention_pair_into", "top4_project_into",
                                      "top4_project_ordered_into", "compact_into", "compact_multi_into", "similarity_topk"};
@@ -655,6 +671,7 @@ TORCH_LIBRARY_IMPL(vgo, CUDA, m) {
   m.impl("dense_block", dense_block);
   m.impl("normalize_rows", normalize_rows);
   m.impl("csr_build", csr_build);
+  m.impl("corner_csr", corner_csr);
   m.impl("segment_mass", segment_mass);
   m.impl("fastvggt_assemble", fastvggt_assemble);
   m.impl("fastvggt_match", fastvggt_match);

@@ -24,7 +24,8 @@ dispatcher, `torch.compile` and fake-tensor tracing see them as single ops:
   last residual pass, a whole unmerged block (layers/block.py:89-129) and a whole
   merged block over a token plan (:219-226), for eager inference; and the plan
   builders' kernels (`vgo::normalize_rows`, `similarity_topk`, `fastvggt_match`,
-  `fastvggt_assemble`, `fastvggt_plan`, `csr_build`, `segment_mass`).
+  `fastvggt_assemble`, `fastvggt_plan`, `csr_build`, `corner_csr`,
+  `segment_mass`).
 
 The CUDA (HIP) implementations are native (csrc/torch_ops.cpp, built into
 `libvgo_torch.so`) and call `libvgo.so` through its C ABI.  The operators a
@@ -89,6 +90,7 @@ _SCHEMAS = (
     "fastvggt_match(Tensor tokens, Tensor sources, Tensor destinations, bool prenormalized) -> (Tensor, Tensor)",
     "normalize_rows(Tensor x, Tensor? rows, float eps, ScalarType out_dtype) -> Tensor",
     "csr_build(Tensor keys, int n_buckets) -> (Tensor, Tensor)",
+    "corner_csr(Tensor parent, int n_dest) -> (Tensor, Tensor)",
     "segment_mass(Tensor offsets, int segs_per_row, Tensor order, Tensor? weights, int rows, float start, "
     "bool want_log) -> (Tensor, Tensor)",
     "fastvggt_assemble(Tensor best, Tensor target, Tensor sources, Tensor destinations, int total, "
@@ -203,6 +205,12 @@ def _(best, target, sources, destinations, total, removed):
 def _(keys, n_buckets):
     return (keys.new_empty((keys.numel(),), dtype=torch.int32),
             keys.new_empty((n_buckets + 1,), dtype=torch.int32))
+
+
+@_fake("corner_csr")
+def _(parent, n_dest):
+    return (parent.new_empty((parent.numel(),), dtype=torch.int32),
+            parent.new_empty((n_dest * parent.shape[-1] + 1,), dtype=torch.int32))
 
 
 @_fake("segment_mass")

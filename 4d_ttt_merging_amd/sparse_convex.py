@@ -189,20 +189,24 @@ def start_sparse_convex_plan(
     n_cand = candidate.numel()
     easy_threshold = threshold + _EARLY_MARGIN
 
-    support = torch.empty((n_cand, 4), device=device, dtype=torch.int64)
     top1 = torch.empty(n_cand, device=device, dtype=torch.float32)
     fit = torch.empty(n_cand, device=device, dtype=torch.float32)
     alpha = torch.empty((n_cand, 4), device=device, dtype=torch.float32)
     failed_list = torch.empty(max(n_cand, 1), device=device, dtype=torch.int32)
-    failed_count = torch.zeros(1, device=device, dtype=torch.int32)
+    failed_count = (torch.empty if n_cand else torch.zeros)(1, device=device, dtype=torch.int32)
     if n_cand:
         cand_bf16 = _kernels.normalize_rows(x, candidate, _NORMALIZE_EPS)
         dest_bf16 = _kernels.normalize_rows(x, destination, _NORMALIZE_EPS)
-        for c0, c1, off1, n_anchor in lay["groups"]:
+        groups = lay["groups"]
+        support = None if len(groups) == 1 else torch.empty((n_cand, 4), device=device, dtype=torch.int64)
+        for c0, c1, off1, n_anchor in groups:
             values, index = _kernels.similarity_topk(
                 cand_bf16[c0:c1], dest_bf16, 4,
                 dict_ranges=(lay["frame0"], off1, lay["frame0"] + n_anchor), index_map=destination)
-            support[c0:c1] = index
+            if support is None:
+                support = index
+            else:
+                support[c0:c1] = index
             top1[c0:c1] = values[:, 0]
         convex_fit(x, candidate, support, top1=top1, easy_threshold=easy_threshold, fit=fit,
                    alpha=alpha)
@@ -216,12 +220,15 @@ def start_sparse_convex_plan(
         convex_fit(x, candidate, support, row_list=failed_list, n_list=failed_count,
                    list_supports=fb_index, fit=fit, alpha=alpha)
 
+    else:
+        support = torch.empty((0, 4), device=device, dtype=torch.int64)
+
     keep_buf = torch.empty(total, device=device, dtype=torch.int64)
     o2c = torch.empty(total, device=device, dtype=torch.int64)
     source_buf = torch.empty(max(n_cand, 1), device=device, dtype=torch.int64)
     parent_buf = torch.empty((max(n_cand, 1), 4), device=device, dtype=torch.int64)
     weight_buf = torch.empty((max(n_cand, 1), 4), device=device, dtype=torch.float32)
-    stats = torch.zeros(4, device=device, dtype=torch.float32)
+    stats = torch.empty(4, device=device, dtype=torch.float32)
     _lib.check(lib.vgo_sparse_convex_assemble(
         fit.data_ptr(), alpha.data_ptr(), support.data_ptr(), candidate.data_ptr(),
         top1.data_ptr(), float(easy_threshold), failed_count.data_ptr(), n_cand, total,
@@ -230,17 +237,18 @@ def start_sparse_convex_plan(
     stats_host = torch.empty(4, dtype=torch.float32, pin_memory=True)
     stats_host.copy_(stats, non_blocking=True)
     copied = torch.cuda.Event()
+    special_compact = o2c.index_select(0, lay["special"])  # covered by the event: any stream may take the plan
     copied.record(torch.cuda.current_stream(device))
 
     def finish(counts: torch.Tensor) -> WeightedBilinearTokenPlan:
-        return _finish_plan(counts, lay, total, keep_buf, o2c, source_buf, parent_buf, weight_buf,
+        return _finish_plan(counts, lay, total, keep_buf, special_compact, source_buf, parent_buf, weight_buf,
                             threshold, preserve_queries, preserve_destination_keys,
                             (fit, alpha, support, top1, failed_list, failed_count))
 
     return PendingSparseConvexPlan(finish, stats_host, copied)
 
 
-def _finish_plan(counts, lay, total, keep_buf, o2c, source_buf, parent_buf, weight_buf, threshold,
+def _finish_plan(counts, lay, total, keep_buf, special_compact, source_buf, parent_buf, weight_buf, threshold,
                  preserve_queries, preserve_destination_keys, fit_state) -> WeightedBilinearTokenPlan:
     """The plan over the assemble kernel's buffers, sized by its counts (host copy)."""
     merged, hard, fallback, fit_sum = (float(v) for v in counts)
@@ -250,7 +258,6 @@ def _finish_plan(counts, lay, total, keep_buf, o2c, source_buf, parent_buf, weig
     parent_compact = parent_buf[:m].view(1, -1, 4)
     weights = weight_buf[:m].view(1, -1, 4)
     special_original = lay["special"]
-    special_compact = o2c.index_select(0, special_original)
     plan = WeightedBilinearTokenPlan(
         keep=keep, source_original=source_original,
         source_parent_compact=parent_compact,

@@ -66,11 +66,7 @@ class _Csr:
 # ----------------------------------------------------------------------------
 def _corner_csr(parent_compact: torch.Tensor, kept_tokens: int) -> _Csr:
     """Stable CSR of (destination, corner) pairs: item p = i*S + c, key = parent*S + c."""
-    corners = parent_compact.shape[-1]
-    parent = parent_compact.reshape(-1, corners)
-    key = parent * corners + torch.arange(corners, device=parent.device)
-    key = torch.where(parent >= 0, key, torch.full_like(key, kept_tokens * corners))
-    order, offsets = _kernels.csr_build(key.reshape(-1), kept_tokens * corners)
+    order, offsets = _kernels.corner_csr(parent_compact.reshape(-1, parent_compact.shape[-1]), kept_tokens)
     return _Csr(order, offsets)
 
 

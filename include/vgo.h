@@ -349,6 +349,16 @@ int vgo_csr_build(const uint32_t* keys, int64_t n_items, int64_t n_buckets, void
                   size_t workspace_bytes, uint32_t* order, int32_t* offsets, void* stream);
 
 /*
+ * vgo_csr_build of the (destination, corner) pairs of a weighted plan: item
+ * p = source * corners + corner has key parent[p] * corners + corner, or none with
+ * a parent outside [0, n_dest).  Workspace: vgo_csr_workspace(n_items, n_dest * corners).
+ * vggt_omega/models/token_merging.py:323-333, 51-54.
+ */
+int vgo_corner_csr(const int64_t* parent, int64_t n_items, int64_t corners, int64_t n_dest,
+                   void* workspace, size_t workspace_bytes, uint32_t* order, int32_t* offsets,
+                   void* stream);
+
+/*
  * Per-row mass: mass[k] = (((start + S_0) + S_1) + ...), S_c = sequential sum of
  * weights[p] over the items p of segment (k, c) in CSR order (weights == NULL
  * counts items); log_mass (nullable) = log(mass).  With start = 1 and one

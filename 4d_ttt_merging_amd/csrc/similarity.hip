@@ -437,10 +437,9 @@ constexpr int kRKc = 32;
 constexpr int kRStages = 5;                 // 5 x 32 KB: all of the CU's LDS
 constexpr int kRAhead = kRStages - 1;       // steps in flight ahead of the one computed
 constexpr int kRTileElems = kRTile * kRKc;
-constexpr int kRDmaPerStep = 4;  // per wave: two 16-row blocks of each operand
 __device__ __forceinline__ int sw4(int row) { return (row >> 2) & 3; }
 
-template <int K, bool kStreamK>
+template <int K, bool kStreamK, int NB = 4>
 __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
     const bf16_t* __restrict__ src, int64_t src_stride, int64_t src_capacity,
     const int64_t* __restrict__ src_rows, const int* __restrict__ n_src_dev, int n_src,
@@ -449,7 +448,11 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
     uint64_t* __restrict__ partial, int parts, bf16_t* __restrict__ scores,
     int64_t scores_stride, int units, DeviceSplit split) {
   static_assert(!kStreamK || K == 1, "the stream-K schedule is the top-1 kernel's");
-  __shared__ __attribute__((aligned(16))) bf16_t a_lds[kRStages * kRTileElems];
+  static_assert(NB == 4 || (NB == 2 && K == 4 && !kStreamK), "half dictionary tiles: the split top-4 kernel");
+  constexpr int kDTile = 64 * NB;                  // dictionary rows of a tile
+  constexpr int kDTileElems = kDTile * kRKc;
+  constexpr int kDma = NB / 2 + 2;                 // per wave and step: 16-row blocks of both operands
+  __shared__ __attribute__((aligned(16))) bf16_t a_lds[kRStages * kDTileElems];
   __shared__ __attribute__((aligned(16))) bf16_t b_lds[kRStages * kRTileElems];
 
   int ns = n_src;
@@ -485,21 +488,22 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
     s0 = (task / parts) * kRTile;
     if (s0 >= ns) return;
     part = task % parts;
-    d_begin = part * tiles_per_part * kRTile;
-    d_end = min(n_dict, d_begin + tiles_per_part * kRTile);
+    d_begin = part * tiles_per_part * kDTile;
+    d_end = min(n_dict, d_begin + tiles_per_part * kDTile);
   }
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wd = wave & 1;   // dictionary half (128 rows)
+  const int wd = wave & 1;   // dictionary half (32 NB rows)
   const int ws = wave >> 1;  // source quarter (64 rows)
   const int l32 = lane & 31;
   const int hh = lane >> 5;
 
   // DMA lanes: a 1 KB block is 16 rows x 4 physical chunks; lane i fills row
   // i/4, physical chunk i%4 with logical chunk (i%4) ^ sw4(row).  This wave
-  // loads rows 32*wave + 16*j + i/4 (j = 0, 1) of both operands.
+  // loads rows 32*wave + 16*j + i/4 (j = 0, 1) of the sources, and of the dictionary
+  // the same or, of half tiles, rows 16*wave + i/4.
   const int dr = lane >> 2;
   const int dpc = lane & 3;
   const bf16_t* src_p[2];
@@ -529,16 +533,16 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
   set_epilogue_stile(s0 / kRTile);
 
   const int n_chunks = dim / kRKc;
-  const int n_dtiles = kStreamK ? n_units : d_end > d_begin ? (d_end - d_begin + kRTile - 1) / kRTile : 0;
+  const int n_dtiles = kStreamK ? n_units : d_end > d_begin ? (d_end - d_begin + kDTile - 1) / kDTile : 0;
   const int n_steps = n_dtiles * n_chunks;
 
-  const bf16_t* dict_p[2] = {dict, dict};
+  const bf16_t* dict_p[NB / 2];
   int cur_dt = -1;
   auto set_dtile = [&](int dt) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int r = 32 * wave + 16 * j + dr;
-      const int jj = min(d_begin + dt * kRTile + r, d_end - 1);  // rows past the end repeat a valid row
+    for (int j = 0; j < NB / 2; ++j) {
+      const int r = 8 * NB * wave + 16 * j + dr;
+      const int jj = min(d_begin + dt * kDTile + r, d_end - 1);  // rows past the end repeat a valid row
       const int row = jj < n0 ? jj : off1 + (jj - n0);
       dict_p[j] = dict + static_cast<int64_t>(row) * dict_stride + 8 * (dpc ^ sw4(r));
     }
@@ -551,18 +555,21 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
   // outstanding" would no longer mean that the oldest step has landed.
   int iss_step = 0, iss_dt = dt_begin, iss_kc = 0, iss_stage = 0;
   int iss_st = st_begin;  // kStreamK: the issued step's source tile
-  // DMA q (0..3) of the next step: block q >> 1 of the dictionary (q even) or
-  // source (q odd) operand; the last one moves on to the following step.
+  // DMA q (0..kDma - 1) of the next step: block q >> 1 of the dictionary (q even) or
+  // source (q odd) operand -- of half tiles the dictionary's block, then the sources'
+  // two; the last one moves on to the following step.
   auto issue_one = [&](int q) {
     if (q == 0 && iss_dt != cur_dt) set_dtile(iss_dt);
     if constexpr (kStreamK)
       if (q == 0 && iss_dt == 0 && iss_kc == 0 && iss_step > 0) set_stile(iss_st);
-    const int blk = (32 * wave + 16 * (q >> 1)) * kRKc;
-    if ((q & 1) == 0)
-      lds_dma16_addr(dict_p[q >> 1] + iss_kc, lds_offset(a_lds + iss_stage * kRTileElems + blk));
+    const bool of_dict = NB == 4 ? (q & 1) == 0 : q == 0;
+    const int j = NB == 4 ? q >> 1 : q == 0 ? 0 : q - 1;
+    if (of_dict)
+      lds_dma16_addr(dict_p[j] + iss_kc,
+                     lds_offset(a_lds + iss_stage * kDTileElems + (8 * NB * wave + 16 * j) * kRKc));
     else
-      lds_dma16_addr(src_p[q >> 1] + iss_kc, lds_offset(b_lds + iss_stage * kRTileElems + blk));
-    if (q == 3) {
+      lds_dma16_addr(src_p[j] + iss_kc, lds_offset(b_lds + iss_stage * kRTileElems + (32 * wave + 16 * j) * kRKc));
+    if (q == kDma - 1) {
       iss_stage = iss_stage == kRStages - 1 ? 0 : iss_stage + 1;
       if (++iss_step < n_steps) {
         iss_kc += kRKc;
@@ -581,7 +588,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
   };
   auto issue_next = [&]() {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) issue_one(q);
+    for (int q = 0; q < kDma; ++q) issue_one(q);
   };
   // Operand read offsets (elements) within a 32-row block: logical chunk 2t+hh
   // of row l32; sw4 of rows 32*x + l32 + base depends on l32 only.
@@ -594,39 +601,39 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
   best[1].init();
   float top_v[2] = {-__builtin_inff(), -__builtin_inff()};
   int top_j[2] = {-1, -1};
-  f32x16 acc[4][2];
+  f32x16 acc[NB][2];
 #pragma unroll
-  for (int x = 0; x < 4; ++x)
+  for (int x = 0; x < NB; ++x)
 #pragma unroll
     for (int y = 0; y < 2; ++y) acc[x][y] = f32x16{};
 
   // Operands of one 16-wide k-step t of the step in stage `stg`: this wave's
-  // 128 dictionary rows (4 blocks) and 64 source rows (2 blocks).
-  auto read_half = [&](int stg, int t, bf16x8 (&a)[4], bf16x8 (&b)[2]) {
-    const bf16_t* al = a_lds + stg * kRTileElems + wd * 128 * kRKc;
+  // dictionary rows (NB blocks of 32) and 64 source rows (2 blocks).
+  auto read_half = [&](int stg, int t, bf16x8 (&a)[NB], bf16x8 (&b)[2]) {
+    const bf16_t* al = a_lds + stg * kDTileElems + wd * 32 * NB * kRKc;
     const bf16_t* bl = b_lds + stg * kRTileElems + ws * 64 * kRKc;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) a[x] = *reinterpret_cast<const bf16x8*>(al + x * 32 * kRKc + off[t]);
+    for (int x = 0; x < NB; ++x) a[x] = *reinterpret_cast<const bf16x8*>(al + x * 32 * kRKc + off[t]);
 #pragma unroll
     for (int y = 0; y < 2; ++y) b[y] = *reinterpret_cast<const bf16x8*>(bl + y * 32 * kRKc + off[t]);
   };
-  auto mma_half = [&](const bf16x8 (&a)[4], const bf16x8 (&b)[2]) {
+  auto mma_half = [&](const bf16x8 (&a)[NB], const bf16x8 (&b)[2]) {
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+    for (int x = 0; x < NB; ++x)
 #pragma unroll
       for (int y = 0; y < 2; ++y)
         acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x], b[y], acc[x][y], 0, 0, 0);
   };
   // k-step 0 operands of the current step (read a step ahead) and k-step 1
   // operands (read at the step's start, under k-step 0's MFMAs).
-  bf16x8 a0[4], b0[2], a1[4], b1[2];
+  bf16x8 a0[NB], b0[2], a1[NB], b1[2];
   if (n_steps > 0) {
     // The index loads above complete here, so no compiler-inserted wait for
     // them (which would count the untracked DMAs too) lands in the ring.
     wait_vmem<0>();
 #pragma unroll
     for (int st = 0; st < kRAhead; ++st) issue_next();
-    wait_vmem<(kRAhead - 1) * kRDmaPerStep>();  // step 0 has landed
+    wait_vmem<(kRAhead - 1) * kDma>();  // step 0 has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read_half(0, 0, a0, b0);
@@ -640,23 +647,23 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
     // the previous barrier.  A wave arriving at the barrier leaves MFMAs in
     // the pipe, and the other wave of its SIMD keeps issuing them, so barrier
     // skew does not idle the matrix cores.
-    if (K == 1) {
+    if constexpr (K == 1) {
       // The compiler interleaves the reads with the MFMAs.
       read_half(stage, 1, a1, b1);
       mma_half(a0, b0);
     } else {
       // One read after each MFMA (the top-4 epilogue leaves the compiler
       // fewer registers to hoist the reads with).
-      const bf16_t* al = a_lds + stage * kRTileElems + wd * 128 * kRKc;
+      const bf16_t* al = a_lds + stage * kDTileElems + wd * 32 * NB * kRKc;
       const bf16_t* bl = b_lds + stage * kRTileElems + ws * 64 * kRKc;
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
+      for (int x = 0; x < NB; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y) {
           acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0[x], b0[y], acc[x][y], 0, 0, 0);
           const int q = 2 * x + y;
-          if (q < 4) a1[q] = *reinterpret_cast<const bf16x8*>(al + q * 32 * kRKc + off[1]);
-          else if (q < 6) b1[q - 4] = *reinterpret_cast<const bf16x8*>(bl + (q - 4) * 32 * kRKc + off[1]);
+          if (q < NB) a1[q] = *reinterpret_cast<const bf16x8*>(al + q * 32 * kRKc + off[1]);
+          else if (q < NB + 2) b1[q - NB] = *reinterpret_cast<const bf16x8*>(bl + (q - NB) * 32 * kRKc + off[1]);
           __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -665,7 +672,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
     // has finished step - 1, whose stage the DMAs below refill.  A wave's
     // reads of a stage are consumed by its MFMAs before its next barrier, so
     // the barrier need not wait for LDS reads in flight.
-    wait_vmem<(kRAhead - 2) * kRDmaPerStep>();
+    wait_vmem<(kRAhead - 2) * kDma>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     // k-step 1's MFMAs with step + 4's four DMAs issued between them: a DMA
@@ -674,10 +681,10 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
     // next step's k-step 0 operands are unconditional: after the last step
     // they read a stage nobody uses, and a branch here would make the wait
     // above cover them too.
-    if (K == 1) {
+    if constexpr (K == 1) {
       read_half(next, 0, a0, b0);
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
+      for (int x = 0; x < NB; ++x) {
 #pragma unroll
         for (int y = 0; y < 2; ++y)
           acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1[x], b1[y], acc[x][y], 0, 0, 0);
@@ -686,19 +693,20 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      const bf16_t* al = a_lds + next * kRTileElems + wd * 128 * kRKc;
+      const bf16_t* al = a_lds + next * kDTileElems + wd * 32 * NB * kRKc;
       const bf16_t* bl = b_lds + next * kRTileElems + ws * 64 * kRKc;
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
+      for (int x = 0; x < NB; ++x) {
 #pragma unroll
         for (int y = 0; y < 2; ++y) {
           acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1[x], b1[y], acc[x][y], 0, 0, 0);
           const int q = 2 * x + y;
-          if (q < 4) a0[q] = *reinterpret_cast<const bf16x8*>(al + q * 32 * kRKc + off[0]);
-          else if (q < 6) b0[q - 4] = *reinterpret_cast<const bf16x8*>(bl + (q - 4) * 32 * kRKc + off[0]);
+          if (q < NB) a0[q] = *reinterpret_cast<const bf16x8*>(al + q * 32 * kRKc + off[0]);
+          else if (q < NB + 2) b0[q - NB] = *reinterpret_cast<const bf16x8*>(bl + (q - NB) * 32 * kRKc + off[0]);
           __builtin_amdgcn_sched_barrier(0);
         }
         issue_one(x);
+        if (NB == 2 && x == 1) issue_one(2);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -708,28 +716,28 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
 #pragma unroll
         for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-          for (int db = 0; db < 4; ++db)
+          for (int db = 0; db < NB; ++db)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[db][sb][r] = src_ok[sb] ? acc[db][sb][r] : 0.0f;
       }
       if constexpr (kStreamK) s0 = st * kRTile;
-      const int d0 = d_begin + dt * kRTile;
+      const int d0 = d_begin + dt * kDTile;
       if (!kStreamK && scores) {  // the stream-K kernel never writes scores
 #pragma unroll
         for (int sb = 0; sb < 2; ++sb) {
           const int i = s0 + 64 * ws + 32 * sb + l32;
 #pragma unroll
-          for (int db = 0; db < 4; ++db)
+          for (int db = 0; db < NB; ++db)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-              const int jj = d0 + 128 * wd + 32 * db + 8 * (r >> 2) + 4 * hh + (r & 3);
+              const int jj = d0 + 32 * NB * wd + 32 * db + 8 * (r >> 2) + 4 * hh + (r & 3);
               if (jj < d_end && i < ns)
                 scores[static_cast<int64_t>(i) * scores_stride + jj] = static_cast<bf16_t>(acc[db][sb][r]);
             }
         }
       }
-      const int jl = d0 + 128 * wd + 4 * hh;  // this lane's first dictionary row
-      if (K == 1) {
+      const int jl = d0 + 32 * NB * wd + 4 * hh;  // this lane's first dictionary row
+      if constexpr (K == 1) {
         // Running top-1 on the bf16-rounded score: a later (higher) j wins only
         // when strictly greater, which is the lower-index rule for ties; a NaN
         // wins over numbers and the first NaN is kept (ranking of the keys).
@@ -743,7 +751,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
         // bf16(m)'s rounding interval -- the first score that rounds to the
         // tile's bf16 maximum -- by one compare and one select per score, where
         // the per-score loop below rounds and compares every score.
-        const bool full = d0 + kRTile <= d_end;
+        const bool full = d0 + kDTile <= d_end;
         bool fast = false;
         float mx[2];
         if (full) {
@@ -751,7 +759,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
           for (int sb = 0; sb < 2; ++sb) {
             float part[4];
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
+            for (int db = 0; db < NB; ++db) {
               float m = acc[db][sb][0];
 #pragma unroll
               for (int r = 1; r < 16; r += 2)
@@ -783,13 +791,13 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
             }
           }
         } else {
-          const int lim = full ? kRTile : d_end - jl;
+          const int lim = full ? kDTile : d_end - jl;
 #pragma unroll
           for (int sb = 0; sb < 2; ++sb) {
             float tv = top_v[sb];
             int tp = -1;
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int db = 0; db < NB; ++db)
 #pragma unroll
               for (int r = 0; r < 16; ++r) {
                 const int pos = 32 * db + 8 * (r >> 2) + (r & 3);
@@ -809,14 +817,14 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
         // in the low half, so a larger key is a larger score or, for equal
         // scores, the lower dictionary row; a sorted list takes a key with one
         // max and three medians.  Other tiles take the per-score inserts.
-        const bool full = d0 + kRTile <= d_end;
+        const bool full = d0 + kDTile <= d_end;
         bool fast = false;
         if (full) {
           float m = acc[0][0][0];
 #pragma unroll
           for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int db = 0; db < NB; ++db)
 #pragma unroll
               for (int r = 0; r < 16; r += 2)
                 m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, acc[db][sb][r]),
@@ -828,7 +836,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
           for (int sb = 0; sb < 2; ++sb) {
             uint32_t l0 = 0, l1 = 0, l2 = 0, l3 = 0;
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int db = 0; db < NB; ++db)
 #pragma unroll
               for (int r = 0; r < 16; ++r) {
                 const uint32_t key = tile_key(acc[db][sb][r], 32 * db + 8 * (r >> 2) + (r & 3));
@@ -839,7 +847,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
                 l1 = n1;
                 l2 = n2;
               }
-            // 64 keys went in, so all four slots hold scores.
+            // 16 NB keys went in, so all four slots hold scores.
             best[sb].insert(tile_key_to_key(l0, jl));
             best[sb].insert(tile_key_to_key(l1, jl));
             best[sb].insert(tile_key_to_key(l2, jl));
@@ -849,7 +857,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
 #pragma unroll
           for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int db = 0; db < NB; ++db)
 #pragma unroll
               for (int r = 0; r < 16; ++r) {
                 const int jj = jl + 32 * db + 8 * (r >> 2) + (r & 3);
@@ -860,7 +868,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int db = 0; db < 4; ++db) acc[db][sb] = f32x16{};
+        for (int db = 0; db < NB; ++db) acc[db][sb] = f32x16{};
       kcs = 0;
       ++dt;
       if constexpr (kStreamK) {
@@ -895,7 +903,7 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
   if constexpr (kStreamK) return;
   __syncthreads();
 
-  if (K == 1) {
+  if constexpr (K == 1) {
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
       if (top_j[sb] >= 0) best[sb].k[0] = make_key(top_v[sb], top_j[sb]);
@@ -1016,27 +1024,49 @@ inline bool use_ring(int64_t n_src, int64_t n_dict, int64_t dim) {
   return dim % kRKc == 0 && (n_src + kRTile - 1) / kRTile * ((n_dict + kRTile - 1) / kRTile) > kStagedTiles;
 }
 
-// Dictionary split for a kernel with `tile` x `tile` steps: the number of parts
-// that minimises (rounds of resident work-groups) x (dictionary tiles per
-// work-group + a half-tile fixed cost).
-int choose_parts(int64_t n_src, int64_t n_dict, int topk, bool ring) {
-  const int64_t tile = ring ? kRTile : kTile;
+// Dictionary split for tiles of `tile` sources x `dict_tile` rows on `slots` resident
+// work-groups: the number of parts that minimises (rounds of resident work-groups) x
+// (dictionary tiles per work-group x `tile_cost` + half a full tile's fixed cost).
+int choose_parts(int64_t n_src, int64_t n_dict, int64_t slots, int64_t tile, int64_t dict_tile, double tile_cost,
+                 double* cost_out) {
   const int64_t src_tiles = (n_src + tile - 1) / tile;
-  const int64_t dict_tiles = (n_dict + tile - 1) / tile;
+  const int64_t dict_tiles = (n_dict + dict_tile - 1) / dict_tile;
+  *cost_out = 0.0;
   if (src_tiles <= 0 || dict_tiles <= 0) return 1;
-  const int64_t slots = topk == 1 ? resident_groups<1>(ring) : resident_groups<4>(ring);
   int best = 1;
   double best_cost = 1e300;
   for (int64_t p = 1; p <= dict_tiles && p <= 4096; ++p) {
     const int64_t rounds = (src_tiles * p + slots - 1) / slots;
     const int64_t tpp = (dict_tiles + p - 1) / p;
-    const double cost = static_cast<double>(rounds) * (static_cast<double>(tpp) + 0.5);
+    const double cost = static_cast<double>(rounds) * (static_cast<double>(tpp) * tile_cost + 0.5);
     if (cost < best_cost) {
       best_cost = cost;
       best = static_cast<int>(p);
     }
   }
+  *cost_out = best_cost;
   return best;
+}
+int choose_parts(int64_t n_src, int64_t n_dict, int topk, bool ring) {
+  const int64_t tile = ring ? kRTile : kTile;
+  double cost;
+  return choose_parts(n_src, n_dict, topk == 1 ? resident_groups<1>(ring) : resident_groups<4>(ring), tile, tile, 1.0,
+                      &cost);
+}
+
+// Parts of a top-4 ring launch with half (128-row) dictionary tiles, or 0 where whole
+// tiles cost less.  A whole tile and a list's fixed cost are about 30 and 19 us, a half
+// tile 17 and 24 (less work per operand read); halves pay where the whole tiles' last
+// round leaves much of the chip idle.  Measured (us, whole / half): 2,304 x 2,304 48 / 38,
+// 5,376 x 1,500 63 / 45, 5,672 x 2,833 79 / 74, 6,144 x 3,072 79 / 76, 3,143 x 2,833
+// 51 / 55, 8,000 x 4,105 111 / 113, 11,000 x 5,000 160 / 166, 30,000 x 9,000 622 / 725.
+constexpr double kHalfTileCost = 0.6;
+int half_tile_parts(int64_t n_src, int64_t n_dict) {
+  const int64_t slots = resident_groups<4>(true);
+  double full, half;
+  choose_parts(n_src, n_dict, slots, kRTile, kRTile, 1.0, &full);
+  const int p = choose_parts(n_src, n_dict, slots, kRTile, kRTile / 2, kHalfTileCost, &half);
+  return half < full ? p : 0;
 }
 
 // Stream-K schedule of the top-1 ring kernel over units = source tiles x
@@ -1077,6 +1107,14 @@ StreamK stream_k_schedule(int64_t n_src, int64_t n_dict) {
   return r;
 }
 
+// Lists with which a count known on the device alone can take the split that suits it: a
+// small count wants more parts than the bound's (3,143 of 5,672 sources against 2,833
+// rows: 12 parts of one tile where the bound's 6 allowed 10 of two, 90 -> 64 us).
+size_t device_lists(int64_t n_src, int64_t n_dict) {
+  const int64_t dict_tiles = (n_dict + kTile - 1) / kTile;
+  return static_cast<size_t>(std::min(n_src * dict_tiles, 2 * resident_groups<4>(true) * kRTile));
+}
+
 }  // namespace
 }  // namespace vgo
 
@@ -1087,9 +1125,9 @@ extern "C" int vgo_similarity_topk_workspace(int64_t n_src, int64_t n_dict, int 
   VGO_REQUIRE(n_src >= 0 && n_dict >= 0, "similarity_topk: negative size");
   // Sized for whichever kernel and schedule the dimension selects.
   int p = std::max(choose_parts(n_src, n_dict, topk, true), choose_parts(n_src, n_dict, topk, false));
-  if (topk == 1) p = std::max(p, stream_k_schedule(n_src, n_dict).lists);
+  p = std::max(p, topk == 1 ? stream_k_schedule(n_src, n_dict).lists : half_tile_parts(n_src, n_dict));
   if (parts) *parts = p;
-  if (bytes) *bytes = static_cast<size_t>(n_src) * p * topk * sizeof(uint64_t);
+  if (bytes) *bytes = std::max(static_cast<size_t>(n_src) * p, device_lists(n_src, n_dict)) * topk * sizeof(uint64_t);
   return VGO_OK;
 }
 
@@ -1117,12 +1155,13 @@ extern "C" int vgo_similarity_topk(const void* src, int64_t src_row_stride, int6
   VGO_REQUIRE(src_rows || n_src <= src_capacity, "similarity_topk: more sources than rows");
   const bool ring = use_ring(n_src, n_dict, dim);
   const StreamK sk = ring && topk == 1 && !scores && !n_src_device ? stream_k_schedule(n_src, n_dict) : StreamK{};
-  const int parts = sk.groups > 0 ? sk.lists : choose_parts(n_src, n_dict, topk, ring);
+  const int half = ring && topk == 4 && !n_src_device ? half_tile_parts(n_src, n_dict) : 0;
+  const int parts = sk.groups > 0 ? sk.lists : half > 0 ? half : choose_parts(n_src, n_dict, topk, ring);
   const size_t need = static_cast<size_t>(n_src) * parts * topk * sizeof(uint64_t);
   VGO_REQUIRE(workspace && workspace_bytes >= need, "similarity_topk: workspace too small");
   VGO_REQUIRE(aligned(workspace, 8), "similarity_topk: workspace must be 8-byte aligned");
   const int64_t tile = ring ? kRTile : kTile;
-  const int64_t dict_tiles = (n_dict + tile - 1) / tile;
+  const int64_t dict_tiles = half > 0 ? (n_dict + tile / 2 - 1) / (tile / 2) : (n_dict + tile - 1) / tile;
   const int tiles_per_part = sk.groups > 0 ? sk.dict_tiles : static_cast<int>((dict_tiles + parts - 1) / parts);
   hipStream_t s = as_stream(stream);
   const int64_t src_tiles = (n_src + tile - 1) / tile;
@@ -1131,7 +1170,10 @@ extern "C" int vgo_similarity_topk(const void* src, int64_t src_row_stride, int6
   int64_t groups = sk.groups > 0 ? sk.groups : src_tiles * parts;
   if (n_src_device) {
     split.slots = static_cast<int>(topk == 1 ? resident_groups<1>(ring) : resident_groups<4>(ring));
-    split.lists = n_src * parts;
+    // (A caller may bring the least workspace, n_src x parts lists.)
+    split.lists = static_cast<int64_t>(std::min(workspace_bytes / (topk * sizeof(uint64_t)),
+                                                std::max(static_cast<size_t>(n_src) * parts,
+                                                         device_lists(n_src, n_dict))));
     groups = device_groups(split, src_tiles);
   }
   dim3 grid(static_cast<unsigned>(groups));
@@ -1153,6 +1195,8 @@ extern "C" int vgo_similarity_topk(const void* src, int64_t src_row_stride, int6
       launch(sim_topk_ring_kernel<1, true>);
     else if (topk == 1)
       launch(sim_topk_ring_kernel<1, false>);
+    else if (half > 0)
+      launch(sim_topk_ring_kernel<4, false, 2>);
     else
       launch(sim_topk_ring_kernel<4, false>);
   } else if (topk == 1) {

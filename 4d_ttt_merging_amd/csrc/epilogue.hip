@@ -153,8 +153,47 @@ int launch_epilogue(const void* qkv, int64_t row_stride, int64_t n_in_rows, cons
   return check_launch("qkv_epilogue");
 }
 
+// Axial RoPE tables (vggt_omega/models/layers/rope_position_encoding.py:51-127 at inference, "max"
+// coordinates): sin and cos of 2 pi (2 (index + 1/2) / max(h, w) - 1) / base^(2 i / (dim / 2)), each
+// [h w, dim] fp32 with the columns (row angle i, column angle i) twice.  The values are those of
+// torch's elementwise operators, a division by a number being a product with its reciprocal.  One
+// launch instead of eighteen, for whose host work a small aggregator waits: its forward of 4 frames
+// of 261 tokens took 2,313 us with them and 2,156 now (means of three pairs of runs).
+__global__ __launch_bounds__(256) void rope_table_kernel(int h, int w, int quarter, float base, float* __restrict__ sin_out,
+                                                         float* __restrict__ cos_out) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int half = 2 * quarter;
+  if (t >= static_cast<int64_t>(h) * w * half) return;
+  const int64_t patch = t / half;
+  const int j = static_cast<int>(t - patch * half);
+  const int i = j < quarter ? j : j - quarter;
+  const float at = static_cast<float>(j < quarter ? patch / w : patch % w) + 0.5f;
+  const float period = powf(base, 2.0f * static_cast<float>(i) * (1.0f / static_cast<float>(half)));
+  const float coord = 2.0f * (at * (1.0f / static_cast<float>(max(h, w)))) - 1.0f;
+  const float angle = 6.28318530717958647692f * coord / period;
+  const float s = sinf(angle), c = cosf(angle);
+  const int64_t o = patch * 2 * half + j;
+  sin_out[o] = s;
+  sin_out[o + half] = s;
+  cos_out[o] = c;
+  cos_out[o + half] = c;
+}
+
 }  // namespace
 }  // namespace vgo
+
+extern "C" int vgo_rope_table(int64_t h, int64_t w, int64_t head_dim, float base, float* sin_out, float* cos_out,
+                              void* stream) {
+  using namespace vgo;
+  VGO_REQUIRE(h >= 1 && w >= 1 && head_dim >= 4 && head_dim % 4 == 0, "rope_table: bad size");
+  VGO_REQUIRE(h < (1LL << 20) && w < (1LL << 20) && head_dim < (1LL << 20) && h * w < (1LL << 34) / head_dim,
+              "rope_table: size too large");
+  VGO_REQUIRE(sin_out && cos_out, "rope_table: null pointer");
+  hipLaunchKernelGGL(rope_table_kernel, dim3(static_cast<unsigned>((h * w * (head_dim / 2) + 255) / 256)), dim3(256), 0,
+                     as_stream(stream), static_cast<int>(h), static_cast<int>(w), static_cast<int>(head_dim / 4), base,
+                     sin_out, cos_out);
+  return check_launch("rope_table");
+}
 
 using namespace vgo;
 

@@ -650,8 +650,19 @@ constexpr const char* kPure[] = {"mass_bias_attention", "top4_project", "qkv_epi
                                  "restore_residual_layer_norm", "mlp_tail", "dense_block", "normalize_rows",
                                  "csr_build", "corner_csr", "segment_mass", "fastvggt_assemble", "fastvggt_match", "fastvggt_plan",
                                  "merged_block"};
+// sin and cos tables into out[0] and out[1] of a contiguous fp32 [2, h * w, head_dim].
+void rope_table(const Tensor& out, int64_t h, int64_t w, double base) {
+  require_gpu({&out});
+  TORCH_CHECK(out.dim() == 3 && out.size(0) == 2 && out.size(1) == h * w && out.scalar_type() == at::kFloat &&
+                  out.is_contiguous(),
+              "rope_table: out must be a contiguous float32 [2, h * w, head_dim]");
+  check(vgo_rope_table(h, w, out.size(2), static_cast<float>(base), ptr<float>(out), ptr<float>(out) + out.stride(0),
+                       stream_of(out)));
+}
+
 constexpr const char* kMutating[] = {"attention_into", "attention_pair_into", "top4_project_into",
-                                     "top4_project_ordered_into", "compact_into", "compact_multi_into", "similarity_topk"};
+                                     "top4_project_ordered_into", "compact_into", "compact_multi_into", "similarity_topk",
+                                     "rope_table"};
 
 }  // namespace
 
@@ -670,6 +681,7 @@ TORCH_LIBRARY_IMPL(vgo, CUDA, m) {
   m.impl("mlp_tail", mlp_tail);
   m.impl("dense_block", dense_block);
   m.impl("normalize_rows", normalize_rows);
+  m.impl("rope_table", rope_table);
   m.impl("csr_build", csr_build);
   m.impl("corner_csr", corner_csr);
   m.impl("segment_mass", segment_mass);

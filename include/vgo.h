@@ -412,6 +412,13 @@ int vgo_compact_multi(const void* x, int64_t x_token_stride, int64_t x_head_stri
                       const int64_t* out_head_strides, int dtype, void* stream);
 
 /*
+ * Axial RoPE tables at inference, "max" coordinates, fp32 [h * w, head_dim] each (head_dim a multiple
+ * of 4): vggt_omega/models/layers/rope_position_encoding.py:51-127.
+ */
+int vgo_rope_table(int64_t h, int64_t w, int64_t head_dim, float base, float* sin_out, float* cos_out,
+                   void* stream);
+
+/*
  * Fused QKV epilogue: from packed projection rows qkv[src] = [q | k | v] (each
  * heads*64 channels), write head-major q/k/v [seq, heads, tokens_out, 64] for
  * output rows r (src = rows ? rows[r] : r; seq = r / tokens_out), applying the

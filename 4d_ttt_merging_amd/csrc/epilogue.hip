@@ -110,12 +110,13 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(
     for (int c0 = lane * 16; c0 < C; c0 += 1024) {
       const int h = c0 >> 6;
       const int64_t o = ((static_cast<int64_t>(seq) * heads + h) * t_out + t) * 64 + d0;
-      // The packed row always holds q, k and v, so the three loads are issued
-      // together, whichever outputs are written, and wait once.
+      // The packed row always holds q, k and v, so the loads are issued together
+      // and wait once; v only where it is written (an attention that reads v from
+      // the packed rows saves both).
       float vq[16], vk[16], vv[16];
       load16(row + c0, vq);
       load16(row + C + c0, vk);
-      load16(row + 2 * C + c0, vv);
+      if (v_out) load16(row + 2 * C + c0, vv);
       if (v_out) store16(v_out + o, vv);
       if (q_out) {
         if (qw) head_layer_norm(vq, ln_lds[0] + d0, ln_lds[1] + d0, eps);

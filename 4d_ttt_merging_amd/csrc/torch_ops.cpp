@@ -430,12 +430,18 @@ Tensor dense_block(const Tensor& x, const c10::List<OptTensor>& norms, at::Array
   const Tensor qkv = linear(h, 0);
   const int64_t prefix = opt(rope_sin) == nullptr ? 0 : tokens - rope_sin->size(-2);
   TORCH_CHECK(prefix >= 0, "dense_block: more RoPE positions than tokens");
+  // The attention takes v where the projection wrote it: copying it head-major was a third of
+  // the epilogue's bytes (a block of 32 x 1,029 tokens 1,384 -> 1,370 us).  Copied only where the
+  // kernels' 32-bit token offsets (stride x tokens < 2^31) do not reach; layers.py `_value_rows`
+  // is the same rule.
+  const bool v_in_place = tokens * 3 * dim < (int64_t{1} << 31);
   const std::vector<Tensor> heads_out =
       qkv_epilogue(qkv.reshape({batch * tokens, 3 * dim}), heads, tokens, tokens, std::nullopt, norms.get(4),
                    norms.get(5), norms.get(6), norms.get(7), eps[2], rope_sin, rope_cos, prefix,
-                   c10::List<bool>({true, true, true}), dtype);
+                   c10::List<bool>({true, true, !v_in_place}), dtype);
+  const Tensor v = v_in_place ? qkv.view({batch, tokens, 3, heads, 64}).select(2, 2).transpose(1, 2) : heads_out[2];
   const Tensor attended = at::empty({batch, tokens, heads, 64}, x.options().dtype(dtype));
-  attention_into(heads_out[0], heads_out[1], heads_out[2], std::nullopt, attended.permute({0, 2, 1, 3}), -1);
+  attention_into(heads_out[0], heads_out[1], v, std::nullopt, attended.permute({0, 2, 1, 3}), -1);
   const std::vector<Tensor> rows =
       residual_layer_norm(x, linear(attended.view({batch, tokens, dim}), 1), gammas.get(0), norms.get(2), norms.get(3),
                           eps[1], true, true, dtype, false, -1.0);

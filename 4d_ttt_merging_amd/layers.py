@@ -276,10 +276,12 @@ class SelfAttention(nn.Module):
             rope_prefix = N - rope[0].shape[-2]
             assert rope_prefix >= 0
         rows = qkv.reshape(B * N, 3 * C)
+        values = _value_rows(qkv, dtype, H)
         q, k, v = _kernels.qkv_epilogue(
             rows, H, tokens_in=N, q_norm=None if qn is None else qn[:2],
             k_norm=None if kn is None else kn[:2], eps=qn[2] if qn is not None else 1e-5,
-            rope=rope, rope_prefix=rope_prefix, out_dtype=dtype)
+            rope=rope, rope_prefix=rope_prefix, want=(True, True, values is None), out_dtype=dtype)
+        v = v if values is None else values
         out = torch.empty((B, N, H, 64), device=qkv.device, dtype=dtype)
         _attention_into(q, k, v, None, out.permute(0, 2, 1, 3))
         return out.view(B, N, C)
@@ -689,6 +691,15 @@ def _cast_linears(*linears: nn.Module) -> tuple | None:
             return None
         cast += pair
     return tuple(cast)
+
+
+def _value_rows(qkv: Tensor, dtype: torch.dtype, heads: int) -> Tensor | None:
+    """v of contiguous packed rows [B, N, 3C] as the attention reads it in place, [B, H, N, 64], or
+    None: rows of another dtype, fp32, or token offsets past the kernels' 32 bits."""
+    B, N, width = qkv.shape
+    if qkv.dtype != dtype or dtype == torch.float32 or not qkv.is_contiguous() or N * width >= 1 << 31:
+        return None
+    return qkv.view(B, N, 3, heads, 64).select(2, 2).transpose(1, 2)
 
 
 def _autocast_dtype() -> torch.dtype | None:

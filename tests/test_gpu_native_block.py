@@ -69,6 +69,24 @@ def test_merged_block(vgo, device, mass):
             block.forward_compacted(x, bad)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch,tokens", [(1, 1), (3, 37), (1, 2700)])  # 2,700: the workspace kernel
+def test_values_in_place(vgo, device, dtype, batch, tokens):
+    """Attention over v in the packed rows equals attention over a head-major copy."""
+    layers = __import__("importlib").import_module("4d_ttt_merging_amd.layers")
+    qkv = torch.randn(batch, tokens, 3 * 128, device=device).to(dtype)
+    v = layers._value_rows(qkv, dtype, 2)
+    q, k, copied = (t.contiguous() for t in qkv.view(batch, tokens, 3, 2, 64).permute(2, 0, 3, 1, 4))
+    assert torch.equal(v, copied)
+    assert torch.equal(torch.ops.vgo.mass_bias_attention(q, k, v, None),
+                       torch.ops.vgo.mass_bias_attention(q, k, copied, None))
+    assert layers._value_rows(qkv.float(), torch.float32, 2) is None
+    assert layers._value_rows(qkv.transpose(0, 2).contiguous().transpose(0, 2), dtype, 2) is None or batch == tokens == 1
+    for n, none in ((5592405, False), (5592406, True)):  # x 384 channels: either side of 2^31
+        far = layers._value_rows(torch.empty(1, n, 384, device="meta", dtype=dtype), dtype, 2)
+        assert (far is None) == none
+
+
 def test_replaced_modules_run_call_by_call(vgo, device):
     """Subclasses, replaced methods, dispatch modes and global hooks all see their calls."""
     from torch.utils._python_dispatch import TorchDispatchMode

@@ -134,6 +134,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_int, _c_p, _c_p, _c_i64, _c_p,
         _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_p, _c_f32, _c_p, _c_p, _c_p, _c_int, _c_p,
     ]),
+    "vgo_gelu_bf16": (_c_int, [_c_p, _c_p, _c_i64, _c_p]),
     "vgo_rope_table": (_c_int, [_c_i64, _c_i64, _c_i64, _c_f32, _c_p, _c_p, _c_p]),
     "vgo_qkv_epilogue": (_c_int, [
         _c_p, _c_i64, _c_i64, _c_int, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p,

@@ -419,6 +419,12 @@ int vgo_rope_table(int64_t h, int64_t w, int64_t head_dim, float base, float* si
                    void* stream);
 
 /*
+ * Exact (erf) GELU of n bf16 values, evaluated in fp32 and rounded once; out may be x.  Both
+ * 16-byte aligned.
+ */
+int vgo_gelu_bf16(const void* x, void* out, int64_t n, void* stream);
+
+/*
  * Fused QKV epilogue: from packed projection rows qkv[src] = [q | k | v] (each
  * heads*64 channels), write head-major q/k/v [seq, heads, tokens_out, 64] for
  * output rows r (src = rows ? rows[r] : r; seq = r / tokens_out), applying the

@@ -300,16 +300,29 @@ class WeightedBilinearTokenPlan:
 
         `layer_norm` = (weight, bias, eps) normalises every gathered row per
         64-channel head before pooling (the q/k norm of the attention)."""
-        keep = self._flat("keep", self.keep, torch.int64)
         if self.source_original.shape[1] == 0 or not self.pool_source_content:
-            return self._gather_into(keep, x, out, layer_norm)
-        return _kernels.compact_into(
-            x, out, base_rows=keep, offsets=self._csr.offsets,
-            segs_per_row=self.source_parent_compact.shape[-1], items=self._csr.order,
-            item_shift=2 if self.source_parent_compact.shape[-1] == 4 else 0,
-            item_rows=self._flat("source", self.source_original, torch.int64),
-            weights=self._flat("pool_w", self.source_pool_weights, torch.float32),
-            normalizer=self._flat("norm", self.normalizer, torch.float32), layer_norm=layer_norm)
+            return self._gather_into(self._flat("keep", self.keep, torch.int64), x, out, layer_norm)
+        return _kernels.compact_into(x, out, layer_norm=layer_norm, **self._segments())
+
+    def _segments(self) -> dict:
+        """The pooling of a compact row: its own row, then its sources' by corner."""
+        return dict(base_rows=self._flat("keep", self.keep, torch.int64), offsets=self._csr.offsets,
+                    segs_per_row=self.source_parent_compact.shape[-1], items=self._csr.order,
+                    item_shift=2 if self.source_parent_compact.shape[-1] == 4 else 0,
+                    item_rows=self._flat("source", self.source_original, torch.int64),
+                    weights=self._flat("pool_w", self.source_pool_weights, torch.float32),
+                    normalizer=self._flat("norm", self.normalizer, torch.float32))
+
+    def pools_qkv_together(self) -> bool:
+        """Queries (where they are compacted), keys and values all are compact_into's rows."""
+        return (type(self) is WeightedBilinearTokenPlan and self.pool_source_content
+                and self.source_original.shape[1] > 0
+                and (not self.preserve_destination_keys if self.preserve_queries else self.query_keep is None))
+
+    def compact_multi_into(self, x: torch.Tensor, outputs) -> None:
+        """compact_into of several channel ranges of one [N, W] row table in one launch (of plans
+        that pool sources); `outputs` holds (channel offset, out, layer_norm or None) per output."""
+        _kernels.compact_multi_into(x, outputs, **self._segments())
 
     def compact(self, value: torch.Tensor, *, merge: bool = True) -> torch.Tensor:
         """Pool source Q/K/V mass into its four retained bilinear parents."""

@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import functools
 import math
+from contextlib import nullcontext
 from dataclasses import dataclass, field
 from typing import Callable
 
@@ -59,6 +60,17 @@ def _zero_offsets(cache: dict, rows: int, device) -> torch.Tensor:
 class _Csr:
     order: torch.Tensor      # int32 item ids grouped by segment (stable)
     offsets: torch.Tensor    # int32 [segments + 1]
+
+
+@dataclass
+class _Built:
+    """The clusters of an `inverse` (at one version of its contents) as a builder's launch left them."""
+
+    inverse: torch.Tensor
+    version: int
+    inverse32: torch.Tensor  # inverse[0] as int32
+    csr: _Csr
+    counts: torch.Tensor     # float32 [K], all members
 
 
 # ----------------------------------------------------------------------------
@@ -126,19 +138,35 @@ class TokenPlan:
         """inverse[b] as int32: the CSR keys and the one-hot restore map."""
         key = ("inverse32", b)
         if key not in self._derived:
-            self._derived[key] = self.inverse[b].to(torch.int32).contiguous()
+            built = self._as_built(b)
+            self._derived[key] = (self.inverse[b].to(torch.int32).contiguous() if built is None
+                                  else built.inverse32)
         return self._derived[key]
 
     def _cluster_csr(self, b: int) -> tuple[_Csr, torch.Tensor]:
         key = ("csr", b)
         if key not in self._derived:
-            order, offsets = _kernels.csr_build(self._inverse32(b), self.kept_tokens)
+            built = self._as_built(b)
+            csr = built.csr if built is not None else _Csr(
+                *_kernels.csr_build(self._inverse32(b), self.kept_tokens))
             contribution = None if self.pool_mask is None else self.pool_mask[b].to(torch.float32)
-            counts, _ = _kernels.segment_mass(offsets, 1, order, contribution, self.kept_tokens,
-                                              0.0, want_log=False)
-            self._derived[key] = (_Csr(order, offsets), counts, contribution)
+            if built is not None and contribution is None:
+                counts = built.counts
+            else:
+                counts, _ = _kernels.segment_mass(csr.offsets, 1, csr.order, contribution, self.kept_tokens,
+                                                  0.0, want_log=False)
+            self._derived[key] = (csr, counts, contribution)
         csr, counts, _ = self._derived[key]
         return csr, counts
+
+    def _as_built(self, b: int) -> _Built | None:
+        """What the builder's launch derived from `inverse`, if `inverse` and the kept count
+        still are what it derived them from."""
+        built = self._derived.get("built") if b == 0 else None
+        if (built is None or built.inverse is not self.inverse or built.version != self.inverse._version
+                or built.csr.offsets.numel() != self.kept_tokens + 1):
+            return None
+        return built
 
     def _contribution(self, b: int) -> torch.Tensor | None:
         self._cluster_csr(b)
@@ -557,22 +585,27 @@ def build_fastvggt_plan(
         raise ValueError("mass-bias FastVGGT plans support batch size one")
     one_launch = batch == 1 and _kernels._lib.load().vgo_fastvggt_plan_fits(sources.numel(), total, removed)
     if one_launch:
-        keep, inverse, flags, inverse32, order, offsets, counts, log_mass = torch.ops.vgo.fastvggt_plan(
-            best, target, sources, destinations, total, removed)
+        # Tensors with a version counter, also under inference mode: a plan is open to its caller,
+        # and what this launch derives from `inverse` holds only while that is as it was.
+        with torch.inference_mode(False) if torch.is_inference_mode_enabled() else nullcontext():
+            keep, inverse, flags, inverse32, order, offsets, counts, log_mass = torch.ops.vgo.fastvggt_plan(
+                best, target, sources, destinations, total, removed)
     else:
         keep, inverse, flags = torch.ops.vgo.fastvggt_assemble(best, target, sources, destinations, total, removed)
     plan = TokenPlan(keep, inverse, total)
     # Match results stay on the device for diagnostics and tests.
     plan._derived["match"] = (sources, destinations, best, target, flags)
     if one_launch:
-        plan._derived[("inverse32", 0)] = inverse32
+        plan._derived["built"] = _Built(inverse, inverse._version, inverse32, _Csr(order, offsets), counts)
     elif mass_bias:
         # One mass pass gives the cluster counts _cluster_csr caches and their logs.
         order, offsets = _kernels.csr_build(plan._inverse32(0), plan.kept_tokens)
         counts, log_mass = _kernels.segment_mass(offsets, 1, order, None, plan.kept_tokens, 0.0,
                                                  want_log=True)
-    if one_launch or mass_bias:
-        plan._derived[("csr", 0)] = (_Csr(order, offsets), counts, None)
     if mass_bias:
+        # The clusters whose sizes the mass is; without it they are derived on first use, from
+        # the plan as it is then (its pool_mask, say).
+        plan._inverse32(0)
+        plan._derived[("csr", 0)] = (_Csr(order, offsets), counts, None)
         plan.key_log_mass = log_mass.view(1, -1)
     return plan

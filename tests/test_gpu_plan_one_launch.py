@@ -55,3 +55,43 @@ def test_plans_that_do_not_fit_take_the_launches(vgo, device):
     total, best, target, sources, destinations = _case(1, 9000, 3000, 289, device, "bf16")
     with pytest.raises(RuntimeError, match="too many tokens"):
         torch.ops.vgo.fastvggt_plan(best, target, sources, destinations, total, 6000)
+
+
+@pytest.mark.parametrize("mode", ["no_grad", "inference"])
+@pytest.mark.parametrize("side", [8, 80])  # 195 and 19,203 tokens: the one launch, and the launches
+def test_a_plan_changed_before_its_first_use_pools_as_changed(vgo, device, side, mode):
+    """A mask, an inverse or its contents set on a built plan count, as on a plan constructed with them."""
+    frames, special = 3, 1
+    per_frame = special + side * side
+    g = torch.Generator(device=device).manual_seed(side)
+    x = torch.randn(1, frames * per_frame, 64, device=device, generator=g)
+
+    def build():
+        return vgo.build_fastvggt_plan(x, frames=frames, tokens_per_frame=per_frame, patch_token_start=special,
+                                       patch_hw=(side, side), merge_ratio=0.5, protect_ratio=0.0)
+
+    with torch.inference_mode() if mode == "inference" else torch.no_grad():
+        plain = build()
+        total, kept = plain.original_tokens, plain.kept_tokens
+        print(f"[changed plan] {total} tokens, {kept} kept, {mode}", flush=True)
+        counts = torch.bincount(plain.inverse[0].cpu(), minlength=kept)
+        assert torch.equal(plain.cluster_counts().cpu(), counts.float())
+        # Every cluster keeps its representative, so that no masked count is zero.
+        mask = torch.rand(1, total, device=device, generator=g) < 0.5
+        mask[0, plain.keep[0]] = True
+        other = plain.inverse.flip(1)
+        expect = vgo.TokenPlan(plain.keep, plain.inverse.clone(), total, pool_mask=mask)
+        flipped = vgo.TokenPlan(plain.keep, other.clone(), total)
+
+        masked = build()
+        masked.pool_mask = mask
+        assert torch.equal(masked.cluster_counts(), expect.cluster_counts())
+        assert torch.equal(masked.compact(x), expect.compact(x)) and not torch.equal(masked.compact(x), plain.compact(x))
+        replaced = build()
+        replaced.inverse = other
+        written = build()
+        written.inverse.copy_(other)
+        for plan in (replaced, written):
+            assert torch.equal(plan._inverse32(0), other[0].int())
+            assert torch.equal(plan.cluster_counts(), flipped.cluster_counts())
+            assert torch.equal(plan.compact(x), flipped.compact(x))

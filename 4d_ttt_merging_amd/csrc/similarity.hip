@@ -536,7 +536,11 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void sim_topk_ring_kernel(
   const int n_dtiles = kStreamK ? n_units : d_end > d_begin ? (d_end - d_begin + kDTile - 1) / kDTile : 0;
   const int n_steps = n_dtiles * n_chunks;
 
+  // Without a first value here the compiler lays the loop's refill out of line, which costs the
+  // top-1 kernels (23,808 x 8,960 404.5 us without, 401.7 with; 23,464 x 8,232 396.2 and 391.2);
+  // the top-4 kernel is the faster one without (473.8 and 476.2).
   const bf16_t* dict_p[NB / 2];
+  if constexpr (K == 1) dict_p[0] = dict_p[1] = dict;
   int cur_dt = -1;
   auto set_dtile = [&](int dt) {
 #pragma unroll

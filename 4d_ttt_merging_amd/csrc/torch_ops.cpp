@@ -8,11 +8,13 @@
 //
 // Every implementation checks shapes and types, allocates outputs and
 // workspaces with torch, and launches on torch's current stream of the
-// tensors' device; none synchronises.  Autograd: outputs of inputs that
+// tensors' device, which is the current device meanwhile (`on_device`); none
+// synchronises.  Autograd: outputs of inputs that
 // require grad have a backward that raises (the path is inference only), and
 // operators have no batching rule (vmap raises).
 #include <ATen/ATen.h>
 #include <ATen/core/grad_mode.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/library.h>
@@ -681,32 +683,48 @@ constexpr const char* kMutating[] = {"attention_into", "attention_pair_into", "t
                                      "top4_project_ordered_into", "compact_into", "compact_multi_into", "similarity_topk",
                                      "rope_table"};
 
+// `fn` with its first argument's device as the current device.  The kernels' launches, the device
+// properties that size them and static scratch all go by the current device, and torch's default
+// stream of any device is the null stream, that is, the current device's.
+template <auto fn>
+struct OnDevice;
+template <typename R, typename... Rest, R (*fn)(const Tensor&, Rest...)>
+struct OnDevice<fn> {
+  static R call(const Tensor& first, Rest... rest) {
+    c10::OptionalDeviceGuard guard;
+    if (first.is_cuda()) guard.reset_device(first.device());
+    return fn(first, std::forward<Rest>(rest)...);
+  }
+};
+template <auto fn>
+constexpr auto on_device = &OnDevice<fn>::call;
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(vgo, CUDA, m) {
-  m.impl("mass_bias_attention", mass_bias_attention);
-  m.impl("attention_into", attention_into);
-  m.impl("attention_pair_into", attention_pair_into);
-  m.impl("top4_project", top4_project);
-  m.impl("top4_project_into", top4_project_into);
-  m.impl("top4_project_ordered_into", top4_project_ordered_into);
-  m.impl("compact_into", compact_into);
-  m.impl("compact_multi_into", compact_multi_into);
-  m.impl("qkv_epilogue", qkv_epilogue);
-  m.impl("residual_layer_norm", residual_layer_norm);
-  m.impl("restore_residual_layer_norm", restore_residual_layer_norm);
-  m.impl("mlp_tail", mlp_tail);
-  m.impl("dense_block", dense_block);
-  m.impl("normalize_rows", normalize_rows);
-  m.impl("rope_table", rope_table);
-  m.impl("csr_build", csr_build);
-  m.impl("corner_csr", corner_csr);
-  m.impl("segment_mass", segment_mass);
-  m.impl("fastvggt_assemble", fastvggt_assemble);
-  m.impl("fastvggt_match", fastvggt_match);
-  m.impl("fastvggt_plan", fastvggt_plan);
-  m.impl("similarity_topk", similarity_topk);
-  m.impl("merged_block", merged_block);
+  m.impl("mass_bias_attention", on_device<mass_bias_attention>);
+  m.impl("attention_into", on_device<attention_into>);
+  m.impl("attention_pair_into", on_device<attention_pair_into>);
+  m.impl("top4_project", on_device<top4_project>);
+  m.impl("top4_project_into", on_device<top4_project_into>);
+  m.impl("top4_project_ordered_into", on_device<top4_project_ordered_into>);
+  m.impl("compact_into", on_device<compact_into>);
+  m.impl("compact_multi_into", on_device<compact_multi_into>);
+  m.impl("qkv_epilogue", on_device<qkv_epilogue>);
+  m.impl("residual_layer_norm", on_device<residual_layer_norm>);
+  m.impl("restore_residual_layer_norm", on_device<restore_residual_layer_norm>);
+  m.impl("mlp_tail", on_device<mlp_tail>);
+  m.impl("dense_block", on_device<dense_block>);
+  m.impl("normalize_rows", on_device<normalize_rows>);
+  m.impl("rope_table", on_device<rope_table>);
+  m.impl("csr_build", on_device<csr_build>);
+  m.impl("corner_csr", on_device<corner_csr>);
+  m.impl("segment_mass", on_device<segment_mass>);
+  m.impl("fastvggt_assemble", on_device<fastvggt_assemble>);
+  m.impl("fastvggt_match", on_device<fastvggt_match>);
+  m.impl("fastvggt_plan", on_device<fastvggt_plan>);
+  m.impl("similarity_topk", on_device<similarity_topk>);
+  m.impl("merged_block", on_device<merged_block>);
 }
 
 TORCH_LIBRARY_IMPL(vgo, Autograd, m) {

@@ -3,7 +3,7 @@
 Every `csrc/*.hip` file is compiled to an object under `_build/` and linked
 into one shared library next to this file.  The library exports only the
 `extern "C"` entry points declared in `include/vgo.h`.  `csrc/torch_ops.cpp`
-(host code: the torch operators' implementations) becomes `libvgo_torch.so`,
+(host code: the torch operators' implementations) becomes `libvgo_ops.so`,
 linked against it and torch.
 """
 from __future__ import annotations
@@ -18,7 +18,7 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC = PACKAGE_DIR / "csrc"
 BUILD_DIR = PACKAGE_DIR / "_build"
 LIBRARY = PACKAGE_DIR / "libvgo.so"
-OPS_LIBRARY = PACKAGE_DIR / "libvgo_torch.so"
+OPS_LIBRARY = PACKAGE_DIR / "libvgo_ops.so"
 OFFLOAD_ARCH = "gfx950"
 
 # Packed fp32 VALU forms are switched off for every device compile.

@@ -7,6 +7,7 @@ back to a CPU implementation: a missing library or a CPU tensor is an error.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -14,7 +15,7 @@ import torch
 
 PACKAGE_DIR = Path(__file__).resolve().parent
 LIBRARY_PATH = PACKAGE_DIR / "libvgo.so"
-OPS_LIBRARY_PATH = PACKAGE_DIR / "libvgo_torch.so"
+OPS_LIBRARY_PATH = PACKAGE_DIR / "libvgo_ops.so"
 
 VGO_OK = 0
 VGO_EINVAL = -1
@@ -163,24 +164,51 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 _ops_loaded = False
+_stubs: torch.library.Library | None = None
 
 
 class ExtensionUnavailable(RuntimeError):
     """Raised when the HIP library is missing or cannot be loaded."""
 
 
-def load_ops() -> bool:
-    """Load `libvgo_torch.so`, the implementations of torch.ops.vgo.*, once; False while it is
-    not built (the operators then have schemas but no kernels)."""
+def load_ops() -> None:
+    """Load `libvgo_ops.so`, the implementations of torch.ops.vgo.*, once."""
     global _ops_loaded
     with _lock:
-        if not _ops_loaded and OPS_LIBRARY_PATH.exists() and LIBRARY_PATH.exists():
-            try:
-                torch.ops.load_library(str(OPS_LIBRARY_PATH))
-            except OSError as error:
-                raise ExtensionUnavailable(f"vgo torch operators failed to load: {error}") from error
-            _ops_loaded = True
-        return _ops_loaded
+        if _ops_loaded:
+            return
+        missing = [path for path in (LIBRARY_PATH, OPS_LIBRARY_PATH) if not path.exists()]
+        if missing:
+            raise ExtensionUnavailable(f"vgo HIP extension is unavailable: {missing[0]} is not built "
+                                       "(run __graft_entry__.build())")
+        try:
+            register = ctypes.CDLL(str(OPS_LIBRARY_PATH)).vgo_torch_register
+        except (OSError, AttributeError) as error:
+            raise ExtensionUnavailable(f"vgo torch operators failed to load: {error} "
+                                       "(run __graft_entry__.build())") from error
+        register.restype = ctypes.c_char_p
+        wrong = register()
+        if wrong is not None:
+            raise ExtensionUnavailable("vgo torch operators were built for other operator schemas (run "
+                                       f"__graft_entry__.build()): {wrong.decode(errors='replace')}")
+        _ops_loaded = True
+
+
+def load_ops_or_stubs(names: list[str]) -> None:
+    """Load the operators' implementations; where that fails, give operator `names` ones that
+    raise what load() raises (or run, if the library has been built since)."""
+    global _stubs
+    try:
+        load_ops()
+    except ExtensionUnavailable:
+        _stubs = torch.library.Library("vgo", "IMPL")
+        for name in names:
+            _stubs.impl(name, functools.partial(_unloaded, name), "CUDA")
+
+
+def _unloaded(name: str, *args):
+    load()
+    return getattr(torch.ops.vgo, name)(*args)
 
 
 def load() -> ctypes.CDLL:
@@ -188,10 +216,7 @@ def load() -> ctypes.CDLL:
     global _lib
     if _lib is not None:
         return _lib
-    if not load_ops():
-        raise ExtensionUnavailable(
-            f"vgo HIP extension is unavailable: {LIBRARY_PATH} and {OPS_LIBRARY_PATH} are not built "
-            "(run __graft_entry__.build())")
+    load_ops()
     with _lock:
         if _lib is not None:
             return _lib

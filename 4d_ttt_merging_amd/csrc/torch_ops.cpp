@@ -20,7 +20,9 @@
 #include <torch/library.h>
 
 #include <array>
+#include <memory>
 #include <optional>
+#include <string>
 #include <vector>
 
 #include "../../include/vgo.h"
@@ -699,9 +701,7 @@ struct OnDevice<fn> {
 template <auto fn>
 constexpr auto on_device = &OnDevice<fn>::call;
 
-}  // namespace
-
-TORCH_LIBRARY_IMPL(vgo, CUDA, m) {
+void register_cuda(torch::Library& m) {
   m.impl("mass_bias_attention", on_device<mass_bias_attention>);
   m.impl("attention_into", on_device<attention_into>);
   m.impl("attention_pair_into", on_device<attention_pair_into>);
@@ -727,16 +727,43 @@ TORCH_LIBRARY_IMPL(vgo, CUDA, m) {
   m.impl("merged_block", on_device<merged_block>);
 }
 
-TORCH_LIBRARY_IMPL(vgo, Autograd, m) {
+void register_autograd(torch::Library& m) {
   for (const char* name : kPure) m.impl(name, torch::autograd::autogradNotImplementedFallback());
   for (const char* name : kMutating) m.impl(name, torch::autograd::autogradNotImplementedFallback());
 }
 
-TORCH_LIBRARY_IMPL(vgo, ADInplaceOrView, m) {
+void register_inplace(torch::Library& m) {
   for (const char* name : kMutating) m.impl(name, torch::autograd::autogradNotImplementedInplaceOrViewFallback());
 }
 
-TORCH_LIBRARY_IMPL(vgo, FuncTorchBatched, m) {
+void register_batched(torch::Library& m) {
   for (const char* name : kPure) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&no_batching>());
   for (const char* name : kMutating) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&no_batching>());
+}
+
+}  // namespace
+
+// Registers the implementations with the schemas that ops.py defined; null, or what is wrong (the
+// text stays valid), with nothing registered.  A call and not the initialisers of TORCH_LIBRARY_IMPL:
+// an exception there, as where the library was built for other schemas, ends the process that loads it.
+extern "C" __attribute__((visibility("default"))) const char* vgo_torch_register() {
+  static std::string message;
+  try {
+    std::vector<std::unique_ptr<torch::Library>> libraries;
+    const auto add = [&](c10::DispatchKey key, void (*fill)(torch::Library&)) {
+      libraries.push_back(std::make_unique<torch::Library>(torch::Library::IMPL, "vgo", key, __FILE__, __LINE__));
+      fill(*libraries.back());
+    };
+    add(c10::DispatchKey::CUDA, register_cuda);
+    add(c10::DispatchKey::Autograd, register_autograd);
+    add(c10::DispatchKey::ADInplaceOrView, register_inplace);
+    add(c10::DispatchKey::FuncTorchBatched, register_batched);
+    for (auto& library : libraries) (void)library.release();  // they last as long as the process
+    return nullptr;
+  } catch (const c10::Error& error) {
+    message = error.what_without_backtrace();
+  } catch (const std::exception& error) {
+    message = error.what();
+  }
+  return message.c_str();
 }

@@ -28,7 +28,7 @@ dispatcher, `torch.compile` and fake-tensor tracing see them as single ops:
   `segment_mass`).
 
 The CUDA (HIP) implementations are native (csrc/torch_ops.cpp, built into
-`libvgo_torch.so`) and call `libvgo.so` through its C ABI.  The operators a
+`libvgo_ops.so`) and call `libvgo.so` through its C ABI.  The operators a
 traced graph can hold have fake implementations that only describe their
 outputs; the block sequences, which tracing never takes, have none.  There is no
 CPU implementation: CPU tensors fail in the dispatcher.
@@ -103,10 +103,7 @@ _SCHEMAS = (
 _library = torch.library.Library("vgo", "DEF")
 for _schema in _SCHEMAS:
     _library.define(_schema, tags=(torch.Tag.pt2_compliant_tag,))
-try:
-    _lib.load_ops()
-except _lib.ExtensionUnavailable:  # a stale build: _lib.load() reports it on first use
-    pass
+_lib.load_ops_or_stubs([_schema.split("(")[0] for _schema in _SCHEMAS])
 
 
 def _fake(name):

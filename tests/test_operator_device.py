@@ -12,7 +12,7 @@ from tests.conftest import PACKAGE, ROOT, import_package
 def test_every_operator_sets_its_device():
     """Each registered implementation goes through the device guard, and each schema has one."""
     source = (ROOT / PACKAGE / "csrc" / "torch_ops.cpp").read_text()
-    block = re.search(r"TORCH_LIBRARY_IMPL\(vgo, CUDA, m\) \{(.*?)\n\}", source, re.S).group(1)
+    block = re.search(r"void register_cuda\(torch::Library& m\) \{(.*?)\n\}", source, re.S).group(1)
     implementations = re.findall(r'm\.impl\("(\w+)",\s*(.*?)\);', block)
     assert {f"on_device<{name}>" for name, _ in implementations} == {how for _, how in implementations}
     schemas = import_package("ops")._SCHEMAS

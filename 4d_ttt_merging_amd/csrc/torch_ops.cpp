@@ -671,14 +671,14 @@ constexpr const char* kPure[] = {"mass_bias_attention", "top4_project", "qkv_epi
                                  "restore_residual_layer_norm", "mlp_tail", "dense_block", "normalize_rows",
                                  "csr_build", "corner_csr", "segment_mass", "fastvggt_assemble", "fastvggt_match", "fastvggt_plan",
                                  "merged_block"};
-// sin and cos tables into out[0] and out[1] of a contiguous fp32 [2, h * w, head_dim].
-void rope_table(const Tensor& out, int64_t h, int64_t w, double base) {
-  require_gpu({&out});
-  TORCH_CHECK(out.dim() == 3 && out.size(0) == 2 && out.size(1) == h * w && out.scalar_type() == at::kFloat &&
-                  out.is_contiguous(),
-              "rope_table: out must be a contiguous float32 [2, h * w, head_dim]");
-  check(vgo_rope_table(h, w, out.size(2), static_cast<float>(base), ptr<float>(out), ptr<float>(out) + out.stride(0),
-                       stream_of(out)));
+// sin and cos tables into two contiguous fp32 [h * w, head_dim].
+void rope_table(const Tensor& sin, const Tensor& cos, int64_t h, int64_t w, double base) {
+  require_gpu({&sin, &cos});
+  for (const Tensor* t : {&sin, &cos})
+    TORCH_CHECK(t->dim() == 2 && t->size(0) == h * w && t->sizes() == sin.sizes() && t->device() == sin.device() &&
+                    t->scalar_type() == at::kFloat && t->is_contiguous(),
+                "rope_table: sin and cos must be contiguous float32 [h * w, head_dim]");
+  check(vgo_rope_table(h, w, sin.size(1), static_cast<float>(base), ptr<float>(sin), ptr<float>(cos), stream_of(sin)));
 }
 
 constexpr const char* kMutating[] = {"attention_into", "attention_pair_into", "top4_project_into",

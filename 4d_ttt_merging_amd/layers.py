@@ -743,11 +743,12 @@ def init_weights_vit(module: nn.Module, name: str = "") -> None:
 
 
 def _one_launch_rope(H, W, head_dim, base, device) -> bool:
-    """Plain sizes on a GPU, outside tracing, dispatch modes and function transforms (which see torch's
-    operators)."""
+    """Plain sizes that the kernel takes on a GPU, outside tracing, dispatch modes and function transforms
+    (which see torch's operators)."""
     return (device is not None and torch.device(device).type == "cuda"
             and type(H) is int and type(W) is int and type(head_dim) is int and type(base) in (int, float)
-            and H > 0 and W > 0 and head_dim >= 4 and head_dim % 4 == 0 and base > 1
+            and 0 < H < 1 << 20 and 0 < W < 1 << 20 and head_dim >= 4 and head_dim % 4 == 0 and base > 1
+            and H * W * head_dim < 1 << 31
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None)
@@ -758,9 +759,8 @@ def rope_sincos(H: int, W: int, head_dim: int, base: float = 100.0,
     """Axial RoPE tables of RopePositionEmbedding(normalize_coords="max") at inference
     (vggt_omega/models/layers/rope_position_encoding.py:51-127), fp32 [H*W, head_dim]."""
     if _one_launch_rope(H, W, head_dim, base, device):
-        out = torch.empty((2, H * W, head_dim), device=device, dtype=torch.float32)
-        torch.ops.vgo.rope_table(out, H, W, base)
-        sin, cos = out.unbind()
+        sin, cos = (torch.empty((H * W, head_dim), device=device, dtype=torch.float32) for _ in range(2))
+        torch.ops.vgo.rope_table(sin, cos, H, W, base)
         return sin, cos
     dd = dict(device=device, dtype=torch.float32)
     periods = base ** (2 * torch.arange(head_dim // 4, **dd) / (head_dim // 2))

@@ -89,7 +89,7 @@ _SCHEMAS = (
     "Tensor(c!)? scores) -> ()",
     "fastvggt_match(Tensor tokens, Tensor sources, Tensor destinations, bool prenormalized) -> (Tensor, Tensor)",
     "normalize_rows(Tensor x, Tensor? rows, float eps, ScalarType out_dtype) -> Tensor",
-    "rope_table(Tensor(a!) out, int h, int w, float base) -> ()",
+    "rope_table(Tensor(a!) sin, Tensor(b!) cos, int h, int w, float base) -> ()",
     "csr_build(Tensor keys, int n_buckets) -> (Tensor, Tensor)",
     "corner_csr(Tensor parent, int n_dest) -> (Tensor, Tensor)",
     "segment_mass(Tensor offsets, int segs_per_row, Tensor order, Tensor? weights, int rows, float start, "

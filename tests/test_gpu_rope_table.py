@@ -49,3 +49,27 @@ def test_transforms_and_devices_take_torch_operators(vgo, device):
     x = torch.randn(5, 12, 8, device=device)
     out = torch.func.vmap(lambda v: v * layers.rope_sincos(3, 4, 8, device=device)[0])(x)
     assert torch.equal(out, x * layers.rope_sincos(3, 4, 8, device=device)[0])
+
+
+def test_sizes_past_the_kernel_take_torch_operators(vgo, device):
+    """The kernel's limits: 2^20 rows or columns of patches, 2^31 values."""
+    layers = import_package("layers")
+    for h, w, dim in ((1 << 20, 1, 4), (1, 1 << 20, 4), (1 << 10, 1 << 11, 1024)):
+        assert not layers._one_launch_rope(h, w, dim, 100.0, device)
+        assert layers._one_launch_rope(h - (h > 1), w - (w > 1), dim, 100.0, device)
+    sin, cos = layers.rope_sincos(1 << 20, 1, 4, device=device)
+    with _TorchOnly():
+        expect = layers.rope_sincos(1 << 20, 1, 4, device=device)
+    assert torch.equal(sin, expect[0]) and torch.equal(cos, expect[1])
+
+
+def test_tables_are_tensors_of_their_own(vgo, device):
+    """Each may be written in place, under autograd too, without a trace in the other."""
+    layers = import_package("layers")
+    sin, cos = layers.rope_sincos(3, 4, 8, device=device)
+    expect, version = sin.clone(), cos._version
+    assert not sin._is_view() and sin.untyped_storage().data_ptr() != cos.untyped_storage().data_ptr()
+    scale = torch.full((8,), 2.0, device=device, requires_grad=True)
+    sin.mul_(scale)
+    sin.sum().backward()
+    assert torch.equal(sin.detach(), 2 * expect) and torch.equal(scale.grad, expect.sum(0)) and cos._version == version

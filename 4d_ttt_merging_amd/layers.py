@@ -586,6 +586,12 @@ class SelfAttentionBlock(nn.Module):
             return None
         return _cast_linears(mlp.fc1, mlp.fc2)
 
+    def _replaces_steps(self) -> bool:
+        """The block's class or the block itself replaces a step that a native sequence passes by."""
+        own = type(self)
+        return not _STEPS.isdisjoint(self.__dict__) or (own is not SelfAttentionBlock and any(
+            getattr(own, name) is not getattr(SelfAttentionBlock, name) for name in _STEPS))
+
     def _native_parameters(self, x: Tensor) -> tuple | None:
         """(norms, eps, linears, gammas, heads) of torch.ops.vgo.dense_block and merged_block
         for an x [B, N, C], or None."""
@@ -617,7 +623,7 @@ class SelfAttentionBlock(nn.Module):
 
     def _native_dense(self, x: Tensor, rope) -> tuple | None:
         """The arguments of torch.ops.vgo.dense_block after x, or None."""
-        if not _plain_call(x):
+        if not _plain_call(x) or self._replaces_steps():
             return None
         sin = cos = None
         if rope is not None:
@@ -630,7 +636,7 @@ class SelfAttentionBlock(nn.Module):
     def _native_merged(self, x: Tensor, plan, normalized: Tensor | None) -> tuple | None:
         """The arguments of torch.ops.vgo.merged_block after x, or None: one batch element and a
         plain TokenPlan that pools and removes tokens."""
-        if not _plain_call(x):
+        if not _plain_call(x) or self._replaces_steps():
             return None
         dtype = _autocast_dtype()
         if (type(plan) is not TokenPlan or x.ndim != 3 or x.shape[0] != 1 or self.attn.training
@@ -661,7 +667,9 @@ class SelfAttentionBlock(nn.Module):
         return self._mlp_tail(x_attn, h)
 
 
-# Methods whose replacement on an instance a native sequence would pass by.
+# Steps of a block that a native sequence passes by.
+_STEPS = frozenset(("_norm1_input", "_fused_tail", "_fused_restore_tail", "_mlp_tail"))
+# Methods of its modules whose replacement on an instance a native sequence would pass by.
 _METHODS = frozenset(("forward", "compute_attention", "_forward_merged", "_merged_fused", "_dense_fused", "_attend",
                       "_attention_dtype", "_fusable", "_norm_params", "_bias", "_cast_params", "_cast_sources"))
 
@@ -673,10 +681,13 @@ def _plain(module: nn.Module, *types: type) -> bool:
             and _METHODS.isdisjoint(module.__dict__))
 
 
+_TENSORS = (Tensor, nn.Parameter)
+
+
 def _plain_call(x: Tensor) -> bool:
     """Nothing observes the calls a block makes: no tracing, dispatch or function mode, tensor
     subclass, global module hook or profiling span."""
-    return (type(x) in (Tensor, nn.Parameter) and not torch.compiler.is_compiling() and not profiling.enabled()
+    return (type(x) in _TENSORS and not torch.compiler.is_compiling() and not profiling.enabled()
             and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and not nn.modules.module._has_any_global_hook())
 
@@ -700,7 +711,7 @@ def _cast_linears(*linears: nn.Module) -> tuple | None:
 
 def _vector_rows(rows: Tensor) -> bool:
     """Rows the one-launch compaction takes (16-byte chunks); one output at a time takes any."""
-    return (not torch.compiler.is_compiling() and type(rows) in (Tensor, nn.Parameter)
+    return (not torch.compiler.is_compiling() and type(rows) in _TENSORS
             and rows.stride(0) % 8 == 0 and rows.data_ptr() % 16 == 0)
 
 

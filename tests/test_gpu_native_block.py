@@ -117,6 +117,40 @@ def test_replaced_modules_run_call_by_call(vgo, device):
         assert block._native_dense(x, None) is None and not torch.equal(block(x), ref)
 
 
+@pytest.mark.parametrize("where", ["class", "instance"])
+def test_replaced_steps_of_a_block_are_called(vgo, device, where):
+    """A block whose own steps are replaced, by a subclass or on the object, calls them."""
+    seen = []
+
+    def replaced(name):
+        def step(self, *args):
+            seen.append(name)
+            return getattr(vgo.SelfAttentionBlock, name)(self, *args)
+        return step
+
+    block = _block(vgo, 128, 2, device, use_qk_norm=True, init_values=0.5)
+    x = torch.randn(1, 90, 128, device=device)
+    plan = vgo.TokenPlan(torch.arange(41, device=device)[None], (torch.arange(90, device=device) % 41)[None], 90)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        dense, merged = block(x), block.forward_compacted(x, plan)
+        assert block._native_dense(x, None) is not None
+        for name, called_by in (("_norm1_input", "both"), ("_fused_tail", "dense"), ("_fused_restore_tail", "merged"),
+                                ("_mlp_tail", "both")):
+            if where == "class":
+                block.__class__ = type("Changed", (vgo.SelfAttentionBlock,), {name: replaced(name)})
+            else:
+                block.__dict__[name] = replaced(name).__get__(block)
+            for route, call, expect in (("dense", lambda: block(x), dense),
+                                        ("merged", lambda: block.forward_compacted(x, plan), merged)):
+                seen.clear()
+                assert torch.equal(call(), expect)
+                assert seen == ([name] if called_by in (route, "both") else []), (name, route)
+            block.__class__ = vgo.SelfAttentionBlock
+            block.__dict__.pop(name, None)
+        block.__class__ = type("Same", (vgo.SelfAttentionBlock,), {})  # a subclass that replaces no step
+        assert block._native_dense(x, None) is not None
+
+
 def test_operators_refuse_backward_and_vmap(vgo, device):
     table = torch.randn(8, 16, device=device, requires_grad=True)
     index = torch.zeros(5, 4, dtype=torch.int32, device=device)

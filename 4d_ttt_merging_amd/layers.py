@@ -700,7 +700,8 @@ def _cast_linears(*linears: nn.Module) -> tuple | None:
         return None
     cast = []
     for linear in linears:
-        if not _plain(linear, Linear, LinearKMaskedBias) or not linear.weight.is_cuda:
+        if not (_plain(linear, Linear, LinearKMaskedBias) and linear.weight.is_cuda
+                and type(linear.weight) in _TENSORS and (linear.bias is None or type(linear.bias) in _TENSORS)):
             return None
         pair = linear._cast_params(dtype)
         if pair is None:

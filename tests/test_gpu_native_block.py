@@ -151,6 +151,33 @@ def test_replaced_steps_of_a_block_are_called(vgo, device, where):
         assert block._native_dense(x, None) is not None
 
 
+@pytest.mark.parametrize("linear", ["attn.qkv", "attn.proj", "mlp.fc1", "mlp.fc2"])
+@pytest.mark.parametrize("parameter", ["weight", "bias"])
+def test_tensor_subclasses_as_weights_see_the_product(vgo, device, linear, parameter):
+    """A weight of a tensor subclass answers the linear call itself (as quantised weights do)."""
+    products = []
+
+    class Watched(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            if func is torch.nn.functional.linear:
+                products.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    block = _block(vgo, 128, 2, device, use_qk_norm=True, init_values=0.5)
+    module = block.get_submodule(linear)
+    x = torch.randn(1, 90, 128, device=device)
+    plan = vgo.TokenPlan(torch.arange(41, device=device)[None], (torch.arange(90, device=device) % 41)[None], 90)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        dense, merged = block(x), block.forward_compacted(x, plan)
+        watched = getattr(module, parameter).detach().clone().as_subclass(Watched)
+        setattr(module, parameter, torch.nn.Parameter(watched, requires_grad=False))
+        for call, expect in ((lambda: block(x), dense), (lambda: block.forward_compacted(x, plan), merged)):
+            products.clear()
+            out = call()
+            assert products and torch.equal(out.as_subclass(torch.Tensor), expect)
+
+
 def test_operators_refuse_backward_and_vmap(vgo, device):
     table = torch.randn(8, 16, device=device, requires_grad=True)
     index = torch.zeros(5, 4, dtype=torch.int32, device=device)

@@ -22,6 +22,7 @@ def _c(ptr_or_tensor):
 def normalize_rows(x: torch.Tensor, rows: torch.Tensor | None, eps: float,
                    out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """out[r] = x[rows[r]] / max(||x[rows[r]]||, eps) for a 2-D x (unit column stride)."""
+    _lib.require_plain(x, rows)
     return torch.ops.vgo.normalize_rows(x, rows, float(eps), out_dtype)
 
 
@@ -42,6 +43,7 @@ def similarity_topk(src: torch.Tensor, dictionary: torch.Tensor, topk: int, *,
     """
     _lib.load()
     _lib.require_gpu(src, dictionary, src_rows, n_src_device, index_map, scores)
+    _lib.require_plain(src, dictionary, src_rows, n_src_device, index_map, scores)
     if src.dtype != torch.bfloat16 or dictionary.dtype != torch.bfloat16:
         raise ValueError("similarity_topk expects bf16 operands")
     if dict_ranges is None:
@@ -63,11 +65,13 @@ def similarity_topk(src: torch.Tensor, dictionary: torch.Tensor, topk: int, *,
 
 def csr_build(keys: torch.Tensor, n_buckets: int) -> tuple[torch.Tensor, torch.Tensor]:
     """Stable bucket order: (order [n] int32 item ids, offsets [n_buckets+1] int32)."""
+    _lib.require_plain(keys)
     return torch.ops.vgo.csr_build(keys, n_buckets)
 
 
 def corner_csr(parent: torch.Tensor, n_dest: int) -> tuple[torch.Tensor, torch.Tensor]:
     """csr_build of the (destination, corner) pairs: item p = i*S + c, key = parent*S + c of [M, S] parents."""
+    _lib.require_plain(parent)
     return torch.ops.vgo.corner_csr(parent, n_dest)
 
 
@@ -75,6 +79,7 @@ def segment_mass(offsets: torch.Tensor, segs_per_row: int, order: torch.Tensor,
                  weights: torch.Tensor | None, rows: int, start: float,
                  want_log: bool = True) -> tuple[torch.Tensor, torch.Tensor | None]:
     """Sequential per-segment sums from `start` (fp32 [rows]) and, if asked, their logarithms."""
+    _lib.require_plain(offsets, order, weights)
     mass, log_mass = torch.ops.vgo.segment_mass(offsets, segs_per_row, order, weights, rows, float(start),
                                                 want_log)
     return mass, log_mass if want_log else None

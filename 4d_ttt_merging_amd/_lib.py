@@ -252,6 +252,14 @@ def require_gpu(*tensors: torch.Tensor) -> None:
             raise RuntimeError("vgo kernels run on the GPU only; got a CPU tensor")
 
 
+def require_plain(*tensors: torch.Tensor) -> None:
+    """The planners' operators leave no trace in autograd, so a function transform (vmap, grad, jvp)
+    over one would silently lose its derivative."""
+    for tensor in tensors:
+        if tensor is not None and torch._C._functorch.is_functorch_wrapped_tensor(tensor):
+            raise RuntimeError("vgo planners take no tensors of function transforms (vmap, grad, jvp)")
+
+
 def stream_of(tensor: torch.Tensor) -> int:
     """hipStream_t of torch's current stream on the tensor's device."""
     return torch.cuda.current_stream(tensor.device).cuda_stream

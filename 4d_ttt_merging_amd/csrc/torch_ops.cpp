@@ -9,14 +9,18 @@
 // Every implementation checks shapes and types, allocates outputs and
 // workspaces with torch, and launches on torch's current stream of the
 // tensors' device, which is the current device meanwhile (`on_device`); none
-// synchronises.  Autograd: outputs of inputs that
-// require grad have a backward that raises (the path is inference only), and
+// synchronises.  Autograd: outputs of a path operator whose inputs
+// require grad have a backward that raises (the path is inference only), those
+// of a planner's operator do not require grad, and tangents are dropped;
 // operators have no batching rule (vmap raises).
 #include <ATen/ATen.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
-#include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/variable.h>
 #include <torch/library.h>
 
 #include <array>
@@ -662,15 +666,6 @@ Tensor merged_block(const Tensor& x, const OptTensor& h0, const OptTensor& qkv0,
   return mlp_tail(rows[0], rows[1], *linears.get(4), linears.get(5), *linears.get(6), linears.get(7), gammas.get(1));
 }
 
-// vmap over an operator: refused, as no operator has a batching rule.
-void no_batching(const c10::OperatorHandle& op, c10::DispatchKeySet, torch::jit::Stack*) {
-  TORCH_CHECK(false, op.operator_name().name, " has no batching rule (vmap)");
-}
-
-constexpr const char* kPure[] = {"mass_bias_attention", "top4_project", "qkv_epilogue", "residual_layer_norm",
-                                 "restore_residual_layer_norm", "mlp_tail", "dense_block", "normalize_rows",
-                                 "csr_build", "corner_csr", "segment_mass", "fastvggt_assemble", "fastvggt_match", "fastvggt_plan",
-                                 "merged_block"};
 // sin and cos tables into two contiguous fp32 [h * w, head_dim].
 void rope_table(const Tensor& sin, const Tensor& cos, int64_t h, int64_t w, double base) {
   require_gpu({&sin, &cos});
@@ -681,9 +676,76 @@ void rope_table(const Tensor& sin, const Tensor& cos, int64_t h, int64_t w, doub
   check(vgo_rope_table(h, w, sin.size(1), static_cast<float>(base), ptr<float>(sin), ptr<float>(cos), stream_of(sin)));
 }
 
-constexpr const char* kMutating[] = {"attention_into", "attention_pair_into", "top4_project_into",
-                                     "top4_project_ordered_into", "compact_into", "compact_multi_into", "similarity_topk",
-                                     "rope_table"};
+// Operators by what autograd makes of them.  Path: gradient-free, but part of a recorded graph, whose
+// backward raises; a tensor's tangents end there.  Plan: read their inputs' values alone, as a plan does.
+constexpr const char* kPath[] = {"mass_bias_attention", "top4_project", "qkv_epilogue", "residual_layer_norm",
+                                 "restore_residual_layer_norm", "mlp_tail", "dense_block", "merged_block"};
+constexpr const char* kPathInto[] = {"attention_into", "attention_pair_into", "top4_project_into",
+                                     "top4_project_ordered_into", "compact_into", "compact_multi_into"};
+constexpr const char* kPlan[] = {"normalize_rows", "csr_build", "corner_csr", "segment_mass", "fastvggt_assemble",
+                                 "fastvggt_match", "fastvggt_plan"};
+constexpr const char* kPlanInto[] = {"similarity_topk", "rope_table"};
+
+template <typename Visit>
+void each_tensor(const c10::IValue& value, Visit visit) {
+  if (value.isTensor()) {
+    if (value.toTensor().defined()) visit(value.toTensor());
+  } else if (value.isList()) {
+    for (const c10::IValue& item : value.toListRef()) each_tensor(item, visit);
+  }
+}
+
+// Autograd key.  History: where an input requires grad (and grad mode is on) floating outputs do too,
+// with a backward that raises; written tensors are left as they are.
+template <bool kHistory>
+void autograd(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torch::jit::Stack* stack) {
+  const size_t arguments = op.schema().arguments().size(), returns = op.schema().returns().size();
+  torch::autograd::edge_list inputs;
+  if constexpr (kHistory) {
+    if (at::GradMode::is_enabled()) {
+      bool tangent = false;
+      for (const c10::IValue& value : torch::jit::last(*stack, arguments))
+        each_tensor(value, [&](const Tensor& t) {
+          if (t.requires_grad()) inputs.push_back(torch::autograd::impl::gradient_edge(t));
+          tangent |= t._fw_grad(/*level=*/0).defined();
+        });
+      TORCH_CHECK_NOT_IMPLEMENTED(inputs.empty() || !tangent, op.operator_name().name,
+                                  " has no derivative: tensors that require grad cannot carry tangents through it");
+    }
+  }
+  {
+    const at::AutoDispatchBelowAutograd below;
+    op.redispatchBoxed(keys & c10::after_autograd_keyset, stack);
+  }
+  if (inputs.empty()) return;
+  const std::shared_ptr<torch::autograd::Node> node(
+      new torch::autograd::NotImplemented(op.operator_name().name, std::move(inputs)), torch::autograd::deleteNode);
+  for (const c10::IValue& value : torch::jit::last(*stack, returns))
+    each_tensor(value, [&](const Tensor& t) {
+      if (torch::autograd::isDifferentiableType(t.scalar_type())) torch::autograd::set_history(t, node);
+    });
+}
+
+// ADInplaceOrView key of operators that write arguments: their versions count the write.
+void written(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torch::jit::Stack* stack) {
+  std::vector<Tensor> outputs;
+  const auto& arguments = op.schema().arguments();
+  const auto values = torch::jit::last(*stack, arguments.size());
+  for (size_t i = 0; i < arguments.size(); ++i)
+    if (arguments[i].alias_info() != nullptr && arguments[i].alias_info()->isWrite())
+      each_tensor(values[i], [&](const Tensor& t) { outputs.push_back(t); });
+  {
+    const at::AutoDispatchBelowADInplaceOrView below;
+    op.redispatchBoxed(keys & c10::after_ADInplaceOrView_keyset, stack);
+  }
+  for (const Tensor& t : outputs)
+    if (!t.is_inference()) torch::autograd::impl::bump_version(t);
+}
+
+// vmap over an operator: refused, as no operator has a batching rule.
+void no_batching(const c10::OperatorHandle& op, c10::DispatchKeySet, torch::jit::Stack*) {
+  TORCH_CHECK(false, op.operator_name().name, " has no batching rule (vmap)");
+}
 
 // `fn` with its first argument's device as the current device.  The kernels' launches, the device
 // properties that size them and static scratch all go by the current device, and torch's default
@@ -728,17 +790,22 @@ void register_cuda(torch::Library& m) {
 }
 
 void register_autograd(torch::Library& m) {
-  for (const char* name : kPure) m.impl(name, torch::autograd::autogradNotImplementedFallback());
-  for (const char* name : kMutating) m.impl(name, torch::autograd::autogradNotImplementedFallback());
+  for (const char* name : kPath) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<true>>());
+  for (const char* name : kPathInto) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<true>>());
+  for (const char* name : kPlan) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<false>>());
+  for (const char* name : kPlanInto) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<false>>());
 }
 
 void register_inplace(torch::Library& m) {
-  for (const char* name : kMutating) m.impl(name, torch::autograd::autogradNotImplementedInplaceOrViewFallback());
+  for (const char* name : kPathInto) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&written>());
+  for (const char* name : kPlanInto) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&written>());
 }
 
 void register_batched(torch::Library& m) {
-  for (const char* name : kPure) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&no_batching>());
-  for (const char* name : kMutating) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&no_batching>());
+  const auto refuse = [&](const auto& names) {
+    for (const char* name : names) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&no_batching>());
+  };
+  refuse(kPath), refuse(kPathInto), refuse(kPlan), refuse(kPlanInto);
 }
 
 }  // namespace

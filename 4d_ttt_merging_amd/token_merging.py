@@ -578,6 +578,7 @@ def build_fastvggt_plan(
 
     if prenormalized and tokens.dtype != torch.bfloat16:
         raise ValueError("prenormalized FastVGGT tokens must be bf16 unit rows")
+    _kernels._lib.require_plain(tokens)
     best, target = torch.ops.vgo.fastvggt_match(tokens, sources, destinations, prenormalized)
     if after_match is not None:
         after_match()

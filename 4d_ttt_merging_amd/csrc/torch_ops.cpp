@@ -11,8 +11,8 @@
 // tensors' device, which is the current device meanwhile (`on_device`); none
 // synchronises.  Autograd: outputs of a path operator whose inputs
 // require grad have a backward that raises (the path is inference only), those
-// of a planner's operator do not require grad, and tangents are dropped;
-// operators have no batching rule (vmap raises).
+// of a planner's operator do not require grad, and tangents are dropped.
+// No operator has a batching rule (see register_batched).
 #include <ATen/ATen.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
@@ -678,8 +678,10 @@ void rope_table(const Tensor& sin, const Tensor& cos, int64_t h, int64_t w, doub
 
 // Operators by what autograd makes of them.  Path: gradient-free, but part of a recorded graph, whose
 // backward raises; a tensor's tangents end there.  Plan: read their inputs' values alone, as a plan does.
+// Blocks: likewise, whole sequences of launches that only plain tensors reach.
 constexpr const char* kPath[] = {"mass_bias_attention", "top4_project", "qkv_epilogue", "residual_layer_norm",
-                                 "restore_residual_layer_norm", "mlp_tail", "dense_block", "merged_block"};
+                                 "restore_residual_layer_norm"};
+constexpr const char* kBlocks[] = {"mlp_tail", "dense_block", "merged_block"};
 constexpr const char* kPathInto[] = {"attention_into", "attention_pair_into", "top4_project_into",
                                      "top4_project_ordered_into", "compact_into", "compact_multi_into"};
 constexpr const char* kPlan[] = {"normalize_rows", "csr_build", "corner_csr", "segment_mass", "fastvggt_assemble",
@@ -742,7 +744,8 @@ void written(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torch::jit
     if (!t.is_inference()) torch::autograd::impl::bump_version(t);
 }
 
-// vmap over an operator: refused, as no operator has a batching rule.
+// vmap over a planner's or a block's operator: refused.  The path's operators take torch's fallback,
+// which runs one call per batch element where the results are new tensors.
 void no_batching(const c10::OperatorHandle& op, c10::DispatchKeySet, torch::jit::Stack*) {
   TORCH_CHECK(false, op.operator_name().name, " has no batching rule (vmap)");
 }
@@ -792,6 +795,7 @@ void register_cuda(torch::Library& m) {
 void register_autograd(torch::Library& m) {
   for (const char* name : kPath) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<true>>());
   for (const char* name : kPathInto) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<true>>());
+  for (const char* name : kBlocks) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<true>>());
   for (const char* name : kPlan) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<false>>());
   for (const char* name : kPlanInto) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&autograd<false>>());
 }
@@ -805,7 +809,7 @@ void register_batched(torch::Library& m) {
   const auto refuse = [&](const auto& names) {
     for (const char* name : names) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&no_batching>());
   };
-  refuse(kPath), refuse(kPathInto), refuse(kPlan), refuse(kPlanInto);
+  refuse(kBlocks), refuse(kPlan), refuse(kPlanInto);
 }
 
 }  // namespace

@@ -178,12 +178,10 @@ def test_tensor_subclasses_as_weights_see_the_product(vgo, device, linear, param
             assert products and torch.equal(out.as_subclass(torch.Tensor), expect)
 
 
-def test_operators_refuse_backward_and_vmap(vgo, device):
+def test_operators_refuse_backward(vgo, device):
     table = torch.randn(8, 16, device=device, requires_grad=True)
     index = torch.zeros(5, 4, dtype=torch.int32, device=device)
     weight = torch.rand(5, 4, device=device)
     out = vgo.top4_project(table, index, weight)
     with pytest.raises(RuntimeError):
         out.sum().backward()
-    with pytest.raises(RuntimeError):
-        torch.func.vmap(lambda t: torch.ops.vgo.top4_project(t, index, weight))(torch.randn(2, 8, 16, device=device))

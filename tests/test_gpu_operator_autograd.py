@@ -102,3 +102,25 @@ def test_outputs_written_in_place(vgo, device):
         vgo.top4_project(table, index, w, out=out)
         assert torch.equal(out, expect) and out.grad_fn is None
         assert before is None or out._version > before
+
+
+def test_vmap_runs_one_call_per_element(vgo, device):
+    """Operators with new tensors as results run under vmap; those that write arguments, planners and blocks refuse."""
+    g = torch.Generator(device=device).manual_seed(8)
+    q, k, v = (torch.randn(3, 1, 2, 50, 64, device=device, generator=g) for _ in range(3))
+    mass, table = torch.randn(50, device=device, generator=g), torch.randn(3, 20, C, device=device, generator=g)
+    index = torch.randint(0, 20, (30, 4), dtype=torch.int32, device=device, generator=g)
+    w = torch.rand(30, 4, device=device, generator=g)
+    got = torch.func.vmap(lambda a, b, c: vgo.mass_bias_attention(a, b, c, mass))(q, k, v)
+    assert torch.equal(got, torch.stack([vgo.mass_bias_attention(*t, mass) for t in zip(q, k, v)]))
+    got = torch.func.vmap(lambda t: vgo.top4_project(t, index, w), in_dims=0, out_dims=1)(table)
+    assert torch.equal(got, torch.stack([vgo.top4_project(t, index, w) for t in table], dim=1))
+    none = [None] * 8
+    for refused in (lambda t: vgo.top4_project(t, index, w, out=torch.empty(30, C, device=device)),
+                    lambda t: torch.ops.vgo.residual_layer_norm(t, None, None, None, None, 1e-5, True, True,
+                                                                torch.bfloat16, False, -1.0)[1],
+                    lambda t: torch.ops.vgo.normalize_rows(t, None, 1e-12, torch.bfloat16),
+                    lambda t: torch.ops.vgo.dense_block(t[None], none, [1e-5] * 3, none, none[:2], 2, None, None,
+                                                        torch.bfloat16)):
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(refused)(table)

@@ -91,6 +91,13 @@ def restore_map(total: int, *, device: torch.device, keep: torch.Tensor | None =
                 inverse: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """Dense [total, 4] (int32 index, fp32 weight) rows consumed by top4_project."""
     lib = _lib.load()
+    _lib.require_gpu(keep, source, parent, weight, inverse)
+    n_keep = 0 if keep is None else keep.numel()
+    n_source = 0 if source is None else source.numel()
+    if inverse is not None and inverse.numel() < total:
+        raise ValueError(f"restore_map: {inverse.numel()} inverse entries for {total} tokens")
+    if n_source and (parent is None or weight is None or min(parent.numel(), weight.numel()) < 4 * n_source):
+        raise ValueError("restore_map: four parents and weights per source")
     # With `inverse` the kernel writes every row; otherwise rows outside keep and
     # source stay zero (zero weights, as the reference's `new_zeros` output).
     if inverse is not None:
@@ -99,8 +106,6 @@ def restore_map(total: int, *, device: torch.device, keep: torch.Tensor | None =
     else:  # one fill for both
         index_out, weight_out = torch.zeros((2, total, 4), device=device, dtype=torch.int32).unbind()
         weight_out = weight_out.view(torch.float32)
-    n_keep = 0 if keep is None else keep.numel()
-    n_source = 0 if source is None else source.numel()
     status = lib.vgo_restore_map(
         _c(keep), n_keep, _c(source), _c(parent), _c(weight), n_source, _c(inverse), total,
         index_out.data_ptr(), weight_out.data_ptr(), torch.cuda.current_stream(device).cuda_stream)

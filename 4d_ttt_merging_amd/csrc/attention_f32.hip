@@ -57,9 +57,11 @@ struct Args {
   float* out;
   int heads, nq, nk, n_qblocks, ntiles;
   int64_t qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn;
-  int64_t units;   // (task, key tile) units, split evenly over `groups` work-groups
-  int groups;
-  float* partial;  // two states per work-group (null: groups = tasks, nothing is cut)
+  // Split evenly over `groups` work-groups: the (task, key tile) units or, without partial states,
+  // whole tasks.
+  int64_t units;
+  int tasks, groups;
+  float* partial;  // two states per work-group
 };
 
 // LDS position of element d of K row `row`: 16-byte chunks XOR-permuted by row & 15.
@@ -288,8 +290,9 @@ __global__ __launch_bounds__(kWaves * 64, kGroupsPerCu) void attn_f32_kernel(con
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t u0 = sk_begin(w, a.units, a.groups);
-  const int64_t u1 = sk_begin(w + 1, a.units, a.groups);
+  const bool cut = a.partial != nullptr;
+  const int64_t u0 = cut ? sk_begin(w, a.units, a.groups) : sk_begin(w, a.tasks, a.groups) * a.ntiles;
+  const int64_t u1 = cut ? sk_begin(w + 1, a.units, a.groups) : sk_begin(w + 1, a.tasks, a.groups) * a.ntiles;
   for (int64_t u = u0; u < u1;) {
     const int task = static_cast<int>(u / a.ntiles);
     const int t0 = static_cast<int>(u - static_cast<int64_t>(task) * a.ntiles);
@@ -365,11 +368,19 @@ __global__ __launch_bounds__(256) void attn_f32_merge_kernel(const Args a) {
 int64_t tasks_of(const Problem& p) { return (p.nq + kQTask - 1) / kQTask * p.batch * p.heads; }
 int64_t tiles_of(const Problem& p) { return (p.nk + kKeys - 1) / kKeys; }
 
+// Tasks past this many rounds of the resident work-groups are not cut: the last round is then
+// 1/64 of the time at most, and the merge would run 16 blocks for every task to find the few.
+constexpr int64_t kMaxSplitRounds = 64;
+// Work-groups of a launch without splitting.  A grid holds 2^32 threads; the tasks past that are
+// second ones of a work-group.
+constexpr int64_t kMaxGroups = int64_t{1} << 23;
+
 // Work-groups over which the (task, key tile) units are split: two per CU, with
 // at least kMinUnits tiles each.  0: not split, because the tasks already divide
-// evenly over the resident work-groups, or are more than the pieces.
+// evenly over the resident work-groups, are more than the pieces, or are very many.
 int64_t split_groups(const Problem& p) {
   const int64_t tasks = tasks_of(p), slots = int64_t{device_cus()} * kGroupsPerCu;
+  if (tasks > kMaxSplitRounds * slots) return 0;
   const int64_t groups = std::min<int64_t>(slots, tasks * tiles_of(p) / kMinUnits);
   return groups > tasks || (groups == slots && tasks % groups != 0) ? groups : 0;
 }
@@ -393,7 +404,7 @@ size_t attn_f32_workspace(const Problem& p) {
 
 int launch_attn_f32(const Problem& p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   const int64_t tasks = tasks_of(p);
-  VGO_REQUIRE(tasks <= 0x7fffffff / (kQTask / kMergeRows), "mass_bias_attention: grid too large");
+  VGO_REQUIRE(tasks <= 0x7fffffff, "mass_bias_attention: grid too large");
   Args a;
   a.q = static_cast<const float*>(p.q);
   a.k = static_cast<const float*>(p.k);
@@ -410,7 +421,8 @@ int launch_attn_f32(const Problem& p, void* workspace, size_t workspace_bytes, h
   a.vsb = p.vs[0], a.vsh = p.vs[1], a.vsn = p.vs[2];
   a.osb = p.os[0], a.osh = p.os[1], a.osn = p.os[2];
   a.units = tasks * a.ntiles;
-  a.groups = static_cast<int>(tasks);
+  a.tasks = static_cast<int>(tasks);
+  a.groups = static_cast<int>(std::min(tasks, kMaxGroups));
   a.partial = nullptr;
   const bool split = workspace != nullptr && workspace_bytes > 0 && workspace_bytes >= attn_f32_workspace(p);
   if (split) {

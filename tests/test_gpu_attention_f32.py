@@ -59,6 +59,28 @@ def test_tile_edges(vgo, device, layout, nq, nk):
             assert_close(out.cpu(), ref, torch.float32, what=f"{layout} split={split} bias={b is not None}")
 
 
+@pytest.mark.parametrize("split", [None, False])
+@pytest.mark.parametrize("batch", [16_400, 70_000, (1 << 20) + 3])
+def test_many_small_problems(vgo, device, batch, split):
+    """Tasks past those that are cut, past the merge's grid, and past a grid of one task per work-group.
+
+    With one key the result is its value, in whatever order it is computed."""
+    mba = __import__("importlib").import_module("4d_ttt_merging_amd.mass_bias_attention")
+    heads = 2 if batch < 20_000 else 16
+    g = torch.Generator(device=device).manual_seed(batch)
+    q = torch.randn(batch, heads, 1, 64, device=device, generator=g)
+    v = torch.randn(batch, heads, 1, 64, device=device, generator=g)
+    out = torch.full_like(v, float("nan"))
+    mba._attention_into(q, q, v, None, out, split=split)
+    assert torch.equal(out, v)
+    if batch < 100_000:  # two key tiles each, shared by all batch elements
+        k, v = (torch.randn(1, heads, 65, 64, device=device, generator=g).expand(batch, -1, -1, -1) for _ in range(2))
+        mba._attention_into(q, k, v, None, out.fill_(float("nan")), split=split)
+        for rows in (slice(0, 50), slice(batch // 2, batch // 2 + 50), slice(batch - 50, batch)):
+            assert_close(out[rows].cpu(), _reference(*(t[rows].cpu() for t in (q, k, v)), None), torch.float32)
+        assert torch.isfinite(out).all()
+
+
 def test_split_workspace_is_checked(vgo, device):
     lib_mod = __import__("importlib").import_module("4d_ttt_merging_amd._lib")
     lib = lib_mod.load()

@@ -444,26 +444,28 @@ Tensor dense_block(const Tensor& x, const c10::List<OptTensor>& norms, at::Array
   const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
   const int64_t batch = x.size(0), tokens = x.size(1), dim = x.size(2);
   const auto linear = [&](const Tensor& in, int i) { return at::linear(in, *linears.get(2 * i), linears.get(2 * i + 1)); };
-  const Tensor h = residual_layer_norm(x, std::nullopt, std::nullopt, norms.get(0), norms.get(1), eps[0], true, true,
-                                       dtype, false, -1.0)[1];
-  const Tensor qkv = linear(h, 0);
-  const int64_t prefix = opt(rope_sin) == nullptr ? 0 : tokens - rope_sin->size(-2);
-  TORCH_CHECK(prefix >= 0, "dense_block: more RoPE positions than tokens");
-  // The attention takes v where the projection wrote it: copying it head-major was a third of
-  // the epilogue's bytes (a block of 32 x 1,029 tokens 1,384 -> 1,370 us).  Copied only where the
-  // kernels' 32-bit token offsets (stride x tokens < 2^31) do not reach; layers.py `_value_rows`
-  // is the same rule.
-  const bool v_in_place = tokens * 3 * dim < (int64_t{1} << 31);
-  const std::vector<Tensor> heads_out =
-      qkv_epilogue(qkv.reshape({batch * tokens, 3 * dim}), heads, tokens, tokens, std::nullopt, norms.get(4),
-                   norms.get(5), norms.get(6), norms.get(7), eps[2], rope_sin, rope_cos, prefix,
-                   c10::List<bool>({true, true, !v_in_place}), dtype);
-  const Tensor v = v_in_place ? qkv.view({batch, tokens, 3, heads, 64}).select(2, 2).transpose(1, 2) : heads_out[2];
-  const Tensor attended = at::empty({batch, tokens, heads, 64}, x.options().dtype(dtype));
-  attention_into(heads_out[0], heads_out[1], v, std::nullopt, attended.permute({0, 2, 1, 3}), -1);
-  const std::vector<Tensor> rows =
-      residual_layer_norm(x, linear(attended.view({batch, tokens, dim}), 1), gammas.get(0), norms.get(2), norms.get(3),
-                          eps[1], true, true, dtype, false, -1.0);
+  // In a scope of its own: the packed rows, q, k and the attention's output are free again in the MLP.
+  const std::vector<Tensor> rows = [&] {
+    const Tensor h = residual_layer_norm(x, std::nullopt, std::nullopt, norms.get(0), norms.get(1), eps[0], true, true,
+                                         dtype, false, -1.0)[1];
+    const Tensor qkv = linear(h, 0);
+    const int64_t prefix = opt(rope_sin) == nullptr ? 0 : tokens - rope_sin->size(-2);
+    TORCH_CHECK(prefix >= 0, "dense_block: more RoPE positions than tokens");
+    // The attention takes v where the projection wrote it: copying it head-major was a third of
+    // the epilogue's bytes (a block of 32 x 1,029 tokens 1,384 -> 1,370 us).  Copied only where the
+    // kernels' 32-bit token offsets (stride x tokens < 2^31) do not reach; layers.py `_value_rows`
+    // is the same rule.
+    const bool v_in_place = tokens * 3 * dim < (int64_t{1} << 31);
+    const std::vector<Tensor> heads_out =
+        qkv_epilogue(qkv.reshape({batch * tokens, 3 * dim}), heads, tokens, tokens, std::nullopt, norms.get(4),
+                     norms.get(5), norms.get(6), norms.get(7), eps[2], rope_sin, rope_cos, prefix,
+                     c10::List<bool>({true, true, !v_in_place}), dtype);
+    const Tensor v = v_in_place ? qkv.view({batch, tokens, 3, heads, 64}).select(2, 2).transpose(1, 2) : heads_out[2];
+    const Tensor attended = at::empty({batch, tokens, heads, 64}, x.options().dtype(dtype));
+    attention_into(heads_out[0], heads_out[1], v, std::nullopt, attended.permute({0, 2, 1, 3}), -1);
+    return residual_layer_norm(x, linear(attended.view({batch, tokens, dim}), 1), gammas.get(0), norms.get(2),
+                               norms.get(3), eps[1], true, true, dtype, false, -1.0);
+  }();
   return mlp_tail(rows[0], rows[1], *linears.get(4), linears.get(5), *linears.get(6), linears.get(7), gammas.get(1));
 }
 
@@ -640,29 +642,31 @@ Tensor merged_block(const Tensor& x, const OptTensor& h0, const OptTensor& qkv0,
   const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
   const int64_t tokens = x.size(1), dim = x.size(2), kept = counts.numel();
   const auto linear = [&](const Tensor& in, int i) { return at::linear(in, *linears.get(2 * i), linears.get(2 * i + 1)); };
-  Tensor qkv = opt(qkv0) == nullptr ? Tensor() : *qkv0;
-  if (!qkv.defined()) {
-    const Tensor h = opt(h0) != nullptr ? *h0
-                                        : residual_layer_norm(x, std::nullopt, std::nullopt, norms.get(0),
-                                                              norms.get(1), eps[0], true, true, dtype, false, -1.0)[1];
-    qkv = linear(h, 0);
-  }
-  const Tensor operands = at::empty({3, 1, heads, kept, 64}, x.options().dtype(dtype));
-  const Tensor q = operands.select(0, 0), k = operands.select(0, 1), v = operands.select(0, 2);
-  const std::array<Tensor, 3> outs = {q.select(0, 0), k.select(0, 0), v.select(0, 0)};
-  const std::array<int64_t, 3> at_channel = {0, dim, 2 * dim};
-  const std::array<double, 3> ln_eps = {eps[2], eps[2], 0.0};
-  const c10::List<OptTensor> weights({norms.get(4), norms.get(6), std::nullopt});
-  const c10::List<OptTensor> biases({norms.get(5), norms.get(7), std::nullopt});
-  compact_multi_into(qkv.reshape({tokens, 3 * dim}), at_channel, outs, weights, biases, ln_eps, std::nullopt, offsets,
-                     1, order, 0, std::nullopt, contribution, counts);
-  OptTensor bias;
-  if (opt(log_mass) != nullptr) bias = log_mass->reshape({-1}).to(dtype);
-  const Tensor attended = at::empty({1, kept, heads, 64}, x.options().dtype(dtype));
-  attention_into(q, k, v, bias, attended.permute({0, 2, 1, 3}), -1);
-  const Tensor table = linear(attended.view({kept, dim}), 1);
-  const std::vector<Tensor> rows = restore_residual_layer_norm(x, table, inverse, std::nullopt, gammas.get(0),
-                                                               norms.get(2), norms.get(3), eps[1], dtype);
+  const std::vector<Tensor> rows = [&] {  // (a scope of its own, as dense_block's)
+    Tensor qkv = opt(qkv0) == nullptr ? Tensor() : *qkv0;
+    if (!qkv.defined()) {
+      const Tensor h = opt(h0) != nullptr ? *h0
+                                          : residual_layer_norm(x, std::nullopt, std::nullopt, norms.get(0),
+                                                                norms.get(1), eps[0], true, true, dtype, false, -1.0)[1];
+      qkv = linear(h, 0);
+    }
+    const Tensor operands = at::empty({3, 1, heads, kept, 64}, x.options().dtype(dtype));
+    const Tensor q = operands.select(0, 0), k = operands.select(0, 1), v = operands.select(0, 2);
+    const std::array<Tensor, 3> outs = {q.select(0, 0), k.select(0, 0), v.select(0, 0)};
+    const std::array<int64_t, 3> at_channel = {0, dim, 2 * dim};
+    const std::array<double, 3> ln_eps = {eps[2], eps[2], 0.0};
+    const c10::List<OptTensor> weights({norms.get(4), norms.get(6), std::nullopt});
+    const c10::List<OptTensor> biases({norms.get(5), norms.get(7), std::nullopt});
+    compact_multi_into(qkv.reshape({tokens, 3 * dim}), at_channel, outs, weights, biases, ln_eps, std::nullopt, offsets,
+                       1, order, 0, std::nullopt, contribution, counts);
+    OptTensor bias;
+    if (opt(log_mass) != nullptr) bias = log_mass->reshape({-1}).to(dtype);
+    const Tensor attended = at::empty({1, kept, heads, 64}, x.options().dtype(dtype));
+    attention_into(q, k, v, bias, attended.permute({0, 2, 1, 3}), -1);
+    const Tensor table = linear(attended.view({kept, dim}), 1);
+    return restore_residual_layer_norm(x, table, inverse, std::nullopt, gammas.get(0), norms.get(2), norms.get(3),
+                                       eps[1], dtype);
+  }();
   return mlp_tail(rows[0], rows[1], *linears.get(4), linears.get(5), *linears.get(6), linears.get(7), gammas.get(1));
 }
 

@@ -69,6 +69,29 @@ def test_merged_block(vgo, device, mass):
             block.forward_compacted(x, bad)
 
 
+@pytest.mark.parametrize("kind", ["dense", "merged"])
+def test_a_native_block_holds_no_more_memory(vgo, device, kind):
+    """The attention's tensors are free again when the MLP's are made, as on the call-by-call route."""
+    block = _block(vgo, 512, 8, device, use_qk_norm=True, init_values=0.5)
+    tokens, kept = 40_000, 30_000
+    x = torch.randn(1, tokens, 512, device=device)
+    plan = vgo.TokenPlan(torch.arange(kept, device=device)[None], (torch.arange(tokens, device=device) % kept)[None], tokens)
+
+    def peak():
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = block(x.view(40, 1000, 512)) if kind == "dense" else block.forward_compacted(x, plan)
+        del out
+        return torch.cuda.max_memory_allocated() - before
+
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        peak()  # casts the weights and derives the plan's clusters
+        native, plain, fired = _both(block, peak)
+    print(f"[block memory] {kind}: native {native / 2**20:.0f} MiB, call by call {plain / 2**20:.0f}", flush=True)
+    assert fired == 1 and native <= plain + 2 ** 20
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch,tokens", [(1, 1), (3, 37), (1, 2700)])  # 2,700: the workspace kernel
 def test_values_in_place(vgo, device, dtype, batch, tokens):

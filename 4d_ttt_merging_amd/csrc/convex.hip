@@ -33,13 +33,15 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-// v[i] / d, correctly rounded, with one division for the whole row: y = 1 / d rounded to
-// nearest, q = v y, and one residual step, fma(fma(-q, d, v), y, q), give the rounded quotient
-// (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor",
-// 1990).  A component is no larger than its norm d, so only d itself can leave the range in
-// which that holds; such rows divide.  The 160 divisions of a row's fit were most of its
-// instructions: 5,672 rows, 3,253 to solve, 36 -> 28 us,
-// 3,143 listed rows 31 -> 20.
+// v[i] / d with one division for the whole row: y = 1 / d rounded to nearest, q = v y, and one
+// residual step, fma(fma(-q, d, v), y, q) (Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000 processor", 1990).  A component is no larger than its norm d, so nothing
+// overflows, and it is the correctly rounded quotient where neither q nor the residual is subnormal:
+// |v| >= 2^-100 and |v / d| >= 2^-125.  Below, a quotient may be one unit of its last place (or of the
+// smallest subnormal) off, and -0 gives +0: in a row that is not all as small, nothing that the fit's
+// sums of squares and products with larger components can show.
+// The 160 divisions of a row's fit were most of its instructions: 5,672 rows, 3,253 to solve, 36 ->
+// 28 us, 3,143 listed rows 31 -> 20.
 __device__ __forceinline__ void divide_row(float* v, float d) {
   if (d > 0x1p-60f && d < 0x1p60f) {
     const float y = 1.0f / d;

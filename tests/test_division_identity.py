@@ -5,7 +5,11 @@ kernel uses for every value in [2^-100, FLT_MAX] and normalizers in [1, 2^16]
 (csrc/segment.hip, divide_by_normalizer).  Checked here in exact rational arithmetic
 with one rounding per operation, for integer counts and fractional masses in
 [1, 2^16], random values, values next to exact quotients, sparse mantissas and the
-ends of that range."""
+ends of that range.
+
+The sparse-convex fit divides a row by its norm with the same steps and no look at its
+values (csrc/convex.hip, divide_row): the second test has the range in which that is the
+rounded division, and how far off it is below."""
 import random
 from fractions import Fraction
 
@@ -60,3 +64,30 @@ def test_markstein_corrected_quotient_is_the_rounded_division():
             assert corrected_quotient(a, n) == rn32(Fraction(float(a)) / fn), (a, n)
             checked += 1
     assert checked > 1500
+
+
+def _rounded_division(v: np.float32, d: np.float32) -> np.float32:
+    return rn32(Fraction(float(v)) / Fraction(float(d)))
+
+
+def test_row_division_range():
+    rng = random.Random(12)
+    smallest = Fraction(2) ** -149
+    inside = below = 0
+    for _ in range(60):
+        d = np.float32(rng.uniform(1, 2) * 2.0 ** rng.randint(-59, 58))
+        exponent = int(np.floor(np.log2(float(d))))
+        for _ in range(40):
+            # A component of either sign, from the norm's size down to the subnormals.
+            v = np.float32(rng.uniform(1, 2) * 2.0 ** rng.randint(-148, exponent - 1) * rng.choice((-1, 1)))
+            got, expect = corrected_quotient(v, d), _rounded_division(v, d)
+            if abs(float(v)) >= 2.0 ** -100 and abs(float(v) / float(d)) >= 2.0 ** -125:
+                assert got == expect, (v, d)
+                inside += 1
+            else:
+                unit = max(Fraction(float(np.spacing(np.abs(expect)))), smallest)
+                assert abs(Fraction(float(got)) - Fraction(float(expect))) <= unit, (v, d)
+                below += 1
+    assert inside > 500 and below > 500
+    assert _rounded_division(np.float32(2.0 ** -100), np.float32(1.5)) == corrected_quotient(
+        np.float32(2.0 ** -100), np.float32(1.5))

@@ -775,9 +775,10 @@ __global__ __launch_bounds__(kThreads) void fastvggt_plan_kernel(
   // In-place exclusive scan of chunk_cnt[0, chunks x waves) -> each (chunk, wave)'s base.
   auto scan_chunks = [&](int chunks) {
     __syncthreads();
+    static_assert(kPlanChunks * kWavesS <= kThreads, "one count per thread");
     const int n = chunks * kWavesS;
     int sum = 0;
-    const int mine = tid < n ? chunk_cnt[tid] : 0;  // n <= 640
+    const int mine = tid < n ? chunk_cnt[tid] : 0;
     const int pre = block_exclusive_scan(mine, scan_lds, &sum);
     if (tid < n) chunk_cnt[tid] = pre;
     __syncthreads();

@@ -412,7 +412,7 @@ std::vector<Tensor> restore_residual_layer_norm(const Tensor& x, const Tensor& t
 // -------------------------------------------------------------- whole blocks ----
 // Exact GELU of a tensor that nothing else holds.  From 2^23 bf16 values on the table kernel runs in
 // place, with the bits of torch's kernel (us, torch / table: 2^22 values 6.6 / 8.5, 2^23 10.2 / 9.1,
-// 2^25 29.7 / 23.0, 32,928 x 4,096 122 / 109): below, its table costs more than it saves.
+// 2^25 29.7 / 23.0, 32,928 x 4,096 122 / 107): below, its table costs more than it saves.
 Tensor gelu_owned(const Tensor& t) {
   if (t.scalar_type() != at::kBFloat16 || t.numel() < (int64_t{1} << 23) || !t.is_contiguous() ||
       reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0)

@@ -429,7 +429,8 @@ class SelfAttention(nn.Module):
 
     @staticmethod
     def _attend(q: Tensor, k: Tensor, v: Tensor, bias, x: Tensor, special, output_indices) -> None:
-        """Merged attention into x; with a dense special-query pass, both in one launch.
+        """Merged attention into x; with a dense special-query pass, both in one operator (one launch
+        in bf16 / f16).
 
         The special rows then replace the merged result's rows, as the
         reference's `x.index_copy_` does (attention.py:420)."""

@@ -61,9 +61,9 @@ def _attention_into(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 
 
 def _attention_pair_into(main: tuple, special: tuple) -> None:
-    """Merged attention and the dense special-query pass in one launch
-    (torch.ops.vgo.attention_pair_into).  `main` and `special` are (q, k, v, bias, out) as
-    for `_attention_into`; each output receives its problem's result."""
+    """Merged attention and the dense special-query pass (torch.ops.vgo.attention_pair_into):
+    one launch in bf16 / f16, in fp32 one problem after the other.  `main` and `special` are
+    (q, k, v, bias, out) as for `_attention_into`; each output receives its problem's result."""
     torch.ops.vgo.attention_pair_into(*main, *special)
 
 

@@ -44,7 +44,8 @@ _SCHEMAS = (
     # The same into `out` (any strides with a unit channel stride); split: -1 picks the
     # entry by key length, 0 the entry without a workspace, 1 the workspace entry.
     "attention_into(Tensor q, Tensor k, Tensor v, Tensor? bias, Tensor(a!) out, SymInt split) -> ()",
-    # Merged attention and the dense special-query pass in one launch.
+    # Merged attention and the dense special-query pass: one launch in bf16 / f16, in fp32 one
+    # after the other.
     "attention_pair_into(Tensor q, Tensor k, Tensor v, Tensor? bias, Tensor(a!) out, Tensor special_q, "
     "Tensor special_k, Tensor special_v, Tensor? special_bias, Tensor(b!) special_out) -> ()",
     # out[i] = sum_c weight[i, c] * table[index[i, c]]: table [M, D], index [N, 4] int32,

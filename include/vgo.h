@@ -141,7 +141,8 @@ typedef struct vgo_attn_problem {
 } vgo_attn_problem;
 
 /*
- * Merged global attention and its dense special-query pass in one launch.
+ * Merged global attention and its dense special-query pass in one launch (bf16 / f16; fp32
+ * problems run one after the other).
  * problems[0] is the mass-bias attention over merged keys; problems[1]
  * (count == 2) is the exact pass of the special-token queries over every
  * original key, without bias.  Together they replace the two calls of

@@ -112,8 +112,12 @@ def _attention_split(vgo, q, k, v, bias, split):
     (1, 16, 1044, 522),   # 80 tasks of 9 key tiles spread over ~90 work-groups
     (1, 2, 100, 20000),   # 2 tasks of 313 tiles: each cut over dozens of work-groups
     (2, 3, 700, 1333),    # batch > 1, ragged query and key tails
+    (1, 64, 1044, 522),   # the first and third again, with the register-staged kernel as
+    (2, 24, 700, 1333),   # the one without a workspace (more than 768 groups of 32 queries)
 ])
 def test_stream_k_and_plain_schedules_match_oracle(vgo, device, shape):
+    """The entry with a workspace, and the one without: the key-split kernel for the first three
+    shapes, the register-staged kernel for the last two."""
     b, h, nq, nk = shape
     print(f"[attn schedules] shape={shape}", flush=True)
     q, k, v, mass = _inputs(31 + nq, b, h, nq, nk, torch.bfloat16)
@@ -164,7 +168,7 @@ def _pair(vgo, main, special):
     ((1, 1, 1, 1), (1, 1, 1, 65)),               # single rows
 ])
 def test_pair_launch_matches_oracle(vgo, device, dtype, shapes):
-    """Merged attention and the dense special-query pass in one launch."""
+    """Merged attention and the dense special-query pass in one call (one launch in bf16 / f16)."""
     (b0, h0, nq0, nk0), (b1, h1, nq1, nk1) = shapes
     # fp32: each output averages nk unit-variance values to ~1/sqrt(nk) of their scale,
     # so the rounding of the running sums sets the error; the kernel sums 32 keys at a
@@ -264,17 +268,18 @@ def test_kernel_timing_records_each_workspace_launch(vgo, device):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("std", [1.0, 2.0, 3.0])
-@pytest.mark.parametrize("nk", [1500, 3000])
-def test_wide_logits_match_oracle(vgo, device, dtype, std, nk):
+@pytest.mark.parametrize("heads,nk", [(4, 1500), (48, 1500), (4, 3000)])
+def test_wide_logits_match_oracle(vgo, device, dtype, std, heads, nk):
     """q, k at unit scale (the aggregator's operating point: per-head LayerNorm'd
     q and k) and at 2-3x unit scale (logits of tens in the exp2 domain, which take
-    the lazy softmax's rescaling path on many tiles); both kernels (1,500 keys:
-    register-staged, 3,000: ping-pong) stay within the tolerance of the oracle.
+    the lazy softmax's rescaling path on many tiles); the three kernels (1,500 keys:
+    key-split at 4 heads, 84 groups of 32 queries, and register-staged at 48, 1,008
+    groups; 3,000 keys: ping-pong) stay within the tolerance of the oracle.
     657 queries leave a wave with 17 (past 2 x 256 + 128), which the
     register-staged kernel runs as one 32-query block.  The measured error is
     printed beside the bar."""
-    print(f"[attn] wide logits dtype={dtype} std={std} nk={nk}", flush=True)
-    q, k, v, mass = _inputs(int(std * 10) + nk, 1, 4, 657, nk, dtype, mass_max=16, std=std)
+    print(f"[attn] wide logits dtype={dtype} std={std} heads={heads} nk={nk}", flush=True)
+    q, k, v, mass = _inputs(int(std * 10) + nk, 1, heads, 657, nk, dtype, mass_max=16, std=std)
     out = vgo.mass_bias_attention(q.to(device), k.to(device), v.to(device), mass.log().to(device))
     torch.cuda.synchronize()
     ref = oracle.mass_bias_attention(q, k, v, mass.log())
@@ -306,15 +311,17 @@ def test_c4_unit_scale_rows_match_oracle(vgo, device, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("nk", [1029, 3000])
-def test_zero_mass_leading_keys_match_oracle(vgo, device, dtype, nk):
+@pytest.mark.parametrize("heads,nk", [(3, 1029), (48, 1029), (3, 3000)])
+def test_zero_mass_leading_keys_match_oracle(vgo, device, dtype, heads, nk):
     """Keys of mass 0 (log-mass bias -inf) take no weight.  With the first 80 keys
     and a scattered tenth of the rest at mass 0, the first key tile of every task
-    holds no finite logit: the register-staged kernel (1,029 keys) starts its
-    first-tile softmax with the reference max still at -inf, the ping-pong kernel
-    (3,000 keys) its rescaling path, and both must leave those keys out."""
-    print(f"[attn] zero-mass leading keys dtype={dtype} nk={nk}", flush=True)
-    q, k, v, mass = _inputs(97 + nk, 1, 3, 657, nk, dtype, mass_max=8, std=1.0 if dtype == torch.float32 else 0.5)
+    holds no finite logit: the register-staged kernel (1,029 keys, 48 heads: 1,008
+    groups of 32 queries) starts its first-tile softmax with the reference max still
+    at -inf, so does a wave of the key-split kernel (3 heads: 63 groups), and the
+    ping-pong kernel (3,000 keys) its rescaling path; all must leave those keys out."""
+    print(f"[attn] zero-mass leading keys dtype={dtype} heads={heads} nk={nk}", flush=True)
+    q, k, v, mass = _inputs(97 + nk, 1, heads, 657, nk, dtype, mass_max=8,
+                            std=1.0 if dtype == torch.float32 else 0.5)
     g = torch.Generator().manual_seed(98)
     mass[:80] = 0.0
     mass[torch.randperm(nk, generator=g)[: nk // 10]] = 0.0
@@ -331,8 +338,8 @@ def test_zero_mass_leading_keys_match_oracle(vgo, device, dtype, nk):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("split", [True, False])
 @pytest.mark.parametrize("case", [
-    (8, 1100, 3000),   # split: 24 tasks, every segment a stream-K piece of 4-5 key tiles
-    (64, 2100, 700),   # split: 320 tasks, a round of whole tasks, then stream-K pieces
+    (8, 1100, 3000),   # split: 24 tasks, every segment a stream-K piece of 4-5 key tiles; else key-split
+    (64, 2100, 700),   # split: 320 tasks, a round of whole tasks, then stream-K pieces; else register-staged
 ])
 def test_late_heavy_keys_rescale_mid_segment(vgo, device, dtype, split, case):
     """Keys whose log-mass bias steps up by 11 (more than the lazy softmax's 15 ln 2
@@ -340,8 +347,9 @@ def test_late_heavy_keys_rescale_mid_segment(vgo, device, dtype, split, case):
     the fast path's range on those tiles, which are not the first tile of their
     segment, so the rescaling path runs mid-segment (in the ping-pong kernel, split,
     at the start of the following MFMA phase for both wave groups; in the
-    register-staged kernel before its P.V) and must rescale O and the sums that
-    earlier tiles left.  fp32 runs its own kernel either way."""
+    register-staged kernel and in a wave of the key-split kernel before its P.V) and
+    must rescale O and the sums that earlier tiles left.  fp32 runs its own kernel
+    either way."""
     h, nq, nk = case
     if dtype == torch.float32 and not split:
         pytest.skip("fp32 takes the same kernel for both entries")

@@ -72,9 +72,11 @@ def test_normalize_rows(kern, device, dim, eps):
 # ------------------------------------------------------------- matching ----
 @pytest.mark.parametrize("topk", [1, 4])
 @pytest.mark.parametrize("ns,nd,dim", [(37, 11, 64), (300, 777, 1024), (1000, 130, 128), (260, 300, 72),
-                                        # one or two 32-wide K chunks in all: fewer steps than the
-                                        # ring's look-ahead (regression: the DMA count must stay uniform)
-                                        (513, 40, 32), (700, 257, 32), (90, 600, 64)])
+                                        (513, 40, 32), (700, 257, 32), (90, 600, 64),
+                                        # the ring kernel (more than 64 tiles of 256 x 256); with one or two
+                                        # 32-wide K chunks in all, fewer steps than its look-ahead
+                                        # (regression: the DMA count must stay uniform)
+                                        (16641, 40, 32), (8500, 257, 32), (16390, 200, 64), (4200, 1100, 1024)])
 def test_similarity_selection_is_exact_on_kernel_scores(kern, device, topk, ns, nd, dim):
     print(f"[similarity] topk={topk} ns={ns} nd={nd} dim={dim}", flush=True)
     g = torch.Generator().manual_seed(ns + nd + topk)
@@ -99,10 +101,12 @@ def test_similarity_selection_is_exact_on_kernel_scores(kern, device, topk, ns, 
 @pytest.mark.parametrize("dim", [64, 72])
 @pytest.mark.parametrize("topk", [1, 4])
 @pytest.mark.parametrize("nd", [768, 1000])
-def test_similarity_topk_on_crafted_rounding_ties(kern, device, nd, topk, dim):
-    """With dim 64, full 256-row dictionary tiles take the two-pass top-1 epilogue (the
-    fp32 maximum, then the first score at or above the lower bound of its bf16 rounding
-    interval); dim 72 takes the 128-row kernel.  The dictionary puts scores exactly on
+@pytest.mark.parametrize("repeats", [1, 48])
+def test_similarity_topk_on_crafted_rounding_ties(kern, device, repeats, nd, topk, dim):
+    """With dim 64 and more than 64 tiles (48 times the source rows), full 256-row dictionary
+    tiles take the two-pass top-1 epilogue (the fp32 maximum, then the first score at or
+    above the lower bound of its bf16 rounding interval); dim 72, and fewer tiles, take the
+    128-row kernel.  The dictionary puts scores exactly on
     bf16 midpoints (ties to even, up and down), a quarter ulp either side of them and on
     bf16 values, so several fp32 scores at several positions round to each row's maximum;
     source rows negate them, zero them, and one row (in another wave, which then takes the
@@ -110,7 +114,7 @@ def test_similarity_topk_on_crafted_rounding_ties(kern, device, nd, topk, dim):
     that must rank above +inf after the dictionary parts are merged.  All products and
     sums are exact in fp32, so the kernel's scores equal the exact ones and the selection
     must be the lowest indices of the bf16 maxima."""
-    print(f"[similarity] crafted rounding ties nd={nd} topk={topk} dim={dim}", flush=True)
+    print(f"[similarity] crafted rounding ties nd={nd} topk={topk} dim={dim} x {repeats}", flush=True)
     g = torch.Generator().manual_seed(nd)
     half = 2.0 ** -9
     k = torch.randint(-2, 3, (nd,), generator=g).float()
@@ -124,9 +128,10 @@ def test_similarity_topk_on_crafted_rounding_ties(kern, device, nd, topk, dim):
     for i in range(128):
         src[i, :2] = torch.tensor(kinds[i % len(kinds)])
     src[100, :2] = torch.tensor([float("inf"), 0.0])
+    src = src.repeat(repeats, 1)
     src_b, dst_b = src.bfloat16(), dst.bfloat16()
     assert torch.equal(src_b.float(), src) and torch.equal(dst_b.float(), dst)
-    scores = torch.full((128, nd), float("nan"), dtype=torch.bfloat16, device=device)
+    scores = torch.full((128 * repeats, nd), float("nan"), dtype=torch.bfloat16, device=device)
     values, index = kern.similarity_topk(src_b.to(device), dst_b.to(device), topk, scores=scores)
     ks = scores.float().cpu()
     exact = om.bf16_scores(src_b, dst_b)
@@ -165,23 +170,23 @@ def test_similarity_ranges_rows_and_device_count(kern, device):
     assert torch.isnan(scores[211:].float()).all()  # rows past the device count are untouched
 
 
-@pytest.mark.parametrize("dim", [256, 72])
-def test_similarity_invalid_source_ids_score_zero(kern, device, dim):
+@pytest.mark.parametrize("ns,nd,dim", [(200, 300, 256), (200, 300, 72), (4400, 1200, 256)])
+def test_similarity_invalid_source_ids_score_zero(kern, device, ns, nd, dim):
     # Row ids outside the source buffer read as zero rows: every score is 0 and
-    # the lowest dictionary indices win (both kernels: dim 256 and dim 72).
+    # the lowest dictionary indices win (the 128-row kernel, and the ring kernel at 90 tiles).
     g = torch.Generator().manual_seed(6)
-    src = F.normalize(torch.randn(200, dim, generator=g), dim=-1).bfloat16()
-    dst = F.normalize(torch.randn(300, dim, generator=g), dim=-1).bfloat16()
-    rows = torch.arange(200)
-    rows[[0, 77, 150]] = torch.tensor([200, 10 ** 6, -1])
+    src = F.normalize(torch.randn(ns, dim, generator=g), dim=-1).bfloat16()
+    dst = F.normalize(torch.randn(nd, dim, generator=g), dim=-1).bfloat16()
+    rows = torch.arange(ns)
+    rows[[0, 77, 150]] = torch.tensor([ns, 10 ** 6, -1])
     for topk in (1, 4):
         values, index = kern.similarity_topk(src.to(device), dst.to(device), topk, src_rows=rows.to(device),
-                                             n_src=200)
+                                             n_src=ns)
         v, i = values.cpu(), index.cpu()
         for r in (0, 77, 150):
             assert torch.equal(v[r].reshape(-1), torch.zeros(topk))
             assert torch.equal(i[r].reshape(-1), torch.arange(topk))
-        good = torch.ones(200, dtype=torch.bool)
+        good = torch.ones(ns, dtype=torch.bool)
         good[[0, 77, 150]] = False
         exact = om.bf16_scores(src[rows[good]], dst)
         ref_v, ref_i = om.topk_lowest_index(exact, topk)

@@ -255,6 +255,8 @@ def require_gpu(*tensors: torch.Tensor) -> None:
 def require_plain(*tensors: torch.Tensor) -> None:
     """The planners' operators leave no trace in autograd, so a function transform (vmap, grad, jvp)
     over one would silently lose its derivative."""
+    if torch.compiler.is_compiling():  # a traced graph runs on plain tensors
+        return
     for tensor in tensors:
         if tensor is not None and torch._C._functorch.is_functorch_wrapped_tensor(tensor):
             raise RuntimeError("vgo planners take no tensors of function transforms (vmap, grad, jvp)")

@@ -252,10 +252,13 @@ def require_gpu(*tensors: torch.Tensor) -> None:
             raise RuntimeError("vgo kernels run on the GPU only; got a CPU tensor")
 
 
+_transforms = torch._C._functorch.peek_interpreter_stack
+
+
 def require_plain(*tensors: torch.Tensor) -> None:
     """The planners' operators leave no trace in autograd, so a function transform (vmap, grad, jvp)
     over one would silently lose its derivative."""
-    if torch.compiler.is_compiling():  # a traced graph runs on plain tensors
+    if torch.compiler.is_compiling() or _transforms() is None:  # (a traced graph runs on plain tensors)
         return
     for tensor in tensors:
         if tensor is not None and torch._C._functorch.is_functorch_wrapped_tensor(tensor):

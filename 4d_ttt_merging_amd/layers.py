@@ -701,8 +701,11 @@ def _cast_linears(*linears: nn.Module) -> tuple | None:
         return None
     cast = []
     for linear in linears:
-        if not (_plain(linear, Linear, LinearKMaskedBias) and linear.weight.is_cuda
-                and type(linear.weight) in _TENSORS and (linear.bias is None or type(linear.bias) in _TENSORS)):
+        if not _plain(linear, Linear, LinearKMaskedBias):
+            return None
+        parameters = linear._parameters  # (an attribute of a module costs its __getattr__)
+        weight, bias = parameters.get("weight"), parameters.get("bias")
+        if type(weight) not in _TENSORS or not weight.is_cuda or (bias is not None and type(bias) not in _TENSORS):
             return None
         pair = linear._cast_params(dtype)
         if pair is None:

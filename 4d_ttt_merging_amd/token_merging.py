@@ -596,17 +596,19 @@ def build_fastvggt_plan(
     plan = TokenPlan(keep, inverse, total)
     # Match results stay on the device for diagnostics and tests.
     plan._derived["match"] = (sources, destinations, best, target, flags)
+    if not mass_bias:
+        # Derived on first use, from the plan as it is then (its pool_mask, say).
+        if one_launch:
+            plan._derived["built"] = _Built(inverse, inverse._version, inverse32, _Csr(order, offsets), counts)
+        return plan
+    # The clusters whose sizes the mass is.
     if one_launch:
-        plan._derived["built"] = _Built(inverse, inverse._version, inverse32, _Csr(order, offsets), counts)
-    elif mass_bias:
+        plan._derived[("inverse32", 0)] = inverse32
+    else:
         # One mass pass gives the cluster counts _cluster_csr caches and their logs.
         order, offsets = _kernels.csr_build(plan._inverse32(0), plan.kept_tokens)
         counts, log_mass = _kernels.segment_mass(offsets, 1, order, None, plan.kept_tokens, 0.0,
                                                  want_log=True)
-    if mass_bias:
-        # The clusters whose sizes the mass is; without it they are derived on first use, from
-        # the plan as it is then (its pool_mask, say).
-        plan._inverse32(0)
-        plan._derived[("csr", 0)] = (_Csr(order, offsets), counts, None)
-        plan.key_log_mass = log_mass.view(1, -1)
+    plan._derived[("csr", 0)] = (_Csr(order, offsets), counts, None)
+    plan.key_log_mass = log_mass.view(1, -1)
     return plan

@@ -169,3 +169,58 @@ def test_column_slices_at_their_edges(vgo, device, dtype, m):
         index[0] = torch.tensor([0, m - 1, m - 1, 0], dtype=torch.int32)
         out = vgo.top4_project(table.to(device), index.to(device), weight.to(device))
         assert torch.equal(out.cpu(), oracle.top4_project(table, index, weight))
+
+
+def _rows_like(pattern, n, m, device, seed):
+    """Index and weight of n rows: `kept` and `one_hot` with one corner each (ascending, scattered),
+    `part` half and half with four, `near` four corners within 128 table rows, `mixed` four anywhere."""
+    g = torch.Generator(device=device).manual_seed(seed)
+    ascending = (torch.arange(n, device=device) * m // n)[:, None]
+    index = torch.randint(0, m, (n, 4), device=device, generator=g)
+    weight = torch.rand(n, 4, device=device, generator=g) + 0.01
+    single = torch.zeros(n, dtype=torch.bool, device=device)
+    if pattern == "near":
+        index = (ascending + torch.randint(-64, 65, (n, 4), device=device, generator=g)).clamp_(0, m - 1)
+    if pattern in ("kept", "one_hot", "part"):
+        single = torch.rand(n, device=device, generator=g) < 0.5 if pattern == "part" else ~single
+        if pattern != "one_hot":
+            index[single] = ascending.expand(-1, 4)[single]
+        weight[single] = torch.tensor([1.0, 0.0, 0.0, 0.0], device=device)
+    weight /= weight.sum(1, keepdim=True)
+    index[1], weight[1] = m + 7, 0.25           # poisons its row
+    index[n - 1, 3], weight[n - 1, 3] = -3, 0.0  # no weight: ignored
+    return index.int(), weight
+
+
+# On both sides of the output sizes (96, 256, 512 MB and 1.5 GB), the table sizes (12 MB per slice) and
+# the row lengths (2, 3 and 4 chunks per lane, the last one ragged) at which whole rows come in.
+@pytest.mark.parametrize("dtype,n,m,d", [
+    (torch.float32, 24575, 12288, 1024), (torch.float32, 24577, 12288, 1024), (torch.float32, 24577, 49153, 1024),
+    (torch.float32, 32901, 60000, 768), (torch.float32, 131075, 49153, 512), (torch.float32, 393217, 49152, 1024),
+    (torch.bfloat16, 131073, 3000, 1024), (torch.bfloat16, 43401, 98305, 1160),
+    (torch.bfloat16, 262145, 16384, 1024), (torch.bfloat16, 786433, 98304, 1024),
+    (torch.float16, 131073, 98305, 1000), (torch.float16, 24577, 9000, 2048),
+    (torch.float16, 262145, 98305, 1024), (torch.float16, 786433, 98305, 1024)])
+def test_whole_rows_equal_slices(vgo, device, dtype, n, m, d):
+    """Rows of every kind that the sample tells apart: the whole call, the rows in an order and the
+    same rows in pieces (below 64 MB: by slices) are equal bit for bit, and 256 rows equal the oracle."""
+    from tests.conftest import import_package
+    proj = import_package("projection")
+    table = torch.randn(m, d, device=device, generator=torch.Generator(device=device).manual_seed(n)).to(dtype)
+    order = torch.arange(n - 1, -1, -1, dtype=torch.int32, device=device)
+    piece = (64 << 20) // (d * table.element_size())
+    pick = torch.linspace(0, n - 1, 256).long()
+    for pattern in ("kept", "one_hot", "part", "near", "mixed"):
+        print(f"[project] {pattern} rows dtype={dtype} n={n} m={m} d={d}", flush=True)
+        index, weight = _rows_like(pattern, n, m, device, n + m)
+        out = torch.full((n, d), 7.0, dtype=dtype, device=device)
+        vgo.top4_project(table, index, weight, out=out)
+        assert bool(torch.isnan(out[1]).all()) and bool(torch.isfinite(out[n - 1]).all())
+        for r0 in range(0, n, piece):
+            part = proj.top4_project(table, index[r0:r0 + piece], weight[r0:r0 + piece])
+            assert bool(torch.eq(out[r0:r0 + piece].nan_to_num_(3.0), part.nan_to_num_(3.0)).all()), r0
+        assert bool(torch.eq(proj.top4_project(table, index, weight, order=order).nan_to_num_(3.0), out).all())
+        used = index[pick.to(device)].clamp(0, m - 1).long()
+        ref = oracle.top4_project(table[used.flatten()].cpu(), torch.arange(1024, dtype=torch.int32).view(256, 4),
+                                  weight[pick.to(device)].cpu())
+        assert torch.equal(out[pick.to(device)].cpu(), ref)

@@ -35,7 +35,9 @@ def top4_project(table: torch.Tensor, index: torch.Tensor, weight: torch.Tensor,
 def locality_order(index: torch.Tensor, table_rows: int) -> torch.Tensor:
     """Output rows grouped by their first parent (stable, int32 [N]): computed in this
     order, the rows that share a parent run together and that parent's repeated
-    gathers hit the L2 cache.  Reusable for every restore with the same index."""
+    gathers hit the L2 cache.  Reusable for every restore with the same index.  It gains
+    for rows with one parent (or half of them); with four uniform parents each the plain
+    call is faster (1,048,576 rows over 65,536 of 1,024 in bf16: 1,236 against 1,311 us)."""
     _lib.require_gpu(index)
     if index.ndim != 2 or index.shape[1] != 4 or index.dtype != torch.int32:
         raise ValueError("locality_order requires int32 index [N, 4]")

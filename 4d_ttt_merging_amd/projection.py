@@ -46,7 +46,7 @@ def locality_order(index: torch.Tensor, table_rows: int) -> torch.Tensor:
 
 
 def gather_probe(table: torch.Tensor, index: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """The projection's gathers and arithmetic without its row writes: each output row's
+    """Whole-row gathers and the projection's arithmetic without row writes: each output row's
     values summed in fp32 (float32 [N]).  A measurement probe (vgo_top4_gather_probe):
     its time is what the memory fabric gives `top4_project`'s random-row reads."""
     lib = _lib.load()

@@ -221,7 +221,8 @@ int vgo_top4_project(const void* table, int64_t table_row_stride, const int32_t*
  * is computed exactly as by vgo_top4_project, so any order gives the same
  * result.  An order that groups rows by a shared parent (the stable sort of
  * index[:, 0] that vgo_csr_build gives) lets the repeated gathers of that parent
- * hit the L2 cache.  Same restore as vgo_top4_project (token_merging.py:387-414).
+ * hit the L2 cache; with four uniform parents per row vgo_top4_project is faster.
+ * Same restore as vgo_top4_project (token_merging.py:387-414).
  */
 int vgo_top4_project_ordered(const void* table, int64_t table_row_stride, const int32_t* index,
                              const float* weight, const int32_t* order, void* out,
@@ -229,9 +230,9 @@ int vgo_top4_project_ordered(const void* table, int64_t table_row_stride, const 
                              int64_t dim, int dtype, void* stream);
 
 /*
- * Gather probe: vgo_top4_project's gathers and arithmetic with each output row
- * summed (fp32, over its elements) into row_sums[n_rows] instead of being
- * written, i.e. the projection's reads without its row writes.  No reference
+ * Gather probe: whole-row gathers with vgo_top4_project's arithmetic, each output
+ * row summed (fp32, over its elements) into row_sums[n_rows] instead of being
+ * written, i.e. such a projection's reads without its row writes.  No reference
  * counterpart: a measurement of what the memory fabric gives the restore's
  * random-row reads (bench.py --only gather).  Rows must be whole 16-byte chunks
  * (else VGO_EUNSUPPORTED).

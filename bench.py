@@ -381,11 +381,11 @@ def gather_ceiling(device, steps):
     res["copy_2GB_gbs"] = round(2 * n * d * 2 / sec / 1e9, 1)
     del src
     # The C2 restore split into its two streams.  Read-only: the gather probe
-    # (vgo_top4_gather_probe) does the projection's four random-row gathers per row
-    # from the 128 MB (MALL-resident) C2 table and its arithmetic, and writes one
+    # (vgo_top4_gather_probe) does four random whole-row gathers per row from the
+    # 128 MB (MALL-resident) C2 table and the projection's arithmetic, and writes one
     # float per row.  Write-only: a 2 GiB fill, the size of the C2 output.  Then the
-    # projection itself; its time against the sum of the two says whether the
-    # fabric overlaps its reads with its writes.
+    # projection itself: whole-row gathers took 0.985 of the sum of the two, below
+    # that its column slices are served by the L2s.
     proj = importlib.import_module("4d_ttt_merging_amd.projection")
     m = 65536
     index, weight = c2_inputs(n, m)
